@@ -102,15 +102,54 @@ template <int L> MCB_HD float cdot(float vx, float vy, float vz) {
     }
 }
 
+// ------------------------------------------------- correctly rounded helpers
+// The compiler's IEEE division and square root scale their operands, refine
+// and fix up for the whole float range: 11 instructions for a reciprocal, 28
+// for 1 / sqrtf. The step's arguments need less: 4 and 10. Each form below
+// gives the bits of the expression it stands for on the range it states (every
+// float of it compared on the device); div_fixup supplies zeros, infinities
+// and NaN. Outside that range, where a subnormal or a value beyond 2^126 is
+// involved, the last bit may differ. Host code divides. With the products
+// of gradCalc formed once per staged cell and the halves of HeF once per cell,
+// an FP32 collide lane issues 657 + 61 per normal VALU instructions per plane
+// instead of 714 + 95: 256^3 collide 0.521 -> 0.511 ms (it is bound by its
+// traffic, 5.5 TB/s), phase pass 0.173 -> 0.166 ms.
+#if defined(__HIP_DEVICE_COMPILE__)
+// 1.0f / x for 2^-126 <= |x| <= 2^126, 0, infinities and NaN.
+__device__ __forceinline__ float recip_rn(float x) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y), x, 1.0f);
+}
+// 1.0f / sqrtf(m) for m >= 1e-9 (infinity included). h is just below
+// 1 / (2 sqrt m): with exactly half of it the correction of s rounds to the
+// wrong side where m is the last float below a power of 4.
+__device__ __forceinline__ float rsqrt_rn(float m) {
+    const float s0 = __builtin_amdgcn_sqrtf(m), r = __builtin_amdgcn_rcpf(s0);
+    const float h = r * 0x1.fffffep-2f;
+    const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, m), h, s0);   // sqrtf(m)
+    const float y = __builtin_fmaf(__builtin_fmaf(-s, r, 1.0f), r, r);
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y), s0, 1.0f);
+}
+// x / CSSQ for x = 0, x >= 2^-104 and infinity (1 / CSSQ rounds to 3).
+__device__ __forceinline__ float div_cssq(float x) {
+    const float q = x * INV_CSSQ;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-CSSQ, q, x), INV_CSSQ, q), CSSQ, x);
+}
+#else
+inline float recip_rn(float x) { return 1.0f / x; }
+inline float rsqrt_rn(float m) { return 1.0f / sqrtf(m); }
+inline float div_cssq(float x) { return x / CSSQ; }
+#endif
+
 // ---------------------------------------------------------------- gradCalc
-// lbm.cu:50-71. nb(l) returns phi(x + c_l).
-template <class NB>
-MCB_HD void grad_normal(NB&& nb, const Derived& d, float& nx, float& ny, float& nz, float& ind) {
+// lbm.cu:50-71. nbt(l) returns the product 3 w_l phi(x + c_l).
+template <class NBT>
+MCB_HD void grad_normal_of(NBT&& nbt, float& nx, float& ny, float& nz, float& ind) {
     float gx = 0.0f, gy = 0.0f, gz = 0.0f;
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
         if constexpr (l != 0) {
-            const float t = d.coef[WC[l]] * nb(lc);
+            const float t = nbt(lc);
             gx = acc<CX[l]>(gx, t);
             gy = acc<CY[l]>(gy, t);
             gz = acc<CZ[l]>(gz, t);
@@ -118,11 +157,16 @@ MCB_HD void grad_normal(NB&& nb, const Derived& d, float& nx, float& ny, float& 
     });
     const float gmag_sq = gx * gx + gy * gy + gz * gz;
     const float m = gmag_sq > 1e-9f ? gmag_sq : 1e-9f;   // fmaxf(gmag_sq, 1e-9)
-    const float factor = 1.0f / sqrtf(m);                 // rsqrtf -> IEEE 1/sqrt
+    const float factor = rsqrt_rn(m);                     // rsqrtf -> IEEE 1/sqrt
     nx = gx * factor;
     ny = gy * factor;
     nz = gz * factor;
     ind = gmag_sq * factor;
+}
+// The same with nb(l) returning phi(x + c_l).
+template <class NB>
+MCB_HD void grad_normal(NB&& nb, const Derived& d, float& nx, float& ny, float& nz, float& ind) {
+    grad_normal_of([&](auto lc) { return d.coef[WC[decltype(lc)::value]] * nb(lc); }, nx, ny, nz, ind);
 }
 
 // ----------------------------------------------------------- curvatureCalc
@@ -153,28 +197,31 @@ struct Moments {
 };
 
 // lbm.cu:161-224. fv[l] are the 19 pre-collision populations of the cell.
+// The factor 0.5 of HeF is taken into invRhoCssq once per cell: scaling by a
+// power of two commutes with rounding, and where a subnormal breaks that,
+// HeF is far below the last bit of the value that it is added to.
 MCB_HD Moments moments(const float (&fv)[Q], const Phys& p, float fx, float fy, float fz) {
     Moments m;
     float rho = 0.0f;
     for_links([&](auto lc) { rho += fv[decltype(lc)::value]; });
-    const float invRho = 1.0f / rho;
+    const float invRho = recip_rn(rho);
     const float sumUx = invRho * (fv[1] - fv[2] + fv[7] - fv[8] + fv[9] - fv[10] + fv[13] - fv[14] + fv[15] - fv[16]);
     const float sumUy = invRho * (fv[3] - fv[4] + fv[7] - fv[8] + fv[11] - fv[12] + fv[14] - fv[13] + fv[17] - fv[18]);
     const float sumUz = invRho * (fv[5] - fv[6] + fv[9] - fv[10] + fv[11] - fv[12] + fv[16] - fv[15] + fv[18] - fv[17]);
     const float ux = sumUx + fx * 0.5f * invRho;
     const float uy = sumUy + fy * 0.5f * invRho;
     const float uz = sumUz + fz * 0.5f * invRho;
-    const float uu = 0.5f * (ux * ux + uy * uy + uz * uz) * INV_CSSQ;
-    const float invRhoCssq = 1.0f / (rho * CSSQ);
+    const float uu = (0.5f * INV_CSSQ) * (ux * ux + uy * uy + uz * uz);
+    const float halfInvRhoCssq = 0.5f * recip_rn(rho * CSSQ);
     float fneq[Q];
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
         const float udotc = cdot<l>(ux, uy, uz) * INV_CSSQ;
         const float eqBase = rho * (udotc + 0.5f * udotc * udotc - uu);
         const float common = p.w[WC[l]] * (rho + eqBase);
-        const float HeF = 0.5f * common *
+        const float HeF = common *
                           (((float)CX[l] - ux) * fx + ((float)CY[l] - uy) * fy + ((float)CZ[l] - uz) * fz) *
-                          invRhoCssq;
+                          halfInvRhoCssq;
         const float feq = common - HeF;
         fneq[l] = fv[l] - feq;
     });
@@ -196,7 +243,7 @@ MCB_HD Moments moments(const float (&fv)[Q], const Phys& p, float fx, float fy, 
 struct FluidCell {
     float rho, ux, uy, uz, fx, fy, fz;
     float pxx, pyy, pzz, pxy, pxz, pyz;
-    float uu, invRhoCssq;
+    float uu, halfInvRhoCssq;
 };
 
 MCB_HD FluidCell fluid_cell(const Moments& m, float fx, float fy, float fz) {
@@ -205,8 +252,9 @@ MCB_HD FluidCell fluid_cell(const Moments& m, float fx, float fy, float fz) {
     c.fx = fx; c.fy = fy; c.fz = fz;
     c.pxx = m.pxx; c.pyy = m.pyy; c.pzz = m.pzz;
     c.pxy = m.pxy; c.pxz = m.pxz; c.pyz = m.pyz;
-    c.uu = 0.5f * (m.ux * m.ux + m.uy * m.uy + m.uz * m.uz) / CSSQ;   // division, as lbm.cu:263
-    c.invRhoCssq = 1.0f / (m.rho * CSSQ);
+    // Division, as lbm.cu:263 (a uu below 2^-104 is lost next to rho).
+    c.uu = div_cssq(0.5f * (m.ux * m.ux + m.uy * m.uy + m.uz * m.uz));
+    c.halfInvRhoCssq = 0.5f * recip_rn(m.rho * CSSQ);
     return c;
 }
 
@@ -217,9 +265,9 @@ MCB_HD float fluid_post(const FluidCell& c, const Phys& p, const Derived& d) {
     const float w = p.w[WC[L]];
     const float udotc = cdot<L>(c.ux, c.uy, c.uz) * INV_CSSQ;
     const float feq = w * (c.rho + c.rho * (udotc + 0.5f * udotc * udotc - c.uu));
-    const float HeF = 0.5f * feq *
+    const float HeF = feq *
                       (((float)cx - c.ux) * c.fx + ((float)cy - c.uy) * c.fy + ((float)cz - c.uz) * c.fz) *
-                      c.invRhoCssq;
+                      c.halfInvRhoCssq;
     constexpr float kx = cx != 0 ? DIAG1 : DIAG0;
     constexpr float ky = cy != 0 ? DIAG1 : DIAG0;
     constexpr float kz = cz != 0 ? DIAG1 : DIAG0;

@@ -1134,7 +1134,11 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
     constexpr int HX = TX + 2, HY = TY + 2, HN = HX * HY;  // normal plane + 1-halo
     constexpr int KP = (PN + NT - 1) / NT;
     constexpr int KH = (HN + NT - 1) / NT;
-    __shared__ float s_phi[4][PN];
+    // FP32: gradCalc's products 3 w_l phi of the face and the edge links, formed
+    // once per staged cell instead of 18 times per normal (the same bits);
+    // 16 bits: phi.
+    constexpr int KF = S::kAnchored ? 1 : 2;
+    __shared__ float s_phi[4][KF][PN];
     __shared__ float s_n[3][3][HN];
     __shared__ float s_ind[2][NT];
 
@@ -1159,13 +1163,21 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
     }
 
     const Field phi_f(c.phi, (unsigned)(G.n * 4));
+    auto stage = [&](int z, int e, float v) {
+        float(*dst)[PN] = s_phi[z & 3];
+        if constexpr (S::kAnchored) {
+            dst[0][e] = v;
+        } else {
+            dst[0][e] = d.coef[1] * v;
+            dst[KF - 1][e] = d.coef[2] * v;
+        }
+    };
     auto load_phi = [&](int z) {
         const unsigned zb4 = (unsigned)(wrapmod(z, G.nz) * G.nxy) * 4u;
-        float* dst = s_phi[z & 3];
 #pragma unroll
         for (int q = 0; q < KP; ++q) {
             const int e = tid + q * NT;
-            if (q < KP - 1 || e < PN) dst[e] = phi_f.ld(poff[q], zb4);
+            if (q < KP - 1 || e < PN) stage(z, e, phi_f.ld(poff[q], zb4));
         }
     };
     // Software-pipelined phi staging inside the z loop: fetch_phi() loads a
@@ -1181,18 +1193,17 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
         }
     };
     auto put_phi = [&](int z) {
-        float* dst = s_phi[z & 3];
 #pragma unroll
         for (int q = 0; q < KP; ++q) {
             const int e = tid + q * NT;
-            if (q < KP - 1 || e < PN) dst[e] = preg[q];
+            if (q < KP - 1 || e < PN) stage(z, e, preg[q]);
         }
     };
     auto nslot = [](int z) { return (z + 3) % 3; };  // z >= -3
     auto comp_n = [&](int z) {
-        const float* pm = s_phi[(z - 1) & 3];
-        const float* p0 = s_phi[z & 3];
-        const float* pp = s_phi[(z + 1) & 3];
+        const float(*pm)[PN] = s_phi[(z - 1) & 3];
+        const float(*p0)[PN] = s_phi[z & 3];
+        const float(*pp)[PN] = s_phi[(z + 1) & 3];
         const int sl = nslot(z);
         float* ind_dst = s_ind[z & 1];
 #pragma unroll
@@ -1204,7 +1215,7 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                 float nx, ny, nz, ind;
                 auto nb = [&](auto lc) {
                     constexpr int l = decltype(lc)::value;
-                    return pick<CZ[l]>(pm, p0, pp)[cc + CY[l] * PX + CX[l]];
+                    return pick<CZ[l]>(pm, p0, pp)[S::kAnchored ? 0 : WC[l] - 1][cc + CY[l] * PX + CX[l]];
                 };
                 if constexpr (S::kAnchored) {
                     fast::grad_normal(nb, k16, nx, ny, nz, ind);
@@ -1212,7 +1223,7 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                     // gradCalc updates interior cells only: a face keeps n = 0.
                     nx = ny = nz = ind = 0.0f;
                 } else {
-                    grad_normal(nb, d, nx, ny, nz, ind);
+                    grad_normal_of(nb, nx, ny, nz, ind);
                 }
                 s_n[sl][0][e] = nx;
                 s_n[sl][1][e] = ny;
@@ -1290,7 +1301,6 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
         const float ncx = s_n[s0][0][e0], ncy = s_n[s0][1][e0], ncz = s_n[s0][2][e0];
         const float ind = s_ind[z & 1][tid];
 
-        const float phic = s_phi[z & 3][(ty + 2) * PX + (tx + 2)];
         auto nbn = [&](auto lc, float& ax, float& ay, float& az) {
             constexpr int l = decltype(lc)::value;
             const int slot = pick<CZ[l]>(sm, s0, sp);
@@ -1300,6 +1310,7 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
             if constexpr (CZ[l] != 0) az = s_n[slot][2][e];
         };
         if constexpr (S::kAnchored) {
+            const float phic = s_phi[z & 3][0][(ty + 2) * PX + (tx + 2)];
             cell16<MODE>(c, k16, fsrc, gsrc, fdst, gdst, col, me4, zs, fr, nbn, ncx, ncy, ncz, ind, phic);
         } else {
             float curv, Fx, Fy, Fz;
@@ -1319,13 +1330,13 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                 Field(c.nz, fb).st(me4, z1 * 4u, ncz);
             } else {
                 const FluidCell fc = fluid_cell(m, Fx, Fy, Fz);
-                const PhaseCell pc = phase_cell(c.phys, phic, m.ux, m.uy, m.uz, ncx, ncy, ncz);
                 // BGK phase collision (tau_g != 1): the 19 pre-collision g
                 // (post-stream, gathered) are loaded together here, so their
                 // latency overlaps the fluid collision instead of stalling each
                 // g* store in turn.
-                float gpre[Q];
+                float gpre[Q], phic = 0.0f;
                 if constexpr (MODE == COLLIDE_STEP_BGK) {
+                    phic = phi_f.ld(me4, z1 * 4u);
                     for_links([&](auto lc) {
                         constexpr int l = decltype(lc)::value;
                         gpre[l] = gsrc.template ldb<l>(col.template src<l>(), gsrc.zb(zs[1 - CZ[l]]));
@@ -1336,9 +1347,9 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                     fdst.template stb<l>(col.me(), fdst.zb(z1), fluid_post<l>(fc, c.phys, d));
                 });
                 if (MODE == COLLIDE_STEP && c.gm != GM_POPULATIONS) {
-                    // Moment form: keep what collisionPhase needs (phic is the
-                    // phi buffer of this step, the next step's phi_prev): u,
-                    // and n unless the next phase pass recomputes it from phi.
+                    // Moment form: keep what collisionPhase needs beside the phi
+                    // buffer of this step (the next step's phi_prev): u, and n
+                    // unless the next phase pass recomputes it from phi.
                     Field(c.gm_u[0], fb).st(me4, z1 * 4u, m.ux);
                     Field(c.gm_u[1], fb).st(me4, z1 * 4u, m.uy);
                     Field(c.gm_u[2], fb).st(me4, z1 * 4u, m.uz);
@@ -1349,6 +1360,8 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                     }
                     return;
                 }
+                if constexpr (MODE == COLLIDE_STEP) phic = phi_f.ld(me4, z1 * 4u);
+                const PhaseCell pc = phase_cell(c.phys, phic, m.ux, m.uy, m.uz, ncx, ncy, ncz);
                 for_links([&](auto lc) {
                     constexpr int l = decltype(lc)::value;
                     if constexpr (MODE == COLLIDE_STEP) {
