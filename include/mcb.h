@@ -67,7 +67,7 @@ typedef enum mcb_path { MCB_PATH_AUTO = 0, MCB_PATH_FUSED = 1, MCB_PATH_STAGED =
  * cell). STORED: the collide pass writes n beside u. RECOMPUTED: the phase
  * pass recomputes n from phi with gradCalc's operations (src/lbm.cu:50-71),
  * the same bits, 24 fewer bytes per cell and step and more arithmetic. AUTO:
- * RECOMPUTED where the phase pass runs z-chunks of 32 planes or more (large
+ * RECOMPUTED where the phase pass runs z-chunks of 16 planes or more (large
  * lattices), STORED otherwise. Results are identical in every mode; other
  * paths and forms ignore it. */
 typedef enum mcb_normals { MCB_NORMALS_AUTO = 0, MCB_NORMALS_STORED = 1, MCB_NORMALS_RECOMPUTED = 2 } mcb_normals;

@@ -56,10 +56,9 @@ __global__ __launch_bounds__(PBX * PBY) void k_phase(CaseView c, unsigned gx, un
 }
 
 // Moment-form phase pass (phase_tile_gm, or phase_tile_gm_rn when n is
-// recomputed): the collide pass's tiles and grid. The recomputing form at
-// 512-thread tiles is held to 80 VGPRs: three workgroups per CU (LDS ~49 KB
-// each).
-template <int TX, int TY, bool RN> constexpr int phase_gm_waves_per_eu() { return RN && TX * TY == 512 ? 6 : 1; }
+// recomputed) on the tiles of phase_tiling. The recomputing form's own tile is
+// held to 80 VGPRs: three workgroups per CU (LDS 52 KB each).
+template <int TX, int TY, bool RN> constexpr int phase_gm_waves_per_eu() { return RN && TX == 32 && TY == 16 ? 6 : 1; }
 
 // Tile of the phase pass when it recomputes n (nx, ny at least its sides):
 // its ring cells each compute a normal, so the taller 32x16 tile (100 ring
@@ -439,15 +438,42 @@ Tiling phase_tiling(const Geo& geo, const Tiling& t, bool rn) {
         p.tx = MCB_PHASE_RN_TX;
         p.ty = MCB_PHASE_RN_TY;
     }
-    // Chunks of 64 planes, halved (down to 8) until the pass has two
-    // workgroups per CU.
-    const unsigned layer = (unsigned)((geo.nx + p.tx - 1) / p.tx) * (unsigned)((geo.ny + p.ty - 1) / p.ty);
+    // 4-row collide tiles (small lattices): with 8 rows the ring is 29%
+    // instead of 55% of the tile.
+    if (!rn && p.tx == 64 && p.ty == 4) p.ty = 8;
+    const int layer = ((geo.nx + p.tx - 1) / p.tx) * ((geo.ny + p.ty - 1) / p.ty);
     p.zc = std::min(64, geo.nz);
-    while (p.zc > 8 && layer * (unsigned)((geo.nz + p.zc - 1) / p.zc) < 512u) p.zc = (p.zc + 1) / 2;
+    if (rn) {
+        // Three workgroups fit per CU, so the pass runs in rounds of 768 and a
+        // chunk of zc planes takes about zc + 2 (its two first planes of
+        // normals): the chunk with the shortest product. 256^3 (us): 43
+        // planes, one full round, 135; 22 (two) 145; 26 147; 16 148; 64 (two
+        // thirds of a round) 164; 32 (a round and a third) 155.
+        long long best = 0;
+        for (int n = (geo.nz + p.zc - 1) / p.zc, zc = p.zc; n == 1 || zc > 8; ++n) {
+            zc = (geo.nz + n - 1) / n;
+            const long long rounds = ((long long)layer * ((geo.nz + zc - 1) / zc) + 767) / 768;
+            const long long cost = rounds * (zc + 2);
+            if (best == 0 || cost < best) {
+                best = cost;
+                p.zc = zc;
+            }
+        }
+        return p;
+    }
+    // Chunks of 64 planes, halved until the pass has two workgroups per CU
+    // (each chunk re-reads the planes around it). With chunks kept at 8 planes
+    // or more, 64^3 took 13.2 us against 8.5 with single planes, the reference
+    // preset 16.5 against 14.5 with 4.
+    while (p.zc > 1 && (long long)layer * ((geo.nz + p.zc - 1) / p.zc) < 512) p.zc = (p.zc + 1) / 2;
     return p;
 }
 
-bool phase_recomputes_n(const Geo& geo, const Tiling& t) { return phase_tiling(geo, t, true).zc >= 32; }
+// Recomputing n saves the collide pass 3 of its 25 stores per cell; on chunks
+// this long it costs the phase pass less (192^3: 20 planes, 250 + 75 us
+// against 266 + 70 with n stored; 128^3: 6 planes, 74.5 + 27.2 against
+// 77.2 + 20.6).
+bool phase_recomputes_n(const Geo& geo, const Tiling& t) { return phase_tiling(geo, t, true).zc >= 16; }
 
 hipError_t launch_phase(const CaseView& c0, const Tiling& t, hipStream_t s) {
     if (c0.gm == GM_MOMENTS) {

@@ -149,14 +149,12 @@ Tiling tiling_at(int i);
 // Phase pass; in moment form (gm == GM_MOMENTS) it runs on the tiles t.
 hipError_t launch_phase(const CaseView& c, const Tiling& t, hipStream_t s);
 // Tile and z-chunk of the moment-form phase pass for collide tiles t, rn =
-// n recomputed: the tile is t's, or the recomputing pass's own where the
-// lattice spans it; the chunk is as long as the lattice allows with two
-// workgroups per CU (64 planes, halved down to 8: each chunk also reads the
-// planes around it, and the recomputing pass starts each chunk with two
-// planes of normals).
+// n recomputed: the tile is t's (8 rows where t has 4), or the recomputing
+// pass's own where the lattice spans it; the chunk fills the device (see
+// there).
 Tiling phase_tiling(const Geo& geo, const Tiling& t, bool rn);
 // Whether a single-case FP32 moment-form context recomputes n in the phase
-// pass (CaseView::gm_n null) rather than storing it: on chunks of 32 planes
+// pass (CaseView::gm_n null) rather than storing it: on chunks of 16 planes
 // or more, where the 24 bytes per cell saved outweigh the per-chunk start.
 bool phase_recomputes_n(const Geo& geo, const Tiling& t);
 // n from the state phi into gm_n (a stored-normal case loaded from an image).

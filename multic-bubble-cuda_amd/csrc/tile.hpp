@@ -315,14 +315,17 @@ __device__ __forceinline__ float phase_link(float w, float wphi, float phi_norm,
 // (two rows of TX cells and two columns of TY + 2, corners included).
 template <int TX, int TY> constexpr int gm_ring_cells() { return 2 * TX + 2 * (TY + 2); }
 
-// LDS slots of phase_tile_gm_rn's link values, link-major. Link l (1..18) has a
+// LDS slots of the link values that a tile's cells and its ring send each
+// other, link-major. Links 5 and 6 (along z) stay in their column, hence in
+// their thread's registers, as does the rest link. Any other link l has a
 // row-major region of the cells that lie in the tile or send l into it:
 // x in [-max(c_x, 0), TX - 1 + max(-c_x, 0)] and likewise y, i.e.
-// (TX + |c_x|) x (TY + |c_y|) cells (the rest link stays in a register).
+// (TX + |c_x|) x (TY + |c_y|) cells.
 // A tile cell writes every link at its own position and reads link l at its
 // position - c_l, both at a compile-time offset from one of two row bases;
 // a ring corner's links that enter neither the region nor the tile go to one
 // spare slot that nothing reads.
+constexpr bool crosses(int l) { return CX[l] != 0 || CY[l] != 0; }
 template <int TX, int TY> struct GmSlots {
     static constexpr int w(int l) { return TX + (CX[l] != 0 ? 1 : 0); }
     static constexpr int h(int l) { return TY + (CY[l] != 0 ? 1 : 0); }
@@ -330,10 +333,11 @@ template <int TX, int TY> struct GmSlots {
     static constexpr int lo_y(int l) { return CY[l] > 0 ? -1 : 0; }
     static constexpr int base(int l) {
         int b = 0;
-        for (int k = 1; k < l; ++k) b += w(k) * h(k);
+        for (int k = 1; k < l; ++k)
+            if (crosses(k)) b += w(k) * h(k);
         return b;
     }
-    static constexpr int kSpare = base(Q);   // after the 18 regions
+    static constexpr int kSpare = base(Q);   // after the 16 regions
     static constexpr int kSlots = kSpare + 1;
     static constexpr bool inside(int l, int sx, int sy) {
         return sx >= lo_x(l) && sx < lo_x(l) + w(l) && sy >= lo_y(l) && sy < lo_y(l) + h(l);
@@ -348,6 +352,7 @@ template <int TX, int TY> struct GmSlots {
 template <int TX, int TY> constexpr bool gm_slots_ok() {
     using L = GmSlots<TX, TY>;
     for (int l = 1; l < Q; ++l) {
+        if (!crosses(l)) continue;
         if (L::own(l) < 0 || L::src(l) < 0) return false;
         // Every source of the tile and every tile cell lies in the region.
         for (int sy = -1; sy <= TY; ++sy)
@@ -358,6 +363,30 @@ template <int TX, int TY> constexpr bool gm_slots_ok() {
             }
     }
     return true;
+}
+
+// Slots of the five links that the ring cell of side `side` at halo position
+// (hx, hy) sends into the tile.
+template <int TX, int TY> __device__ __forceinline__ void ring_slots(int side, int hx, int hy, int (&slot)[5]) {
+    using SL = GmSlots<TX, TY>;
+    const int sx = hx - 1, sy = hy - 1;
+    auto fill = [&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        auto one = [&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            constexpr int l = RING_LINK[s][k];
+            slot[k] = SL::inside(l, sx, sy) ? SL::at(l, sx, sy) : SL::kSpare;
+        };
+        one(std::integral_constant<int, 0>{});
+        one(std::integral_constant<int, 1>{});
+        one(std::integral_constant<int, 2>{});
+        one(std::integral_constant<int, 3>{});
+        one(std::integral_constant<int, 4>{});
+    };
+    if (side == 0) fill(std::integral_constant<int, 0>{});
+    else if (side == 1) fill(std::integral_constant<int, 1>{});
+    else if (side == 2) fill(std::integral_constant<int, 2>{});
+    else fill(std::integral_constant<int, 3>{});
 }
 
 // Moment-form phase pass with stored normals (CaseView::gm_n set: the
@@ -385,10 +414,12 @@ template <int TX, int TY> constexpr bool gm_slots_ok() {
 template <int TX, int TY>
 __device__ __forceinline__ void phase_tile_gm(const CaseView& c, int x0, int y0, int zb, int ze) {
     constexpr int NT = TX * TY;
-    constexpr int HX = TX + 2, HY = TY + 2, HN = HX * HY;
     constexpr int NR = gm_ring_cells<TX, TY>();
+    using SL = GmSlots<TX, TY>;
     static_assert(NR <= NT, "a lane per ring cell");
-    __shared__ float s_g[HN * Q];   // [halo cell][link]: g*_l of the source cell
+    static_assert(gm_slots_ok<TX, TY>(), "link slots");
+    static_assert(SL::kSlots < 16384, "LDS offsets");
+    __shared__ float s_g[SL::kSlots];
 
     const Geo& G = c.geo;
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
@@ -408,7 +439,11 @@ __device__ __forceinline__ void phase_tile_gm(const CaseView& c, int x0, int y0,
     // ---- tile cell
     const int x = x0 + tx, y = y0 + ty;
     const bool valid = x < G.nx && y < G.ny;
-    const int e0 = (ty + 1) * HX + (tx + 1);
+    const int row0 = ty * TX + tx, row1 = ty * (TX + 1) + tx;   // row bases of widths TX, TX + 1
+    auto own_slot = [&](auto lc) -> float& {
+        constexpr int l = decltype(lc)::value;
+        return s_g[(SL::w(l) == TX ? row0 : row1) + SL::own(l)];
+    };
     // Cells past the lattice edge (partial tiles) take their periodic image.
     const unsigned own = (unsigned)(wrapmod(y, G.ny) * G.nx + wrapmod(x, G.nx));
     float f[3][7];     // window: phi, ux, uy, uz, nx, ny, nz on planes by slot
@@ -421,15 +456,8 @@ __device__ __forceinline__ void phase_tile_gm(const CaseView& c, int x0, int y0,
     else if (tid < 2 * TX + TY + 2) { hx = 0; hy = tid - 2 * TX; side = 2; }
     else { hx = TX + 1; hy = min(tid - 2 * TX - TY - 2, TY + 1); side = 3; }
     const unsigned roff = (unsigned)(wrapmod(y0 - 1 + hy, G.ny) * G.nx + wrapmod(x0 - 1 + hx, G.nx));
-    const int rbase = (hy * HX + hx) * Q;
-    // The side's five link numbers, 5 bits each.
-    unsigned rlinks = 0;
-#pragma unroll
-    for (int k = 0; k < 5; ++k)
-        rlinks |= (unsigned)(side == 0 ? RING_LINK[0][k]
-                                       : side == 1 ? RING_LINK[1][k] : side == 2 ? RING_LINK[2][k] : RING_LINK[3][k])
-                  << (5 * k);
-    auto rslot = [&](int k) { return s_g + rbase + (int)((rlinks >> (5 * k)) & 31u); };
+    int rslot[5];   // LDS slots of the side's five links at this cell
+    ring_slots<TX, TY>(side, hx, hy, rslot);
     const bool ry = side < 2;                     // the side's axis is y
     const float rs = (side & 1) ? -1.0f : 1.0f;   // and its sign
     float rin[3];      // in-plane links of the ring cell for the next plane
@@ -474,17 +502,21 @@ __device__ __forceinline__ void phase_tile_gm(const CaseView& c, int x0, int y0,
         float r[7];
         if (ring) fetch(r, plane_of(z + 1) + roff);            // used after the tile cell's work
         if (z + 1 < ze) fetch(f[PN], plane_of(z + 2) + own);   // read by the next plane
-        float* dst = s_g + e0 * Q;
+        float g0, g5, g6;   // the links that stay in the column
         {   // c_z = +1 links from plane z-1, computed on the previous plane
             int k = 0;
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
-                if constexpr (CZ[l] > 0) { dst[l] = hold[k]; ++k; }
+                if constexpr (CZ[l] > 0) {
+                    if constexpr (crosses(l)) own_slot(lc) = hold[k];
+                    else g5 = hold[k];
+                    ++k;
+                }
             });
         }
         {   // in-plane links from plane z
             const PhaseCell c0 = cell(f[P0]);
-            dst[0] = phase_post<0>(c0, c.phys);
+            g0 = phase_post<0>(c0, c.phys);
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
                 if constexpr (l != 0 && CZ[l] == 0 && l % 2 == 1) {
@@ -493,8 +525,8 @@ __device__ __forceinline__ void phase_tile_gm(const CaseView& c, int x0, int y0,
                     const float ud = cdot<l>(c0.ux, c0.uy, c0.uz) * INV_CSSQ;
                     const float wa = wl * (c0.phi_norm * cdot<l>(c0.nx, c0.ny, c0.nz));
                     const float wphi = wl * c0.phi;
-                    dst[l] = wphi * (1.0f + ud) + wa;
-                    dst[l + 1] = wphi * (1.0f + -ud) + -wa;
+                    own_slot(lc) = wphi * (1.0f + ud) + wa;
+                    own_slot(LinkC<l + 1>{}) = wphi * (1.0f + -ud) + -wa;
                 }
             });
             int k = 0;
@@ -507,22 +539,24 @@ __device__ __forceinline__ void phase_tile_gm(const CaseView& c, int x0, int y0,
             const PhaseCell cp = cell(f[PP]);
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
-                if constexpr (CZ[l] < 0) dst[l] = phase_post<l>(cp, c.phys);
+                if constexpr (CZ[l] < 0 && crosses(l)) own_slot(lc) = phase_post<l>(cp, c.phys);
+                else if constexpr (CZ[l] < 0) g6 = phase_post<l>(cp, c.phys);
             });
         }
         if (ring) {
-            *rslot(3) = rhold[PH];
-            *rslot(0) = rin[0];
-            *rslot(1) = rin[1];
-            *rslot(2) = rin[2];
-            *rslot(4) = ring_plane(r, rhold[PH]);
+            s_g[rslot[3]] = rhold[PH];
+            s_g[rslot[0]] = rin[0];
+            s_g[rslot[1]] = rin[1];
+            s_g[rslot[2]] = rin[2];
+            s_g[rslot[4]] = ring_plane(r, rhold[PH]);
         }
         __syncthreads();
         if (valid) {
             float sum = 0.0f;
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
-                sum += s_g[(e0 - CY[l] * HX - CX[l]) * Q + l];
+                if constexpr (crosses(l)) sum += s_g[(SL::w(l) == TX ? row0 : row1) + SL::src(l)];
+                else sum += l == 0 ? g0 : (l == 5 ? g5 : g6);
             });
             // Ghost-layer faces take boundaryConditions' copy instead.
             if (c.bc == MCB_BC_REFERENCE && ref_face(G, x, y, z)) sum = ld32(c.phi_prev, ref_clamped(G, x, y, z));
@@ -555,12 +589,17 @@ __device__ __forceinline__ void phase_tile_gm(const CaseView& c, int x0, int y0,
 // step moves phi and u (16 B per cell) instead of phi, u and n (28 B), and
 // the collide pass stores u only. phi planes with a 2-cell halo are staged
 // in a 3-slot LDS ring (a plane is loaded once per chunk plus the chunk's
-// 4 boundary planes).
+// 4 boundary planes) as gradCalc's products 3 w_l phi of the face and the
+// edge links, so that a normal takes 57 VALU instructions, not 93; the LDS
+// for the second product comes from the links along z, which stay in
+// registers. The pass is bound by its instructions (about 175 per tile cell
+// and plane); 256^3: 0.171 -> 0.135 ms, chunks of one full round included
+// (phase_tiling).
 //   Each link value is computed once. In-plane opposite links l, l'
 // (c_l' = -c_l) of a cell share their work: their dot products are exact
 // negatives (IEEE rounding is sign-symmetric), so one evaluation gives both.
 //   Thread (tx, ty) owns tile cell (tx, ty): a 3-plane register window of
-// its u (z, z+1, z+2 in flight) and its n on planes z, z+1. On plane z it
+// its u and phi (z, z+1, z+2 in flight) and its n on planes z, z+1. On plane z it
 // computes n on plane z+1, writes its in-plane links and its c_z = -1 links
 // from plane z+1, and computes its c_z = +1 links from plane z, held (5
 // registers) for plane z+1. Threads tid < gm_ring_cells also own one ring
@@ -580,7 +619,7 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
     static_assert(gm_slots_ok<TX, TY>(), "link slots");
     static_assert(SL::kSlots < 16384, "LDS offsets");
     __shared__ float s_g[SL::kSlots];
-    __shared__ float s_phi[3][PN];
+    __shared__ float s_t[3][2][PN];   // 3 w_l phi of the face and the edge links
 
     const Geo& G = c.geo;
     const Derived d(c.phys);
@@ -590,10 +629,11 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
     const Field phi_f(c.phi_prev, fbytes), ux_f(c.gm_u[0], fbytes), uy_f(c.gm_u[1], fbytes),
         uz_f(c.gm_u[2], fbytes);
     auto plane4 = [&](int z) { return (unsigned)(wrapmod(z, G.nz) * G.nxy) * 4u; };
-    auto fetch_u = [&](float (&u)[3], unsigned cell4, unsigned z4) {
+    auto fetch_u = [&](float (&u)[4], unsigned cell4, unsigned z4) {
         u[0] = ux_f.ld(cell4, z4);
         u[1] = uy_f.ld(cell4, z4);
         u[2] = uz_f.ld(cell4, z4);
+        u[3] = phi_f.ld(cell4, z4);
     };
 
     // In-plane byte offsets of the staged phi cells this thread loads.
@@ -608,12 +648,16 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
         }
         poff[q] = off;
     }
-    auto load_phi = [&](int z, float* dst) {
+    auto stage = [&](float (*dst)[PN], int e, float phi) {
+        dst[0][e] = d.coef[1] * phi;
+        dst[1][e] = d.coef[2] * phi;
+    };
+    auto load_phi = [&](int z, float (*dst)[PN]) {
         const unsigned z4 = plane4(z);
 #pragma unroll
         for (int q = 0; q < KP; ++q) {
             const int e = tid + q * NT;
-            if (q < KP - 1 || e < PN) dst[e] = phi_f.ld(poff[q], z4);
+            if (q < KP - 1 || e < PN) stage(dst, e, phi_f.ld(poff[q], z4));
         }
     };
     // Software-pipelined staging inside the z loop: fetch_phi() loads plane
@@ -628,28 +672,28 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
             if (q < KP - 1 || e < PN) preg[q] = phi_f.ld(poff[q], z4);
         }
     };
-    auto put_phi = [&](float* dst) {
+    auto put_phi = [&](float (*dst)[PN]) {
 #pragma unroll
         for (int q = 0; q < KP; ++q) {
             const int e = tid + q * NT;
-            if (q < KP - 1 || e < PN) dst[e] = preg[q];
+            if (q < KP - 1 || e < PN) stage(dst, e, preg[q]);
         }
     };
     // n of the cell staged at pc on the plane whose phi is p0 (pm below, pp
     // above), as the collide pass computes it; (gx, gy, gz) its lattice
     // coordinates for the ghost-layer test.
-    auto normal = [&](int pc, int gx, int gy, int gz, const float* pm, const float* p0, const float* pp,
-                      float (&n)[3]) {
+    auto normal = [&](int pc, int gx, int gy, int gz, const float (*pm)[PN], const float (*p0)[PN],
+                      const float (*pp)[PN], float (&n)[3]) {
         if (c.bc == MCB_BC_REFERENCE && ref_face(G, gx, gy, gz)) {
             n[0] = n[1] = n[2] = 0.0f;
             return;
         }
         auto nb = [&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            return pick<CZ[l]>(pm, p0, pp)[pc + CY[l] * PX + CX[l]];
+            return pick<CZ[l]>(pm, p0, pp)[WC[l] - 1][pc + CY[l] * PX + CX[l]];
         };
         float ind;
-        grad_normal(nb, d, n[0], n[1], n[2], ind);
+        grad_normal_of(nb, n[0], n[1], n[2], ind);
     };
 
     // ---- tile cell
@@ -663,7 +707,7 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
         constexpr int l = decltype(lc)::value;
         return s_g[(SL::w(l) == TX ? row0 : row1) + SL::own(l)];
     };
-    float u[3][3];     // window: u on planes by slot
+    float u[3][4];     // window: u and phi on planes by slot
     float nn[2][3];    // n on planes by parity
     float hold[5];     // c_z = +1 links for plane z+1, from plane z
     // ---- ring cell (side 0: row y0-1, 1: row y0+TY, 2: column x0-1, 3: column x0+TX)
@@ -678,26 +722,7 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
     const int pc_ring = (hy + 1) * PX + hx + 1;
     // LDS slots of the side's five links at this cell.
     int rslot[5];
-    {
-        const int sx = hx - 1, sy = hy - 1;
-        auto fill = [&](auto sc) {
-            constexpr int s = decltype(sc)::value;
-            auto one = [&](auto kc) {
-                constexpr int k = decltype(kc)::value;
-                constexpr int l = RING_LINK[s][k];
-                rslot[k] = SL::inside(l, sx, sy) ? SL::at(l, sx, sy) : SL::kSpare;
-            };
-            one(std::integral_constant<int, 0>{});
-            one(std::integral_constant<int, 1>{});
-            one(std::integral_constant<int, 2>{});
-            one(std::integral_constant<int, 3>{});
-            one(std::integral_constant<int, 4>{});
-        };
-        if (side == 0) fill(std::integral_constant<int, 0>{});
-        else if (side == 1) fill(std::integral_constant<int, 1>{});
-        else if (side == 2) fill(std::integral_constant<int, 2>{});
-        else fill(std::integral_constant<int, 3>{});
-    }
+    ring_slots<TX, TY>(side, hx, hy, rslot);
     const bool ry = side < 2;                     // the side's axis is y
     const float rs = (side & 1) ? -1.0f : 1.0f;   // and its sign
     float rin[3];      // in-plane links of the ring cell for the next plane
@@ -714,26 +739,26 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
         up = phase_link(w2, w2phi, q.phi_norm, pu + q.uz, pn + q.nz);
         return phase_link(w2, w2phi, q.phi_norm, pu - q.uz, pn - q.nz);
     };
-    auto cell = [&](float phi, const float (&uu)[3], const float (&n)[3]) {
-        return phase_cell(c.phys, phi, uu[0], uu[1], uu[2], n[0], n[1], n[2]);
+    auto cell = [&](const float (&uu)[4], const float (&n)[3]) {
+        return phase_cell(c.phys, uu[3], uu[0], uu[1], uu[2], n[0], n[1], n[2]);
     };
 
     // Prologue. Slot of plane p: (p - zb) mod 3 for the phi ring and the u
     // window (planes zb-2 and zb-1 pass through slots 1 and 2); parity
     // (p - zb) mod 2 for n and the ring's held c_z = +1 link.
-    load_phi(zb - 2, s_phi[1]);
-    load_phi(zb - 1, s_phi[2]);
-    load_phi(zb, s_phi[0]);
+    load_phi(zb - 2, s_t[1]);
+    load_phi(zb - 1, s_t[2]);
+    load_phi(zb, s_t[0]);
     fetch_u(u[2], own4, plane4(zb - 1));
     fetch_u(u[0], own4, plane4(zb));
     fetch_u(u[1], own4, plane4(zb + 1));
-    float rp[3];   // the ring cell's u on a prologue plane
+    float rp[4];   // the ring cell's u and phi on a prologue plane
     if (ring) fetch_u(rp, roff4, plane4(zb - 1));
     __syncthreads();
     {   // plane zb-1: the tile cell's c_z = +1 links, the ring cell's
         float nm[3];
-        normal(pc_own, x, y, zb - 1, s_phi[1], s_phi[2], s_phi[0], nm);
-        const PhaseCell pm = cell(s_phi[2][pc_own], u[2], nm);
+        normal(pc_own, x, y, zb - 1, s_t[1], s_t[2], s_t[0], nm);
+        const PhaseCell pm = cell(u[2], nm);
         int k = 0;
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
@@ -741,47 +766,51 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
         });
         if (ring) {
             float rn[3];
-            normal(pc_ring, rgx, rgy, zb - 1, s_phi[1], s_phi[2], s_phi[0], rn);
-            ring_plane(cell(s_phi[2][pc_ring], rp, rn), rhold[0]);
+            normal(pc_ring, rgx, rgy, zb - 1, s_t[1], s_t[2], s_t[0], rn);
+            ring_plane(cell(rp, rn), rhold[0]);
         }
     }
     __syncthreads();
-    load_phi(zb + 1, s_phi[1]);
+    load_phi(zb + 1, s_t[1]);
     if (ring) fetch_u(rp, roff4, plane4(zb));
     __syncthreads();
     {   // plane zb: the tile cell's n, the ring cell's in-plane and c_z = +1 links
-        normal(pc_own, x, y, zb, s_phi[2], s_phi[0], s_phi[1], nn[0]);
+        normal(pc_own, x, y, zb, s_t[2], s_t[0], s_t[1], nn[0]);
         if (ring) {
             float rn[3];
-            normal(pc_ring, rgx, rgy, zb, s_phi[2], s_phi[0], s_phi[1], rn);
-            ring_plane(cell(s_phi[0][pc_ring], rp, rn), rhold[1]);   // leaves plane zb's in-plane links in rin
+            normal(pc_ring, rgx, rgy, zb, s_t[2], s_t[0], s_t[1], rn);
+            ring_plane(cell(rp, rn), rhold[1]);   // leaves plane zb's in-plane links in rin
         }
     }
     __syncthreads();
-    load_phi(zb + 2, s_phi[2]);
+    load_phi(zb + 2, s_t[2]);
     __syncthreads();
 
     auto iter = [&](int z, auto p0, auto pp, auto pn, auto ph) {
         constexpr int P0 = decltype(p0)::value, PP = decltype(pp)::value, PN = decltype(pn)::value;
         constexpr int PH = decltype(ph)::value;
-        float ru[3];
+        float ru[4];
         if (ring) fetch_u(ru, roff4, plane4(z + 1));   // used after the tile cell's work
         if (z + 1 < ze) {                              // read by the next plane
             fetch_u(u[PN], own4, plane4(z + 2));
             fetch_phi(z + 3);
         }
         // n on plane z+1 (phi planes z, z+1, z+2 in slots P0, PP, PN)
-        normal(pc_own, x, y, z + 1, s_phi[P0], s_phi[PP], s_phi[PN], nn[PH ^ 1]);
+        normal(pc_own, x, y, z + 1, s_t[P0], s_t[PP], s_t[PN], nn[PH ^ 1]);
+        float g0, g5, g6;   // the links that stay in the column
         {   // c_z = +1 links from plane z-1, computed on the previous plane
             int k = 0;
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
-                if constexpr (CZ[l] > 0) { own_slot(lc) = hold[k]; ++k; }
+                if constexpr (CZ[l] > 0) {
+                    if constexpr (crosses(l)) own_slot(lc) = hold[k];
+                    else g5 = hold[k];
+                    ++k;
+                }
             });
         }
-        float g0;
         {   // in-plane links from plane z
-            const PhaseCell c0 = cell(s_phi[P0][pc_own], u[P0], nn[PH]);
+            const PhaseCell c0 = cell(u[P0], nn[PH]);
             g0 = phase_post<0>(c0, c.phys);
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
@@ -802,29 +831,30 @@ __device__ __forceinline__ void phase_tile_gm_rn(const CaseView& c, int x0, int 
             });
         }
         {   // c_z = -1 links from plane z+1
-            const PhaseCell cp = cell(s_phi[PP][pc_own], u[PP], nn[PH ^ 1]);
+            const PhaseCell cp = cell(u[PP], nn[PH ^ 1]);
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
-                if constexpr (CZ[l] < 0) own_slot(lc) = phase_post<l>(cp, c.phys);
+                if constexpr (CZ[l] < 0 && crosses(l)) own_slot(lc) = phase_post<l>(cp, c.phys);
+                else if constexpr (CZ[l] < 0) g6 = phase_post<l>(cp, c.phys);
             });
         }
         if (ring) {
             float rn[3];
-            normal(pc_ring, rgx, rgy, z + 1, s_phi[P0], s_phi[PP], s_phi[PN], rn);
+            normal(pc_ring, rgx, rgy, z + 1, s_t[P0], s_t[PP], s_t[PN], rn);
             s_g[rslot[3]] = rhold[PH];
             s_g[rslot[0]] = rin[0];
             s_g[rslot[1]] = rin[1];
             s_g[rslot[2]] = rin[2];
-            s_g[rslot[4]] = ring_plane(cell(s_phi[PP][pc_ring], ru, rn), rhold[PH]);
+            s_g[rslot[4]] = ring_plane(cell(ru, rn), rhold[PH]);
         }
         __syncthreads();
-        if (z + 1 < ze) put_phi(s_phi[P0]);   // plane z+3 replaces plane z
+        if (z + 1 < ze) put_phi(s_t[P0]);   // plane z+3 replaces plane z
         if (valid) {
             float sum = 0.0f;
-            sum += g0;
             for_links([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
-                if constexpr (l != 0) sum += s_g[(SL::w(l) == TX ? row0 : row1) + SL::src(l)];
+                if constexpr (crosses(l)) sum += s_g[(SL::w(l) == TX ? row0 : row1) + SL::src(l)];
+                else sum += l == 0 ? g0 : (l == 5 ? g5 : g6);
             });
             // Ghost-layer faces take boundaryConditions' copy instead.
             if (c.bc == MCB_BC_REFERENCE && ref_face(G, x, y, z)) sum = ld32(c.phi_prev, ref_clamped(G, x, y, z));
@@ -1546,6 +1576,7 @@ __device__ __forceinline__ void collide_tile_fm(const CaseView& c, int x0, int y
     };
     float hin[9];      // in-plane links (rest first, then c_z = 0 links in link order) for the next plane
     float hup[2][5];   // c_z = +1 links by parity of their destination plane
+    float down6;       // link 6 for the destination plane below (it stays in the column)
     // From a source plane's per-cell values: its c_z = -1 links written for
     // the destination plane below, its in-plane links into hin and its c_z =
     // +1 links into up.
@@ -1554,8 +1585,10 @@ __device__ __forceinline__ void collide_tile_fm(const CaseView& c, int x0, int y
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
             const float v = fluid_post<l>(fc, c.phys, d);
-            if constexpr (CZ[l] < 0) {
+            if constexpr (CZ[l] < 0 && crosses(l)) {
                 if (write_down) own_slot(lc) = v;
+            } else if constexpr (CZ[l] < 0) {
+                down6 = v;
             } else if constexpr (CZ[l] == 0) {
                 hin[ki] = v;
                 ++ki;
@@ -1573,7 +1606,7 @@ __device__ __forceinline__ void collide_tile_fm(const CaseView& c, int x0, int y
                 own_slot(lc) = hin[ki];
                 ++ki;
             } else if constexpr (CZ[l] > 0) {
-                own_slot(lc) = up[ku];
+                if constexpr (crosses(l)) own_slot(lc) = up[ku];
                 ++ku;
             }
         });
@@ -1588,26 +1621,7 @@ __device__ __forceinline__ void collide_tile_fm(const CaseView& c, int x0, int y
     else { hx = TX + 1; hy = min(tid - 2 * TX - TY - 2, TY + 1); side = 3; }
     const unsigned roff4 = (unsigned)(wrapmod(y0 - 1 + hy, G.ny) * G.nx + wrapmod(x0 - 1 + hx, G.nx)) * 4u;
     int rslot[5];
-    {
-        const int sx = hx - 1, sy = hy - 1;
-        auto fill = [&](auto sc) {
-            constexpr int s = decltype(sc)::value;
-            auto one = [&](auto kc) {
-                constexpr int k = decltype(kc)::value;
-                constexpr int l = RING_LINK[s][k];
-                rslot[k] = SL::inside(l, sx, sy) ? SL::at(l, sx, sy) : SL::kSpare;
-            };
-            one(std::integral_constant<int, 0>{});
-            one(std::integral_constant<int, 1>{});
-            one(std::integral_constant<int, 2>{});
-            one(std::integral_constant<int, 3>{});
-            one(std::integral_constant<int, 4>{});
-        };
-        if (side == 0) fill(std::integral_constant<int, 0>{});
-        else if (side == 1) fill(std::integral_constant<int, 1>{});
-        else if (side == 2) fill(std::integral_constant<int, 2>{});
-        else fill(std::integral_constant<int, 3>{});
-    }
+    ring_slots<TX, TY>(side, hx, hy, rslot);
     float rin[3];    // the ring cell's in-plane links for the next plane
     float rup[2];    // its c_z = +1 link by parity of the destination plane
     // The side's five links of a ring cell's plane: in-plane into rin, c_z =
@@ -1671,7 +1685,7 @@ __device__ __forceinline__ void collide_tile_fm(const CaseView& c, int x0, int y
         if (z + 1 < ze) fetch_phi(z + 3);
         // Sources: plane z (held in-plane links), z-1 (held c_z = +1 links),
         // z+1 (built now).
-        const float f0 = hin[0];
+        const float f0 = hin[0], f5 = hup[PAR][0];   // link 5 is the first with c_z = +1
         write_held(hup[PAR]);
         tile_source(fluid_cell_of(v), true, hup[PAR]);
         if (ring) {
@@ -1685,9 +1699,11 @@ __device__ __forceinline__ void collide_tile_fm(const CaseView& c, int x0, int y
         if (!valid) return;
         float fv[Q];
         fv[0] = f0;
+        fv[5] = f5;
+        fv[6] = down6;
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            if constexpr (l != 0) fv[l] = s_f[(SL::w(l) == TX ? row0 : row1) + SL::src(l)];
+            if constexpr (crosses(l)) fv[l] = s_f[(SL::w(l) == TX ? row0 : row1) + SL::src(l)];
         });
         const unsigned fb = (unsigned)(G.n * 4), z4 = (unsigned)(z * G.nxy) * 4u;
         const int sm = nslot(z - 1), s0 = nslot(z), sp = nslot(z + 1);
