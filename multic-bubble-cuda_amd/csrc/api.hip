@@ -479,7 +479,7 @@ mcb_status mcb_create(const mcb_params* p, void* stream, mcb_ctx** out) {
     const long long P = plane_stride(n);
     if (p->storage != MCB_STORE_FP32) {
         c->geo.plane = P;
-        c->batch.reset(new (std::nothrow) Batch(c->device, c->stream, true));
+        c->batch.reset(new (std::nothrow) Batch(c->device, c->stream));
         if (!c->batch) return bail(MCB_ERR_OUT_OF_MEMORY);
         c->tiling = choose_tiling(*p);
     } else if (path == MCB_PATH_FUSED) {
@@ -963,7 +963,7 @@ mcb_status mcb_batch_create(int device, int storage, void* stream, mcb_batch** o
         mcb_batch_destroy(b);
         return MCB_ERR_HIP;
     }
-    b->b.reset(new (std::nothrow) Batch(device, b->stream, true));
+    b->b.reset(new (std::nothrow) Batch(device, b->stream));
     if (!b->b) {
         mcb_batch_destroy(b);
         return MCB_ERR_OUT_OF_MEMORY;
@@ -1020,7 +1020,7 @@ mcb_status mcb_batch_step_timed(mcb_batch* b, int nsteps, double* ms) {
     if (!b || !ms) return MCB_ERR_INVALID_ARG;
     if (hipSetDevice(b->device) != hipSuccess) return MCB_ERR_NO_DEVICE;
     if (b->b->count() > 0) {
-        // Build views, tables and graphs outside the timed region.
+        // Build views and tables outside the timed region.
         mcb_status st = bstat(b, b->b->step(0));
         if (st != MCB_OK) return st;
     }

@@ -22,10 +22,13 @@ unsigned pop_bytes(int storage) { return storage == MCB_STORE_FP32 ? 4u : 2u; }
 
 constexpr int kMacroFields = 10;
 
-// Batches of at least this many cells launch their steps one by one instead
-// of replaying captured step graphs (see rebuild): a step of 8M cells takes
-// ~0.2 ms, several times what enqueueing its launches takes.
-constexpr long long kCellsEager = 8LL << 20;
+// Smallest group that is split for overlap (see rebuild): below, each half is
+// a chain of launches too short to fill the device (a batch of 5.8M cells in
+// FP16 with its largest group split: 199 us per step against 155).
+constexpr long long kSplitCells = 8LL << 20;
+// What a group's launches of a step cost on their lane beside its cells, in
+// cells (about 25 us).
+constexpr long long kGroupCells = 1LL << 20;
 
 // Work items of a case (x fastest, then y, then z chunks), renumbered by
 // xcd_runs: each XCD takes runs of 8 consecutive tiles, so x-neighbouring
@@ -132,12 +135,18 @@ Tiling choose_tiling(const mcb_params& p) {
 }
 
 Tiling batch_tiling(const mcb_params& p) {
-    // FP32 cases of a batch share one tile shape, so a batch step is one phase
-    // and one collide launch for every case: on the 64 'batch' presets (sides
-    // 32-128) 64x8 tiles with 8-plane chunks ran 21.8k MLUPS against 20.5k
-    // with each side's autotuned single-case tile (four launch groups), whose
-    // small groups leave CUs idle while they drain.
-    if (p.storage == MCB_STORE_FP32) return Tiling{64, 8, std::min(8, p.nz)};
+    // FP32, measured on batches of equal cubes (k MLUPS): 64x8 tiles with
+    // 8-plane chunks where they pad rows by less than half a tile (64: 23.3,
+    // 128: 23.5), 32x8 where they would (32: 23.2 against 16.0, 96: 21.8
+    // against 20.3), whole rows of 48 (22.8 against 20.4). The shapes of a
+    // batch run side by side (launch_steps).
+    if (p.storage == MCB_STORE_FP32) {
+        const int over = p.nx % 64;
+        Tiling t = over > 0 && over <= 32 && p.nx < 192 ? Tiling{32, 8, 8} : Tiling{64, 8, 8};
+        if (p.nx == 48) t = Tiling{48, 4, 8};
+        t.zc = std::min(t.zc, p.nz);
+        return t;
+    }
     return choose_tiling(p);
 }
 
@@ -166,16 +175,21 @@ Tiling choose_tiling_single(const mcb_params& p) {
 
 // ------------------------------------------------------------------ Batch
 
-Batch::Batch(int device, hipStream_t stream, bool use_graphs)
-    : device_(device), stream_(stream), use_graphs_(use_graphs) {}
+Batch::Batch(int device, hipStream_t stream) : device_(device), stream_(stream) {}
 
 Batch::~Batch() {
     (void)hipSetDevice(device_);
     (void)hipStreamSynchronize(stream_);
-    for (auto& g : graph_)
-        if (g) (void)hipGraphExecDestroy(g);
-    for (auto& kv : groups_)
-        if (kv.second.d_work) (void)hipFree(kv.second.d_work);
+    for (auto& l : lane_)
+        if (l) {
+            (void)hipStreamSynchronize(l);
+            (void)hipStreamDestroy(l);
+        }
+    if (fork_) (void)hipEventDestroy(fork_);
+    for (auto& e : join_)
+        if (e) (void)hipEventDestroy(e);
+    for (auto& g : groups_)
+        if (g.d_work) (void)hipFree(g.d_work);
     for (auto& v : d_views_)
         if (v) (void)hipFree(v);
     if (d_partial_) (void)hipFree(d_partial_);
@@ -455,8 +469,14 @@ mcb_status Batch::rebuild() {
     B_HIP(hipStreamSynchronize(stream_));
     mcb_status st = ensure_macro_scratch();
     if (st != MCB_OK) return st;
+    // Cases in the order of their groups (tile shape and collide mode).
+    auto key = [&](int id) {
+        const CaseState* c = cases_[id].get();
+        return std::make_tuple(c->tiling.tx, c->tiling.ty, c->mode);
+    };
     order_.clear();
     for (auto& kv : cases_) order_.push_back(kv.first);
+    std::stable_sort(order_.begin(), order_.end(), [&](int a, int b) { return key(a) < key(b); });
     const size_t n = order_.size();
     if (n > views_cap_) {
         for (auto& v : d_views_) {
@@ -468,9 +488,7 @@ mcb_status Batch::rebuild() {
         for (auto& v : d_views_) B_HIP(hipMalloc(reinterpret_cast<void**>(&v), cap * sizeof(CaseView)));
         views_cap_ = cap;
     }
-    std::map<std::tuple<int, int, int>, std::vector<WorkItem>> by_group;
     any_initial_ = false;
-    any_mass_ = false;
     for (int q = 0; q < 2; ++q) hv_[q].clear();
     for (size_t i = 0; i < n; ++i) {
         CaseState* c = cases_[order_[i]].get();
@@ -481,22 +499,51 @@ mcb_status Batch::rebuild() {
             hv_[q].push_back(v);
         }
         if (c->gm == GM_INITIAL) any_initial_ = true;
-        if (c->massq || c->mass) any_mass_ = true;
-        auto tl = tiles_of(*c, (int)i);
-        auto& vec = by_group[std::make_tuple(c->tiling.tx, c->tiling.ty, c->mode)];
-        vec.insert(vec.end(), tl.begin(), tl.end());
         c->slot = (int)i;
     }
     for (int q = 0; q < 2; ++q)
         if (n) B_HIP(hipMemcpyAsync(d_views_[q], hv_[q].data(), n * sizeof(CaseView), hipMemcpyHostToDevice, stream_));
-    for (auto& kv : groups_) kv.second.n = 0;
-    std::vector<std::vector<WorkItem>> staged;
-    for (auto& kv : by_group) {
-        Group& gr = groups_[kv.first];
-        gr.t = Tiling{std::get<0>(kv.first), std::get<1>(kv.first), 0};
-        gr.mode = std::get<2>(kv.first);
-        staged.push_back(xcd_permute(kv.second));
-        const auto& items = staged.back();
+    // Groups, and [start[k], start[k + 1]) their cases. One with more than half
+    // of the work is cut in two, so that there are chains to overlap.
+    auto cells = [&](size_t i) { return cases_[order_[i]]->geo.n; };
+    std::vector<size_t> start;
+    long long total = 0;
+    for (size_t i = 0; i < n; ++i) {
+        if (i == 0 || key(order_[i]) != key(order_[i - 1])) start.push_back(i);
+        total += cells(i);
+    }
+    for (size_t k = 0; k < start.size(); ++k) {
+        const size_t end = k + 1 < start.size() ? start[k + 1] : n;
+        long long work = 0, half = 0;
+        for (size_t i = start[k]; i < end; ++i) work += cells(i);
+        if (2 * work <= total || work < kSplitCells || end - start[k] < 2) continue;
+        size_t cut = start[k];
+        while (cut < end - 1 && 2 * half < work) half += cells(cut++);
+        start.insert(start.begin() + (long)k + 1, cut);
+        break;
+    }
+    n_groups_ = n ? start.size() : 0;
+    if (groups_.size() < n_groups_) groups_.resize(n_groups_);
+    std::vector<std::pair<long long, size_t>> load;   // cost and index of a group
+    for (size_t k = 0; k < n_groups_; ++k) {
+        Group& gr = groups_[k];
+        const size_t end = k + 1 < n_groups_ ? start[k + 1] : n;
+        gr.first = (unsigned)start[k];
+        gr.cases = (unsigned)(end - start[k]);
+        const CaseState* c0 = cases_[order_[start[k]]].get();
+        gr.t = Tiling{c0->tiling.tx, c0->tiling.ty, 0};
+        gr.mode = c0->mode;
+        gr.mass = false;
+        std::vector<WorkItem> items;
+        long long work = 0;
+        for (size_t i = start[k]; i < end; ++i) {
+            const CaseState* c = cases_[order_[i]].get();
+            if (c->massq || c->mass) gr.mass = true;
+            const auto tl = tiles_of(*c, (int)i);
+            items.insert(items.end(), tl.begin(), tl.end());
+            work += c->geo.n;
+        }
+        items = xcd_permute(items);
         if (items.size() > gr.cap) {
             if (gr.d_work) B_HIP(hipFree(gr.d_work));
             gr.d_work = nullptr;
@@ -507,58 +554,52 @@ mcb_status Batch::rebuild() {
         }
         gr.n = (unsigned)items.size();
         B_HIP(hipMemcpyAsync(gr.d_work, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, stream_));
+        B_HIP(hipStreamSynchronize(stream_));   // items is a host temporary
+        load.emplace_back(work + kGroupCells, k);
     }
-    B_HIP(hipStreamSynchronize(stream_));   // hv and staged are host temporaries
-    for (auto& g : graph_) {
-        if (g) B_HIP(hipGraphExecDestroy(g));
-        g = nullptr;
+    B_HIP(hipStreamSynchronize(stream_));   // the copies of hv_
+    // Lanes: each group to the least loaded one, largest first.
+    std::sort(load.rbegin(), load.rend());
+    lanes_ = (int)std::max<size_t>(1, std::min<size_t>(kLanes, n_groups_));
+    long long lane_load[kLanes] = {};
+    for (const auto& l : load) {
+        const int at = (int)(std::min_element(lane_load, lane_load + lanes_) - lane_load);
+        groups_[l.second].lane = at;
+        lane_load[at] += l.first;
     }
-    // Step graphs pay where a step is short next to its launches (a few small
-    // cases); a batch of kCellsEager cells or more keeps the device busy with
-    // launches enqueued one by one, and a serving loop that re-forms it every
-    // round would only pay the capture.
-    long long cells = 0;
-    for (const auto& kv : cases_) cells += kv.second->geo.n;
-    if (use_graphs_ && n && cells < kCellsEager) {
-        for (int q = 0; q < 2; ++q) {
-            hipGraph_t gr = nullptr;
-            if (hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-                (void)hipGetLastError();
-                use_graphs_ = false;
-                break;
-            }
-            mcb_status s1 = launch_step(q), s2 = launch_step(q ^ 1);
-            hipError_t e = hipStreamEndCapture(stream_, &gr);
-            if (s1 != MCB_OK || s2 != MCB_OK || e != hipSuccess) {
-                if (gr) (void)hipGraphDestroy(gr);
-                (void)hipGetLastError();
-                use_graphs_ = false;
-                break;
-            }
-            e = hipGraphInstantiate(&graph_[q], gr, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(gr);
-            if (e != hipSuccess) {
-                (void)hipGetLastError();
-                graph_[q] = nullptr;
-                use_graphs_ = false;
-                break;
-            }
-        }
+    if (lanes_ > 1 && !fork_) B_HIP(hipEventCreateWithFlags(&fork_, hipEventDisableTiming));
+    for (int i = 0; i + 1 < lanes_; ++i) {
+        if (!lane_[i]) B_HIP(hipStreamCreateWithFlags(&lane_[i], hipStreamNonBlocking));
+        if (!join_[i]) B_HIP(hipEventCreateWithFlags(&join_[i], hipEventDisableTiming));
     }
     dirty_ = false;
     return MCB_OK;
 }
 
-mcb_status Batch::launch_step(int q) {
-    for (auto& kv : groups_) {
-        const Group& gr = kv.second;
-        if (gr.n) B_HIP(launch_phase_batch(d_views_[q], gr.d_work, gr.n, gr.t, storage_, stream_));
+mcb_status Batch::launch_steps(int q, int n) {
+    // A caller capturing stream_ gets everything recorded there.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (lanes_ > 1) B_HIP(hipStreamIsCapturing(stream_, &cap));
+    const bool fork = lanes_ > 1 && cap == hipStreamCaptureStatusNone;
+    if (fork) {
+        B_HIP(hipEventRecord(fork_, stream_));
+        for (int i = 0; i + 1 < lanes_; ++i) B_HIP(hipStreamWaitEvent(lane_[i], fork_, 0));
     }
-    if (any_mass_) B_HIP(launch_mass_finish(d_views_[q], (unsigned)order_.size(), stream_));
-    for (auto& kv : groups_) {
-        const Group& gr = kv.second;
-        if (gr.n) B_HIP(launch_collide_batch(d_views_[q], gr.d_work, gr.n, gr.t, gr.mode, storage_, stream_));
+    hipError_t e = hipSuccess;
+    for (int k = 0; k < n && e == hipSuccess; ++k, q ^= 1)
+        for (size_t i = 0; i < n_groups_ && e == hipSuccess; ++i) {
+            const Group& gr = groups_[i];
+            const hipStream_t s = fork && gr.lane ? lane_[gr.lane - 1] : stream_;
+            e = launch_phase_batch(d_views_[q], gr.d_work, gr.n, gr.t, storage_, s);
+            if (e == hipSuccess && gr.mass) e = launch_mass_finish(d_views_[q] + gr.first, gr.cases, s);
+            if (e == hipSuccess) e = launch_collide_batch(d_views_[q], gr.d_work, gr.n, gr.t, gr.mode, storage_, s);
+        }
+    // Also after an error: whatever was launched is ordered before stream_'s next work.
+    for (int i = 0; fork && i + 1 < lanes_; ++i) {
+        B_HIP(hipEventRecord(join_[i], lane_[i]));
+        B_HIP(hipStreamWaitEvent(stream_, join_[i], 0));
     }
+    B_HIP(e);
     return MCB_OK;
 }
 
@@ -575,8 +616,8 @@ mcb_status Batch::step(int nsteps) {
     if (any_initial_) {
         // The first step of moment-form cases reads their initial state; the
         // view of that parity then switches to the moment form (stream-ordered
-        // copy from the persistent host array, so graphs see it).
-        mcb_status st = launch_step(parity_);
+        // copy from the persistent host array).
+        mcb_status st = launch_steps(parity_, 1);
         if (st != MCB_OK) return st;
         const int q = parity_;
         parity_ ^= 1;
@@ -590,16 +631,10 @@ mcb_status Batch::step(int nsteps) {
         }
         any_initial_ = false;
     }
-    while (left > 0) {
-        if (use_graphs_ && graph_[parity_] && left >= 2) {
-            B_HIP(hipGraphLaunch(graph_[parity_], stream_));
-            left -= 2;
-        } else {
-            mcb_status st = launch_step(parity_);
-            if (st != MCB_OK) return st;
-            parity_ ^= 1;
-            left -= 1;
-        }
+    if (left > 0) {
+        mcb_status st = launch_steps(parity_, left);
+        if (st != MCB_OK) return st;
+        parity_ ^= left & 1;
     }
     batch_steps_ += nsteps;
     macro_id_ = 0;  // the macro fields no longer match any case's state
@@ -947,7 +982,7 @@ mcb_status autotune(const mcb_params& p0, int device, Tiling* best, double* ms_p
     double best_ms = 1e30;
     Tiling best_t = choose_tiling(p);
     {
-        Batch b(device, s, false);
+        Batch b(device, s);
         // A centred bubble of radius nx/4 as the scratch state.
         mcb_bubble bub{p.nx * 0.5f, p.ny * 0.5f, p.nz * 0.5f, p.nx * 0.25f};
         int id = 0;

@@ -1,13 +1,13 @@
 // Batched execution of many independent cases on one device.
 //
 // Every case keeps its own lattice, parameters and buffers resident in HBM.
-// A batch step runs the phase pass of all cases, then the collide pass of all
-// cases, each as one launch per tile-shape group: workgroups read a work
-// item (case, tile origin) from a table built in XCD order, then a CaseView
-// from a device array. Two batch steps (both A/B parities) are captured in a
-// hipGraph and replayed; the graph is rebuilt when cases join or leave.
-// Cases never exchange data, so each case's numbers do not depend on what
-// else is in the batch.
+// A batch step runs, for each group of cases of one tile shape, the phase pass
+// of its cases and then their collide pass, one launch each: workgroups read a
+// work item (case, tile origin) from a table built in XCD order, then a
+// CaseView from a device array. Cases never exchange data, so each case's
+// numbers do not depend on what else is in the batch, and the groups advance
+// independently: they run side by side on a few streams (lanes), where one
+// group's drain and its phase pass overlap another's collide pass.
 #pragma once
 #include <map>
 #include <memory>
@@ -70,7 +70,7 @@ size_t case_bytes(const mcb_params& p);
 
 class Batch {
 public:
-    Batch(int device, hipStream_t stream, bool use_graphs);
+    Batch(int device, hipStream_t stream);
     ~Batch();
     Batch(const Batch&) = delete;
     Batch& operator=(const Batch&) = delete;
@@ -114,7 +114,8 @@ private:
     void dev_release(void* ptr, size_t bytes);
     mcb_status build_own_table(CaseState* c);
     mcb_status rebuild();
-    mcb_status launch_step(int q);
+    // n steps from parity q for every group, on the lanes; stream_ waits for all.
+    mcb_status launch_steps(int q, int n);
     // 16-bit storage: reset the mass target and the pending corrections.
     mcb_status set_mass_target(CaseState* c, double target);
     // Keep g as populations from here on (arbitrary g has no moment form):
@@ -133,10 +134,9 @@ private:
 
     int device_;
     hipStream_t stream_;
-    bool use_graphs_;
     std::string err_;
     std::map<int, std::unique_ptr<CaseState>> cases_;
-    std::vector<int> order_;          // case ids in view-array order
+    std::vector<int> order_;          // case ids in view-array order (by group)
     int next_id_ = 1;
     int parity_ = 0;
     long long batch_steps_ = 0;
@@ -145,19 +145,26 @@ private:
     // device arrays
     CaseView* d_views_[2] = {nullptr, nullptr};
     size_t views_cap_ = 0;
+    // Cases of one tile shape and collide mode: views [first, first + cases) of
+    // the arrays, one work table, one lane.
     struct Group {
         Tiling t{};
         int mode = COLLIDE_STEP;
         WorkItem* d_work = nullptr;
         size_t cap = 0;
         unsigned n = 0;
+        unsigned first = 0, cases = 0;
+        bool mass = false;               // a case keeps a mass-drift correction (MassCell or MassQ)
+        int lane = 0;                    // 0: stream_, i: lane_[i - 1]
     };
-    // Launch groups by (tile x, tile y, collide mode), kept across rebuilds.
-    std::map<std::tuple<int, int, int>, Group> groups_;
+    std::vector<Group> groups_;          // the first n_groups_ are in use (tables are kept for reuse)
+    size_t n_groups_ = 0;
+    static constexpr int kLanes = 4;     // hardware queues of a process
+    hipStream_t lane_[kLanes - 1] = {};  // created when a batch first needs them
+    hipEvent_t fork_ = nullptr, join_[kLanes - 1] = {};
+    int lanes_ = 1;                      // lanes in use
     std::vector<CaseView> hv_[2];     // host copies of the view arrays
     bool any_initial_ = false;        // a moment-form case has not stepped yet
-    bool any_mass_ = false;          // a case keeps a mass-drift correction (MassCell or MassQ)
-    hipGraphExec_t graph_[2] = {nullptr, nullptr};
     double* d_partial_ = nullptr;     // reduction scratch (2 * kReduceBlocks + 2 doubles)
     std::vector<void*> macro_bufs_;
     size_t macro_plane_ = 0;
@@ -174,8 +181,8 @@ Tiling choose_tiling(const mcb_params& p);
 // The tiling of a single-case context: as choose_tiling, with z-chunks short
 // enough that a small lattice alone still fills the device.
 Tiling choose_tiling_single(const mcb_params& p);
-// The tiling of a batch case: one shape for all FP32 cases (one launch per
-// pass), the 16-bit rule of choose_tiling otherwise.
+// The tiling of a batch case, where the batch fills the device: by row length
+// in FP32, the 16-bit rule of choose_tiling otherwise.
 Tiling batch_tiling(const mcb_params& p);
 // Measure every supported tile shape and z-chunk on a scratch case and
 // remember the fastest for (nx, ny, nz, storage).

@@ -5,7 +5,7 @@
 // the head of the queue is admitted while its footprint fits the device-memory
 // budget next to the resident cases (arrival order, no overtaking); the
 // resident cases then advance together by min(tick, fewest steps left) steps
-// (one batch launch per pass, graph-replayed); cases that reached their step
+// (see batch.hpp); cases that reached their step
 // count are read out (FP64 sum of phi and kinetic energy, optional phi) and
 // leave, returning their memory to a pool that later cases of the same size
 // reuse. Cases never exchange data, so a request's numbers are the same
@@ -170,7 +170,7 @@ mcb_status serve_batched(const mcb_serve_config& cfg, const mcb_request* reqs, i
         budget = (size_t)(0.9 * (double)free_b);
     }
     const int tick = cfg.tick_steps > 0 ? cfg.tick_steps : 100;
-    Batch batch(cfg.device, stream, true);
+    Batch batch(cfg.device, stream);
     // Freed case buffers are kept for later cases of the same sizes, within
     // the budget that resident cases leave unused.
     batch.set_pool_limit(budget);
@@ -243,7 +243,7 @@ mcb_status serve_batched(const mcb_serve_config& cfg, const mcb_request* reqs, i
         st->rounds += 1;
         const Clock::time_point tr = Clock::now();
         // Read out every case that is done, then release them all: a removal
-        // re-forms the batch (work lists, views, step graphs) before the next
+        // re-forms the batch (work lists, views) before the next
         // macro pass, so removing between read-outs would re-form it once per
         // finished case instead of once per round.
         for (Resident& a : active) {

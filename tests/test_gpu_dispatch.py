@@ -39,3 +39,41 @@ def test_phase_pass_chunks(gpu_lib, nx, ny, nz, normals):
 
 def test_phase_pass_ghost_layers(gpu_lib):
     fp32_matches_oracle(gpu_lib, 6, 66, 19, 70, tau_g=1.0, bc_mode=gpu_lib.BC_REFERENCE, weights=gpu_lib.WEIGHTS_LITERAL)
+
+
+@pytest.mark.parametrize("nx,ny,nz,tau_g", [(64, 64, 5, 0.8), (64, 70, 64, 1.0), (40, 33, 29, 1.0), (96, 20, 40, 0.8),
+                                            (16, 24, 18, 1.0)])
+def test_small_lattice_tiles(gpu_lib, nx, ny, nz, tau_g):
+    fp32_matches_oracle(gpu_lib, 4, nx, ny, nz, tau_g=tau_g)
+
+
+def alone(mcb, p, bubble, steps):
+    lat = mcb.Lattice(p)
+    lat.init_bubbles([bubble], 3.0)
+    lat.step(steps)
+    phi = lat.read("phi")
+    lat.close()
+    return phi
+
+
+@pytest.mark.parametrize("storage", [0, 1])
+def test_batch_groups_side_by_side(gpu_lib, storage):
+    """Cases of several tile shapes, one shape large enough to be split over two lanes: every case as if alone, across
+    steps, a join at odd parity and a leave."""
+    mcb = gpu_lib
+    sides = [(192, 160, 150), (192, 160, 150), (48, 40, 20), (96, 33, 17), (32, 32, 32), (70, 21, 30)]
+    with mcb.Batch(storage) as b:
+        ids = []
+        for i, (nx, ny, nz) in enumerate(sides):
+            p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.55 + 0.02 * i)
+            bub = (0.4 * nx, 0.5 * ny, 0.6 * nz, 0.28 * min(nx, ny, nz))
+            if i == 4:
+                b.step(3)
+            ids.append((b.add(p, [bub], 3.0), p, bub, 7 if i < 4 else 4))
+        b.step(1)
+        gone = ids.pop(3)
+        b.remove(gone[0])
+        b.step(3)
+        for cid, p, bub, steps in ids:
+            got, want = b.read(cid, "phi"), alone(mcb, p, bub, steps)
+            assert np.array_equal(got, want), (p.nx, p.ny, p.nz, int(np.count_nonzero(got != want)))
