@@ -481,7 +481,7 @@ mcb_status mcb_create(const mcb_params* p, void* stream, mcb_ctx** out) {
         c->geo.plane = P;
         c->batch.reset(new (std::nothrow) Batch(c->device, c->stream));
         if (!c->batch) return bail(MCB_ERR_OUT_OF_MEMORY);
-        c->tiling = choose_tiling(*p);
+        c->tiling = choose_tiling_single(*p);
     } else if (path == MCB_PATH_FUSED) {
         c->geo.plane = P;
         // At tau_g = 1 g is kept in moment form: phi (two buffers), u and n

@@ -156,20 +156,25 @@ Tiling choose_tiling_single(const mcb_params& p) {
         auto it = g_tuned.find(std::make_tuple(p.nx, p.ny, p.nz, p.storage));
         if (it != g_tuned.end()) return it->second;
     }
-    // A lattice alone on the device: shorter z-chunks until the pass has two
-    // workgroups per CU (256 CUs), down to 4 planes. The reference preset
-    // (64x64x256) gets 8 tiles per z layer at 64x8, i.e. 128 workgroups with
-    // 16-plane chunks, which leaves half the CUs idle.
+    // A lattice alone on the device: shorter z-chunks until its workgroups
+    // have 16 waves for every CU (256 CUs; what 128 VGPRs allow), whatever the
+    // tile. FP32 (us per collide): the reference preset (64x64x256) 64x8x4,
+    // 64^3 64x8x1 20.2 (64x4x4: 25.6). 16 bits (us per step): 117x90x133
+    // 64x4x4 65 (64x8x32, sized for a full device, 147), 128^3 64x4x8 64
+    // (64x4x16 75), 64^3 64x4x2 22.6 (64x4x16 54).
     Tiling t = choose_tiling(p);
-    auto tiles = [&](const Tiling& q) {
-        return (long long)((p.nx + q.tx - 1) / q.tx) * ((p.ny + q.ty - 1) / q.ty) * ((p.nz + q.zc - 1) / q.zc);
+    const bool fp32 = p.storage == MCB_STORE_FP32;
+    auto lanes = [&](const Tiling& q) {
+        return (long long)((p.nx + q.tx - 1) / q.tx) * ((p.ny + q.ty - 1) / q.ty) * ((p.nz + q.zc - 1) / q.zc) * q.tx *
+               q.ty;
     };
-    while (t.zc > 4 && tiles(t) < 512) t.zc /= 2;
-    // Where the chunks are already down to 4 planes, 4-row tiles give twice
-    // the workgroups for the same halo restaging per plane (the reference
-    // preset: 64x4x4 0.0591-0.0595 ms per step against 0.0610-0.0613 with
-    // 64x8x4; 64^3: 0.0317 against 0.0363 ms).
-    if (t.zc <= 4 && t.tx == 64 && t.ty == 8 && p.storage == MCB_STORE_FP32) t.ty = 4;
+    while (t.zc > (fp32 ? 1 : 2) && lanes(t) < 256 * 16 * 64) t.zc /= 2;
+    // Where the chunks are down to 4 planes, 4-row tiles give twice the
+    // workgroups for the same halo restaging per plane (the reference
+    // preset: 64x4x4 43.9 us per collide against 46.4 with 64x8x4); with one
+    // or two planes a tile's own halo weighs more (64^3: 64x8x1 20.2, 64x4x1
+    // 22.4; 16 bits keep 4 rows, 2 planes being their least).
+    if (t.zc <= 4 && (t.zc > 2 || !fp32) && t.tx == 64 && t.ty == 8) t.ty = 4;
     return t;
 }
 
