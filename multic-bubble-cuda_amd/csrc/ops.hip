@@ -2,7 +2,7 @@
 // kernel of src/kernels.cuh, on the reference's SoA layout. Thread per cell,
 // 64-wide rows along x (one wave64 per row segment) instead of the reference's
 // 8x8x8 blocks, so every population plane is read and written in 256-byte
-// runs. The per-cell arithmetic lives in lattice.hpp and is shared with the
+// runs; the boundary kernels run over the faces. The per-cell arithmetic lives in lattice.hpp and is shared with the
 // fused step kernels.
 #include "bubble.hpp"
 #include "common.hpp"
@@ -38,9 +38,32 @@ __device__ __forceinline__ long long lin(int i, int j, int k, const Geo& g) {
     return (long long)k * g.nxy + (long long)j * g.nx + i;
 }
 
-template <int L> __device__ __forceinline__ long long nbr(int i, int j, int k, const Geo& g) {
-    return lin(shift<CX[L]>(i, g.nx), shift<CY[L]>(j, g.ny), shift<CZ[L]>(k, g.nz), g);
+// Element access at an offset from a wave-uniform pointer. The kernels of the
+// loop read and write up to 51 values per cell, and 64-bit addresses per lane
+// cost as many instructions as their arithmetic (gradCalc on 64x64x256: 8.2 us,
+// bound by them). Below 2^30 cells (Off = unsigned) an access is a scalar base
+// and a 32-bit byte offset; larger lattices keep 64-bit offsets.
+template <class Off> __device__ __forceinline__ float get(const float* base, Off o) {
+    if constexpr (sizeof(Off) == 4) return ld32(base, o);
+    else return base[o];
 }
+template <class Off> __device__ __forceinline__ void put(float* base, Off o, float v) {
+    if constexpr (sizeof(Off) == 4) st32(base, o, v);
+    else base[o] = v;
+}
+
+// A cell's offset and those of its neighbours x + SIGN c_l, periodic.
+template <class Off> struct Here {
+    Off xs[3], ys[3], zs[3];
+    __device__ __forceinline__ Here(int i, int j, int k, const Geo& g)
+        : xs{(Off)shift<-1>(i, g.nx), (Off)i, (Off)shift<1>(i, g.nx)},
+          ys{(Off)shift<-1>(j, g.ny) * (Off)g.nx, (Off)j * (Off)g.nx, (Off)shift<1>(j, g.ny) * (Off)g.nx},
+          zs{(Off)shift<-1>(k, g.nz) * (Off)g.nxy, (Off)k * (Off)g.nxy, (Off)shift<1>(k, g.nz) * (Off)g.nxy} {}
+    __device__ __forceinline__ Off me() const { return zs[1] + ys[1] + xs[1]; }
+    template <int L, int SIGN = 1> __device__ __forceinline__ Off nb() const {
+        return zs[1 + SIGN * CZ[L]] + ys[1 + SIGN * CY[L]] + xs[1 + SIGN * CX[L]];
+    }
+};
 
 // ------------------------------------------------------------------ init.cu
 
@@ -87,66 +110,83 @@ __global__ __launch_bounds__(256) void k_initDist(const float* rho, const float*
 
 // ------------------------------------------------------------------- lbm.cu
 
-__global__ __launch_bounds__(256) void k_phiCalc(float* phi, const float* g, OpArgs a) {
+template <class Off> __global__ __launch_bounds__(256) void k_phiCalc(float* phi, const float* g, OpArgs a) {
     int i, j, k;
     if (!cell_of(a, true, i, j, k)) return;
-    const long long x = lin(i, j, k, a.geo);
+    const Off x = Here<Off>(i, j, k, a.geo).me();
     float sum = 0.0f;
-    for_links([&](auto lc) { sum += g[x + decltype(lc)::value * a.geo.plane]; });
-    phi[x] = sum;
+    for_links([&](auto lc) { sum += get(g + decltype(lc)::value * a.geo.plane, x); });
+    put(phi, x, sum);
 }
 
+template <class Off>
 __global__ __launch_bounds__(256) void k_gradCalc(const float* phi, float* normx, float* normy, float* normz,
                                                   float* indicator, OpArgs a) {
     int i, j, k;
     if (!cell_of(a, true, i, j, k)) return;
     const Derived d(a.phys);
+    const Here<Off> h(i, j, k, a.geo);
     float nx, ny, nz, ind;
-    grad_normal([&](auto lc) { return phi[nbr<decltype(lc)::value>(i, j, k, a.geo)]; }, d, nx, ny, nz, ind);
-    const long long x = lin(i, j, k, a.geo);
-    normx[x] = nx; normy[x] = ny; normz[x] = nz; indicator[x] = ind;
+    grad_normal([&](auto lc) { return get(phi, h.template nb<decltype(lc)::value>()); }, d, nx, ny, nz, ind);
+    const Off x = h.me();
+    put(normx, x, nx);
+    put(normy, x, ny);
+    put(normz, x, nz);
+    put(indicator, x, ind);
 }
 
+template <class Off>
 __global__ __launch_bounds__(256) void k_curvatureCalc(float* curvature, const float* indicator, const float* normx,
                                                        const float* normy, const float* normz, float* ffx, float* ffy,
                                                        float* ffz, OpArgs a) {
     int i, j, k;
     if (!cell_of(a, true, i, j, k)) return;
     const Derived d(a.phys);
-    const long long x = lin(i, j, k, a.geo);
+    const Here<Off> h(i, j, k, a.geo);
+    const Off x = h.me();
     float curv, fx, fy, fz;
     curvature_force(
         [&](auto lc, float& ax, float& ay, float& az) {
             constexpr int l = decltype(lc)::value;
-            const long long o = nbr<l>(i, j, k, a.geo);
-            if constexpr (CX[l] != 0) ax = normx[o];
-            if constexpr (CY[l] != 0) ay = normy[o];
-            if constexpr (CZ[l] != 0) az = normz[o];
+            const Off o = h.template nb<l>();
+            if constexpr (CX[l] != 0) ax = get(normx, o);
+            if constexpr (CY[l] != 0) ay = get(normy, o);
+            if constexpr (CZ[l] != 0) az = get(normz, o);
         },
-        a.phys, d, normx[x], normy[x], normz[x], indicator[x], curv, fx, fy, fz);
-    curvature[x] = curv;
-    ffx[x] = fx; ffy[x] = fy; ffz[x] = fz;
+        a.phys, d, get(normx, x), get(normy, x), get(normz, x), get(indicator, x), curv, fx, fy, fz);
+    put(curvature, x, curv);
+    put(ffx, x, fx);
+    put(ffy, x, fy);
+    put(ffz, x, fz);
 }
 
+template <class Off>
 __global__ __launch_bounds__(256) void k_momentiCalc(float* ux, float* uy, float* uz, float* rho, const float* ffx,
                                                      const float* ffy, const float* ffz, const float* f, float* pxx,
                                                      float* pyy, float* pzz, float* pxy, float* pxz, float* pyz,
                                                      OpArgs a) {
     int i, j, k;
     if (!cell_of(a, true, i, j, k)) return;
-    const long long x = lin(i, j, k, a.geo);
+    const Off x = Here<Off>(i, j, k, a.geo).me();
     float fv[Q];
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        fv[l] = f[x + l * a.geo.plane];
+        fv[l] = get(f + l * a.geo.plane, x);
     });
-    const Moments m = moments(fv, a.phys, ffx[x], ffy[x], ffz[x]);
-    pxx[x] = m.pxx; pyy[x] = m.pyy; pzz[x] = m.pzz;
-    pxy[x] = m.pxy; pxz[x] = m.pxz; pyz[x] = m.pyz;
-    ux[x] = m.ux; uy[x] = m.uy; uz[x] = m.uz;
-    rho[x] = m.rho;
+    const Moments m = moments(fv, a.phys, get(ffx, x), get(ffy, x), get(ffz, x));
+    put(pxx, x, m.pxx);
+    put(pyy, x, m.pyy);
+    put(pzz, x, m.pzz);
+    put(pxy, x, m.pxy);
+    put(pxz, x, m.pxz);
+    put(pyz, x, m.pyz);
+    put(ux, x, m.ux);
+    put(uy, x, m.uy);
+    put(uz, x, m.uz);
+    put(rho, x, m.rho);
 }
 
+template <class Off>
 __global__ __launch_bounds__(256) void k_collisionFluid(float* f, const float* ux, const float* uy, const float* uz,
                                                         const float* ffx, const float* ffy, const float* ffz,
                                                         const float* rho, const float* pxx, const float* pyy,
@@ -155,55 +195,108 @@ __global__ __launch_bounds__(256) void k_collisionFluid(float* f, const float* u
     int i, j, k;
     if (!cell_of(a, true, i, j, k)) return;
     const Derived d(a.phys);
-    const long long x = lin(i, j, k, a.geo);
+    const Here<Off> h(i, j, k, a.geo);
+    const Off x = h.me();
     Moments m;
-    m.rho = rho[x]; m.ux = ux[x]; m.uy = uy[x]; m.uz = uz[x];
-    m.pxx = pxx[x]; m.pyy = pyy[x]; m.pzz = pzz[x];
-    m.pxy = pxy[x]; m.pxz = pxz[x]; m.pyz = pyz[x];
-    const FluidCell c = fluid_cell(m, ffx[x], ffy[x], ffz[x]);
+    m.rho = get(rho, x);
+    m.ux = get(ux, x);
+    m.uy = get(uy, x);
+    m.uz = get(uz, x);
+    m.pxx = get(pxx, x);
+    m.pyy = get(pyy, x);
+    m.pzz = get(pzz, x);
+    m.pxy = get(pxy, x);
+    m.pxz = get(pxz, x);
+    m.pyz = get(pyz, x);
+    const FluidCell c = fluid_cell(m, get(ffx, x), get(ffy, x), get(ffz, x));
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        f[nbr<l>(i, j, k, a.geo) + l * a.geo.plane] = fluid_post<l>(c, a.phys, d);
+        put(f + l * a.geo.plane, h.template nb<l>(), fluid_post<l>(c, a.phys, d));
     });
 }
 
+template <class Off>
 __global__ __launch_bounds__(256) void k_collisionPhase(float* g, const float* ux, const float* uy, const float* uz,
                                                         const float* phi, const float* normx, const float* normy,
                                                         const float* normz, OpArgs a) {
     int i, j, k;
     if (!cell_of(a, true, i, j, k)) return;
     const Derived d(a.phys);
-    const long long x = lin(i, j, k, a.geo);
-    const PhaseCell c = phase_cell(a.phys, phi[x], ux[x], uy[x], uz[x], normx[x], normy[x], normz[x]);
+    const Off x = Here<Off>(i, j, k, a.geo).me();
+    const PhaseCell c = phase_cell(a.phys, get(phi, x), get(ux, x), get(uy, x), get(uz, x), get(normx, x),
+                                   get(normy, x), get(normz, x));
     if (a.tau_g_one) {
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            g[x + l * a.geo.plane] = phase_post<l>(c, a.phys);
+            put(g + l * a.geo.plane, x, phase_post<l>(c, a.phys));
         });
     } else {
+        float pre[Q];
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            const long long o = x + l * a.geo.plane;
-            g[o] = phase_post_bgk<l>(c, a.phys, d, g[o]);
+            pre[l] = get(g + l * a.geo.plane, x);
+        });
+        for_links([&](auto lc) {
+            constexpr int l = decltype(lc)::value;
+            put(g + l * a.geo.plane, x, phase_post_bgk<l>(c, a.phys, d, pre[l]));
         });
     }
 }
 
-__global__ __launch_bounds__(256) void k_streamingCalc(const float* g, float* g_out, OpArgs a) {
+template <class Off> __global__ __launch_bounds__(256) void k_streamingCalc(const float* g, float* g_out, OpArgs a) {
     int i, j, k;
     if (!cell_of(a, false, i, j, k)) return;
-    const long long x = lin(i, j, k, a.geo);
+    const Here<Off> h(i, j, k, a.geo);
+    float v[Q];
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        const long long src = lin(shift<-CX[l]>(i, a.geo.nx), shift<-CY[l]>(j, a.geo.ny), shift<-CZ[l]>(k, a.geo.nz), a.geo);
-        g_out[x + l * a.geo.plane] = g[src + l * a.geo.plane];
+        v[l] = get(g + l * a.geo.plane, h.template nb<l, -1>());
     });
+    for_links([&](auto lc) {
+        constexpr int l = decltype(lc)::value;
+        put(g_out + l * a.geo.plane, h.me(), v[l]);
+    });
+}
+
+// Cell e of the lattice's faces: the two z faces, then the two y faces and the
+// two x faces without the cells of those before, x (or y) fastest. Launched
+// over the faces only: with a thread per cell of the lattice nearly every wave
+// held a face lane or two (x = 0, x = nx - 1) and walked through all links for
+// them (fgBoundary on 64x64x256: 27.6 us for 7% of the cells).
+__host__ __device__ __forceinline__ long long face_cells(const Geo& g) {
+    return 2LL * g.nxy + 2LL * g.nx * (g.nz - 2) + 2LL * (g.ny - 2) * (g.nz - 2);
+}
+__device__ __forceinline__ bool face_of(long long e, const Geo& g, int& i, int& j, int& k) {
+    if (e < 2LL * g.nxy) {
+        const unsigned r = (unsigned)(e % g.nxy);
+        k = e < g.nxy ? 0 : g.nz - 1;
+        j = (int)(r / (unsigned)g.nx);
+        i = (int)(r % (unsigned)g.nx);
+        return true;
+    }
+    e -= 2LL * g.nxy;
+    const long long ny_face = (long long)g.nx * (g.nz - 2), nx_face = (long long)(g.ny - 2) * (g.nz - 2);
+    if (e < 2 * ny_face) {
+        const unsigned r = (unsigned)(e % ny_face);
+        j = e < ny_face ? 0 : g.ny - 1;
+        k = 1 + (int)(r / (unsigned)g.nx);
+        i = (int)(r % (unsigned)g.nx);
+        return true;
+    }
+    e -= 2 * ny_face;
+    if (e < 2 * nx_face) {
+        const unsigned r = (unsigned)(e % nx_face);
+        i = e < nx_face ? 0 : g.nx - 1;
+        k = 1 + (int)(r / (unsigned)(g.ny - 2));
+        j = 1 + (int)(r % (unsigned)(g.ny - 2));
+        return true;
+    }
+    return false;
 }
 
 __global__ __launch_bounds__(256) void k_fgBoundary(float* f, const float* rho, float* g, const float* phi, OpArgs a) {
     int i, j, k;
-    if (!cell_of(a, false, i, j, k)) return;
-    if (is_interior(i, j, k, a.geo)) return;
+    if (!face_of((long long)blockIdx.x * 256 + threadIdx.x, a.geo, i, j, k)) return;
     const long long x = lin(i, j, k, a.geo);
     const float r = rho[x], ph = phi[x];
     auto inside = [&](int ni, int nj, int nk) {
@@ -212,12 +305,10 @@ __global__ __launch_bounds__(256) void k_fgBoundary(float* f, const float* rho, 
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
         const int ni = i + CX[l], nj = j + CY[l], nk = k + CZ[l];
-        if (inside(ni, nj, nk)) f[lin(ni, nj, nk, a.geo) + l * a.geo.plane] = r * a.phys.w[WC[l]];
-    });
-    for_links([&](auto lc) {
-        constexpr int l = decltype(lc)::value;
-        const int ni = i + CX[l], nj = j + CY[l], nk = k + CZ[l];
-        if (inside(ni, nj, nk)) g[lin(ni, nj, nk, a.geo) + l * a.geo.plane] = ph * a.phys.w[WC[l]];
+        if (!inside(ni, nj, nk)) return;
+        const long long o = lin(ni, nj, nk, a.geo) + l * a.geo.plane;
+        f[o] = r * a.phys.w[WC[l]];
+        g[o] = ph * a.phys.w[WC[l]];
     });
 }
 
@@ -227,8 +318,7 @@ __global__ __launch_bounds__(256) void k_fgBoundary(float* f, const float* rho, 
 // nodes only read interior nodes.
 __global__ __launch_bounds__(256) void k_boundaryConditions(float* phi, OpArgs a) {
     int i, j, k;
-    if (!cell_of(a, false, i, j, k)) return;
-    if (is_interior(i, j, k, a.geo)) return;
+    if (!face_of((long long)blockIdx.x * 256 + threadIdx.x, a.geo, i, j, k)) return;
     const int ci = min(max(i, 1), a.geo.nx - 2);
     const int cj = min(max(j, 1), a.geo.ny - 2);
     const int ck = min(max(k, 1), a.geo.nz - 2);
@@ -283,6 +373,15 @@ OpArgs make_args(int NX, int NY, int NZ, const mcb_op_consts* c) {
 dim3 grid_of(const Geo& g) { return dim3((g.nx + OBX - 1) / OBX, (g.ny + OBY - 1) / OBY, g.nz); }
 const dim3 kBlock(OBX, OBY, 1);
 
+dim3 face_grid(const Geo& g) { return dim3((unsigned)((face_cells(g) + 255) / 256)); }
+
+// Launches kernel K<Off> over the cells with the offset type the lattice needs.
+#define MCB_LAUNCH_CELLS(K, ...)                                                                            \
+    do {                                                                                                    \
+        if (a.geo.n < (1LL << 30)) hipLaunchKernelGGL(K<unsigned>, grid_of(a.geo), kBlock, 0, s, __VA_ARGS__); \
+        else hipLaunchKernelGGL(K<long long>, grid_of(a.geo), kBlock, 0, s, __VA_ARGS__);                   \
+    } while (0)
+
 mcb_status launched() { return hip_status(hipGetLastError()); }
 
 template <class... P> bool any_null(P... p) { return ((p == nullptr) || ...); }
@@ -328,14 +427,14 @@ mcb_status mcb_initDist(const float* rho, const float* phi, float* f, float* g, 
 
 mcb_status mcb_phiCalc(float* phi, const float* g, int NX, int NY, int NZ, const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(phi, g);
-    hipLaunchKernelGGL(k_phiCalc, grid_of(a.geo), kBlock, 0, s, phi, g, a);
+    MCB_LAUNCH_CELLS(k_phiCalc, phi, g, a);
     return launched();
 }
 
 mcb_status mcb_gradCalc(const float* phi, float* normx, float* normy, float* normz, float* indicator, int NX, int NY,
                         int NZ, const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(phi, normx, normy, normz, indicator);
-    hipLaunchKernelGGL(k_gradCalc, grid_of(a.geo), kBlock, 0, s, phi, normx, normy, normz, indicator, a);
+    MCB_LAUNCH_CELLS(k_gradCalc, phi, normx, normy, normz, indicator, a);
     return launched();
 }
 
@@ -343,7 +442,7 @@ mcb_status mcb_curvatureCalc(float* curvature, const float* indicator, const flo
                              const float* normz, float* ffx, float* ffy, float* ffz, int NX, int NY, int NZ,
                              const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(curvature, indicator, normx, normy, normz, ffx, ffy, ffz);
-    hipLaunchKernelGGL(k_curvatureCalc, grid_of(a.geo), kBlock, 0, s, curvature, indicator, normx, normy, normz, ffx,
+    MCB_LAUNCH_CELLS(k_curvatureCalc, curvature, indicator, normx, normy, normz, ffx,
                        ffy, ffz, a);
     return launched();
 }
@@ -352,7 +451,7 @@ mcb_status mcb_momentiCalc(float* ux, float* uy, float* uz, float* rho, const fl
                            const float* ffz, const float* f, float* pxx, float* pyy, float* pzz, float* pxy,
                            float* pxz, float* pyz, int NX, int NY, int NZ, const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(ux, uy, uz, rho, ffx, ffy, ffz, f, pxx, pyy, pzz, pxy, pxz, pyz);
-    hipLaunchKernelGGL(k_momentiCalc, grid_of(a.geo), kBlock, 0, s, ux, uy, uz, rho, ffx, ffy, ffz, f, pxx, pyy, pzz,
+    MCB_LAUNCH_CELLS(k_momentiCalc, ux, uy, uz, rho, ffx, ffy, ffz, f, pxx, pyy, pzz,
                        pxy, pxz, pyz, a);
     return launched();
 }
@@ -362,7 +461,7 @@ mcb_status mcb_collisionFluid(float* f, const float* ux, const float* uy, const 
                               const float* pzz, const float* pxy, const float* pxz, const float* pyz, int NX, int NY,
                               int NZ, const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(f, ux, uy, uz, ffx, ffy, ffz, rho, pxx, pyy, pzz, pxy, pxz, pyz);
-    hipLaunchKernelGGL(k_collisionFluid, grid_of(a.geo), kBlock, 0, s, f, ux, uy, uz, ffx, ffy, ffz, rho, pxx, pyy,
+    MCB_LAUNCH_CELLS(k_collisionFluid, f, ux, uy, uz, ffx, ffy, ffz, rho, pxx, pyy,
                        pzz, pxy, pxz, pyz, a);
     return launched();
 }
@@ -371,7 +470,7 @@ mcb_status mcb_collisionPhase(float* g, const float* ux, const float* uy, const 
                               const float* normx, const float* normy, const float* normz, int NX, int NY, int NZ,
                               const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(g, ux, uy, uz, phi, normx, normy, normz);
-    hipLaunchKernelGGL(k_collisionPhase, grid_of(a.geo), kBlock, 0, s, g, ux, uy, uz, phi, normx, normy, normz, a);
+    MCB_LAUNCH_CELLS(k_collisionPhase, g, ux, uy, uz, phi, normx, normy, normz, a);
     return launched();
 }
 
@@ -379,20 +478,20 @@ mcb_status mcb_streamingCalc(const float* g, float* g_out, int NX, int NY, int N
                              void* stream) {
     MCB_OP_PROLOGUE(g, g_out);
     if (g == g_out) return MCB_ERR_INVALID_ARG;
-    hipLaunchKernelGGL(k_streamingCalc, grid_of(a.geo), kBlock, 0, s, g, g_out, a);
+    MCB_LAUNCH_CELLS(k_streamingCalc, g, g_out, a);
     return launched();
 }
 
 mcb_status mcb_fgBoundary(float* f, const float* rho, float* g, const float* phi, int NX, int NY, int NZ,
                           const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(f, rho, g, phi);
-    hipLaunchKernelGGL(k_fgBoundary, grid_of(a.geo), kBlock, 0, s, f, rho, g, phi, a);
+    hipLaunchKernelGGL(k_fgBoundary, face_grid(a.geo), dim3(256), 0, s, f, rho, g, phi, a);
     return launched();
 }
 
 mcb_status mcb_boundaryConditions(float* phi, int NX, int NY, int NZ, const mcb_op_consts* c, void* stream) {
     MCB_OP_PROLOGUE(phi);
-    hipLaunchKernelGGL(k_boundaryConditions, grid_of(a.geo), kBlock, 0, s, phi, a);
+    hipLaunchKernelGGL(k_boundaryConditions, face_grid(a.geo), dim3(256), 0, s, phi, a);
     return launched();
 }
 

@@ -172,3 +172,13 @@ def test_op_matches_oracle_across_magnitudes(gpu_lib, name):
         assert np.array_equal(got, want, equal_nan=True), (k, int(np.count_nonzero(~((got == want) | (np.isnan(got) & np.isnan(want))))))
     for d in dev.values():
         d.free()
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (3, 7, 4), (65, 3, 9), (5, 40, 3), (33, 18, 35)])
+@pytest.mark.parametrize("name", ["fgBoundary", "boundaryConditions", "streamingCalc", "collisionFluid", "gradCalc"])
+def test_face_and_neighbour_ops_on_odd_shapes(gpu_lib, name, shape):
+    mcb = gpu_lib
+    nx, ny, nz = shape
+    p = mcb.make_params(nx, ny, nz, bc_mode=mcb.BC_REFERENCE, weights=mcb.WEIGHTS_LITERAL, tau_f=0.505)
+    bad = run_op(mcb, name, p, random_state((nz, ny, nx), seed=nx + 7 * ny))
+    assert not bad, f"{name} {shape}: " + "; ".join(bad)
