@@ -123,14 +123,10 @@ void reference_faces_from_interior(const mcb_params& p, float* phi) {
         }
 }
 
-// Plane stride: cells rounded up to 256 elements, so every population
-// plane starts 1 KiB-aligned.
-long long plane_stride(long long n) { return plane_stride_cells(n); }
-
 // The fused kernels address all 19 planes of a buffer through one 32-bit
 // buffer resource (FP32 lattices up to ~56.5M cells, 16-bit up to ~113M).
 bool fused_fits(const mcb_params& p) {
-    const long long P = plane_stride((long long)p.nx * p.ny * p.nz);
+    const long long P = plane_stride_cells((long long)p.nx * p.ny * p.nz);
     return P * 19 * (p.storage == MCB_STORE_FP32 ? 4 : 2) <= 0xFFFFFFFFLL;
 }
 
@@ -153,15 +149,13 @@ int resolve_path(const mcb_params& p) {
 // pass: as asked, or (AUTO) where its tiling gives the pass long z-chunks.
 bool ctx_recomputes_n(const mcb_params& p) {
     if (p.normals != MCB_NORMALS_AUTO) return p.normals == MCB_NORMALS_RECOMPUTED;
-    const Geo g{p.nx, p.ny, p.nz, p.nx * p.ny, (long long)p.nx * p.ny * p.nz, 0};
-    return phase_recomputes_n(g, choose_tiling_single(p));
+    return phase_recomputes_n(fused_geo(p), choose_tiling_single(p));
 }
 
 size_t footprint(const mcb_params& p, int path) {
     // 16-bit: the case plus the batch's ten macro fields.
-    if (p.storage != MCB_STORE_FP32) return case_bytes(p) + 10 * (size_t)plane_stride((long long)p.nx * p.ny * p.nz) * 4;
-    const long long n = (long long)p.nx * p.ny * p.nz;
-    const long long P = plane_stride(n);
+    const long long P = path == MCB_PATH_FUSED ? fused_geo(p).plane : plane_stride_cells((long long)p.nx * p.ny * p.nz);
+    if (p.storage != MCB_STORE_FP32) return case_bytes(p) + 10 * (size_t)P * 4;
     size_t floats = 0;
     if (path == MCB_PATH_FUSED && p.f_form == MCB_F_MOMENTS)   // 13 moments A/B (u among them), phi twice, n
         floats = 2 * 13 * (size_t)P + (ctx_recomputes_n(p) ? 12 : 15) * (size_t)P;
@@ -460,9 +454,7 @@ mcb_status mcb_create(const mcb_params* p, void* stream, mcb_ctx** out) {
     c->device = p->device;
     c->phys = host_phys(*p);
     mcb_op_consts_from_params(p, &c->oc);
-    c->geo.nx = p->nx; c->geo.ny = p->ny; c->geo.nz = p->nz;
-    c->geo.nxy = p->nx * p->ny;
-    c->geo.n = (long long)p->nx * p->ny * p->nz;
+    c->geo = fused_geo(*p);
 
     auto bail = [&](mcb_status s) { mcb_destroy(c); return s; };
     if (hipSetDevice(c->device) != hipSuccess) return bail(MCB_ERR_NO_DEVICE);
@@ -475,21 +467,16 @@ mcb_status mcb_create(const mcb_params* p, void* stream, mcb_ctx** out) {
     for (auto& e : c->ev)
         if (hipEventCreate(&e) != hipSuccess) return bail(MCB_ERR_HIP);
 
-    const long long n = c->geo.n;
-    const long long P = plane_stride(n);
+    const long long n = c->geo.n, P = c->geo.plane;
     if (p->storage != MCB_STORE_FP32) {
-        c->geo.plane = P;
         c->batch.reset(new (std::nothrow) Batch(c->device, c->stream));
         if (!c->batch) return bail(MCB_ERR_OUT_OF_MEMORY);
         c->tiling = choose_tiling_single(*p);
     } else if (path == MCB_PATH_FUSED) {
-        c->geo.plane = P;
         // At tau_g = 1 g is kept in moment form: phi (two buffers), u and n
         // (or n recomputed by the phase pass) instead of two sets of 19 planes.
         const bool moments = p->tau_g == 1.0f;
         c->fm = p->f_form == MCB_F_MOMENTS;
-        // Populations in 64-cell blocks where a z plane holds whole blocks.
-        c->geo.blocked = MCB_POP_BLOCKS && !c->fm && c->geo.nxy % 64 == 0;
         for (int b = 0; b < 2; ++b) {
             if ((st = alloc(c, &c->f[b], (c->fm ? kFm : 19) * (size_t)P)) != MCB_OK) return bail(st);
             if (!moments && (st = alloc(c, &c->g[b], 19 * (size_t)P)) != MCB_OK) return bail(st);

@@ -14,9 +14,7 @@ namespace mcb {
 
 namespace {
 
-long long plane_of(const mcb_params& p) {
-    return plane_stride_cells((long long)p.nx * p.ny * p.nz);
-}
+long long plane_of(const mcb_params& p) { return fused_geo(p).plane; }
 
 unsigned pop_bytes(int storage) { return storage == MCB_STORE_FP32 ? 4u : 2u; }
 
@@ -313,15 +311,9 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
     c->storage = p.storage;
     c->mode = p.tau_g == 1.0f ? COLLIDE_STEP : COLLIDE_STEP_BGK;
     c->tiling = t;
-    c->geo.nx = p.nx;
-    c->geo.ny = p.ny;
-    c->geo.nz = p.nz;
-    c->geo.nxy = p.nx * p.ny;
-    c->geo.n = (long long)p.nx * p.ny * p.nz;
-    c->geo.plane = P;
-    // FP32 populations in 64-cell blocks where a z plane holds whole blocks
-    // (16-bit ones stay in planes: with blocks the FP16 batch ran 3% slower).
-    c->geo.blocked = MCB_POP_BLOCKS && p.storage == MCB_STORE_FP32 && c->geo.nxy % 64 == 0;
+    // FP32 populations in 64-cell blocks (16-bit ones stay in planes: with
+    // blocks the FP16 batch ran 3% slower).
+    c->geo = fused_geo(p);
     c->phys = host_phys(p);
     auto alloc = [&](size_t bytes, void** out) -> mcb_status {
         mcb_status s = dev_alloc(bytes, out);

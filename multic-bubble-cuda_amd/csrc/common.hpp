@@ -13,30 +13,33 @@ namespace mcb {
 // and the layout of its FP32 population buffers (16-bit ones are always in
 // planes).
 //
-// Population layouts (cell index i = z*nxy + y*nx + x, link l):
-//   planes (blocked = 0): element l*plane + i, one plane of cells per link;
+// Population layouts (cell r of z plane z, link l, i = z*zpop + r):
+//   planes (blocked = 0): element l*plane + i, one plane of cells per link,
+//     zpop = nxy;
 //   blocks (blocked = 1): element (i >> 6)*19*64 + l*64 + (i & 63), groups of
-//     64 consecutive cells holding their 19 links side by side.
-// Blocks need nxy to be a multiple of 64, so a z plane is a whole number of
-// groups and an offset splits into a wave-uniform z part (z*nxy*19 elements)
-// and a per-lane in-plane part. A cell's 19 links then lie within 19*64
-// elements instead of 19 planes apart, and a wave's gathers and stores open
-// fewer DRAM pages (256^3: 0.577 -> 0.544 ms per FP32 collide).
+//     64 consecutive cells holding their 19 links side by side, zpop = nxy
+//     rounded up to 64.
+// A z plane is a whole number of groups, so an offset splits into a
+// wave-uniform z part (z*zpop*19 elements) and a per-lane in-plane part. A
+// cell's 19 links then lie within 19*64 elements instead of 19 planes apart,
+// and a wave's gathers and stores open fewer DRAM pages (256^3: 0.577 -> 0.544
+// ms per FP32 collide, 150x105x77, whose planes end in a partial group:
+// RAGGED).
 struct Geo {
     int nx, ny, nz;
     int nxy;          // nx*ny
     long long n;      // nx*ny*nz
-    long long plane;  // elements between population planes (>= n)
+    long long plane;  // elements between population planes (>= nz*zpop)
     int blocked = 0;  // FP32 populations in 64-cell blocks (see above)
+    int zpop = 0;     // population cells per z plane
 };
 
-#ifndef MCB_POP_BLOCKS
-#define MCB_POP_BLOCKS 1   // 0: FP32 populations always in planes
-#endif
-
-// Element offset of link l of cell i in a population buffer of layout blk.
-__host__ __device__ __forceinline__ long long pop_index(const Geo& G, int blk, int l, long long i) {
-    return blk ? (i >> 6) * (19 * 64) + l * 64 + (i & 63) : l * G.plane + i;
+// Element offset of link l of cell r of z plane z in a population buffer of
+// layout blk.
+__host__ __device__ __forceinline__ long long pop_index(const Geo& G, int blk, int l, int z, int r) {
+    if (!blk) return l * G.plane + (long long)z * G.nxy + r;
+    const long long i = (long long)z * G.zpop + r;
+    return (i >> 6) * (19 * 64) + l * 64 + (i & 63);
 }
 
 __device__ __forceinline__ int wrap_lo(int a, int n) { return a < 0 ? a + n : a; }
@@ -103,7 +106,7 @@ struct Planes {
     __amdgpu_buffer_rsrc_t r;
     unsigned lb;   // bytes between the links of a cell
     unsigned bb;   // bytes per group of 64 cells
-    unsigned zm;   // bytes per unit of a z plane's cell offset z*nxy
+    unsigned zm;   // bytes per unit of a z plane's population offset z*zpop
     __device__ __forceinline__ Planes(const float* base, const Geo& G)
         : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)(19u * (unsigned)G.plane * 4u),
                                               kBufferConfigWord)),
@@ -112,7 +115,7 @@ struct Planes {
           zm(G.blocked ? 76u : 4u) {}
     // Byte offset of cell index e (whole, or within its z plane) for link 0.
     __device__ __forceinline__ unsigned col(unsigned e) const { return (e >> 6) * bb + (e & 63u) * 4u; }
-    // Byte offset of the z plane whose first cell index is zc (= z*nxy).
+    // Byte offset of the z plane whose first population is zc (= z*zpop).
     __device__ __forceinline__ unsigned zb(unsigned zc) const { return zc * zm; }
     template <int L> __device__ __forceinline__ float ld(unsigned elem) const {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, col(elem), L * lb, 0));
@@ -161,6 +164,24 @@ inline long long plane_stride_cells(long long n) { return (n + 255) / 256 * 256 
 
 // Largest plane stride (cells) the fused kernels address through Planes.
 constexpr long long kMaxFusedPlane = 0xFFFFFFFFLL / (19 * 4);
+
+// Geometry of a lattice on the fused kernels; blocks: FP32 populations in
+// blocks where the padded z planes fit the kernels' 32-bit buffers.
+inline Geo fused_geo(int nx, int ny, int nz, bool blocks) {
+    Geo g{nx, ny, nz, nx * ny, (long long)nx * ny * nz, 0, 0, nx * ny};
+    g.plane = plane_stride_cells(g.n);
+    const int zp = (g.nxy + 63) / 64 * 64;
+    const long long padded = plane_stride_cells((long long)zp * nz);
+    if (blocks && padded <= kMaxFusedPlane) {
+        g.blocked = 1;
+        g.zpop = zp;
+        g.plane = padded;
+    }
+    return g;
+}
+inline Geo fused_geo(const mcb_params& p) {
+    return fused_geo(p.nx, p.ny, p.nz, p.storage == MCB_STORE_FP32 && p.f_form == MCB_F_POPULATIONS);
+}
 
 inline mcb_status hip_status(hipError_t e) {
     if (e == hipSuccess) return MCB_OK;

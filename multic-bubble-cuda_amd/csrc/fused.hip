@@ -47,7 +47,7 @@ __global__ __launch_bounds__(PBX * PBY) void k_phase(CaseView c, unsigned gx, un
                             (unsigned)(shift<1>(z, G.nz) * G.nxy)};
     const PopPlanes<StoreF32> gp(c.gsrc, G);
     const unsigned me = zs[1] + ys[1] + xs[1];
-    float v = phase_sum<StoreF32>(c, gp, Columns(xs, ys, gp), xs, ys, zs);
+    float v = phase_sum<StoreF32>(c, gp, Columns(xs, ys, gp), xs, ys, zs, PopZ(z, G).v);
     // Ghost-layer faces (moment form): before the first step a face keeps its
     // initial phi, later it takes boundaryConditions' copy.
     if (c.bc == MCB_BC_REFERENCE && ref_face(G, x, y, z))
@@ -146,12 +146,12 @@ __global__ __launch_bounds__(PBX * PBY) void k_init_pull(const float* __restrict
     const int xs[3] = {shift<-1>(x, G.nx), x, shift<1>(x, G.nx)};
     const int ys[3] = {shift<-1>(y, G.ny) * G.nx, y * G.nx, shift<1>(y, G.ny) * G.nx};
     const int zs[3] = {shift<-1>(z, G.nz) * G.nxy, z * G.nxy, shift<1>(z, G.nz) * G.nxy};
-    const int me = zs[1] + ys[1] + xs[1];
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
         const float w = p.w[WC[l]];
-        f[pop_index(G, G.blocked, l, me)] = w * 1.0f;
-        if (g) g[pop_index(G, G.blocked, l, me)] = w * phi[zs[1 + CZ[l]] + ys[1 + CY[l]] + xs[1 + CX[l]]];
+        const long long at = pop_index(G, G.blocked, l, z, y * G.nx + x);
+        f[at] = w * 1.0f;
+        if (g) g[at] = w * phi[zs[1 + CZ[l]] + ys[1 + CY[l]] + xs[1 + CX[l]]];
     });
 }
 
@@ -217,11 +217,11 @@ __global__ __launch_bounds__(PBX * PBY) void k_link_shift(const float* __restric
     if (x >= G.nx || y >= G.ny) return;
     const int xs[3] = {shift<-1>(x, G.nx), x, shift<1>(x, G.nx)};
     const int ys[3] = {shift<-1>(y, G.ny) * G.nx, y * G.nx, shift<1>(y, G.ny) * G.nx};
-    const int zs[3] = {shift<-1>(z, G.nz) * G.nxy, z * G.nxy, shift<1>(z, G.nz) * G.nxy};
+    const int zs[3] = {shift<-1>(z, G.nz), z, shift<1>(z, G.nz)};
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        dst[pop_index(G, dblk, l, zs[1] + ys[1] + xs[1])] =
-            src[pop_index(G, sblk, l, zs[1 - SIGN * CZ[l]] + ys[1 - SIGN * CY[l]] + xs[1 - SIGN * CX[l]])];
+        dst[pop_index(G, dblk, l, z, ys[1] + xs[1])] =
+            src[pop_index(G, sblk, l, zs[1 - SIGN * CZ[l]], ys[1 - SIGN * CY[l]] + xs[1 - SIGN * CX[l]])];
     });
 }
 
@@ -230,11 +230,13 @@ __global__ __launch_bounds__(PBX * PBY) void k_link_shift(const float* __restric
 template <class T>
 __global__ __launch_bounds__(256) void k_pop_relayout(const T* __restrict__ src, int sblk, T* __restrict__ dst,
                                                       int dblk, Geo G) {
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < G.n; i += (long long)gridDim.x * 256)
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < G.n; i += (long long)gridDim.x * 256) {
+        const int z = (int)(i / G.nxy), r = (int)(i - (long long)z * G.nxy);
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            dst[pop_index(G, dblk, l, i)] = src[pop_index(G, sblk, l, i)];
+            dst[pop_index(G, dblk, l, z, r)] = src[pop_index(G, sblk, l, z, r)];
         });
+    }
 }
 
 // --------------------------------------------------------------- reductions

@@ -253,16 +253,23 @@ template <int L> __device__ __forceinline__ float g_from_moments(const CaseView&
     return phase_post<L>(pc, c.phys);
 }
 
+// Population offsets (cells) of the z planes z-1, z, z+1, wave-uniform.
+struct PopZ {
+    unsigned v[3];
+    __device__ __forceinline__ PopZ(int z, const Geo& G)
+        : v{(unsigned)(shift<-1>(z, G.nz) * G.zpop), (unsigned)(z * G.zpop), (unsigned)(shift<1>(z, G.nz) * G.zpop)} {}
+};
+
 // phiCalc (src/lbm.cu:18-25) for one cell of a pull-form state: the
 // post-stream g_l(x) is g*_l(x - c_l). xs/ys/zs: offsets of x-1, x, x+1 etc.
 // From stored populations, or before the first step from initDist's
 // g_l = w_l phi0 (GM_INITIAL); the moment form runs phase_tile_gm (FP32) or
 // phase_tile_ab (16-bit forms) instead.
-// col: the columns of xs/ys in gp's layout.
+// col: the columns of xs/ys in gp's layout; zp: PopZ of the cell.
 template <class S>
 __device__ __forceinline__ float phase_sum(const CaseView& c, const PopPlanes<S>& gp, const Columns& col,
                                            const unsigned (&xs)[3], const unsigned (&ys)[3],
-                                           const unsigned (&zs)[3]) {
+                                           const unsigned (&zs)[3], const unsigned (&zp)[3]) {
     float sum = 0.0f;
     if (c.gm == GM_INITIAL) {
         const float p0 = ld32(c.phi_prev, zs[1] + ys[1] + xs[1]);
@@ -271,7 +278,7 @@ __device__ __forceinline__ float phase_sum(const CaseView& c, const PopPlanes<S>
     }
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        const float v = gp.template ldb<l>(col.template src<l>(), gp.zb(zs[1 - CZ[l]]));
+        const float v = gp.template ldb<l>(col.template src<l>(), gp.zb(zp[1 - CZ[l]]));
         if constexpr (S::kAnchored)
             sum += pop_from_offset<l>(c.phys, ld32(c.phi_prev, zs[1 - CZ[l]] + ys[1 - CY[l]] + xs[1 - CX[l]]), v);
         else sum += v;
@@ -1290,11 +1297,10 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
     // in registers; 16-bit forms decode at use).
     using Raw = typename PopPlanes<S>::Raw;
     auto fetch_f = [&](Raw (&r)[Q], int z) {
-        const unsigned zs[3] = {(unsigned)(shift<-1>(z, G.nz) * G.nxy), (unsigned)(z * G.nxy),
-                                (unsigned)(shift<1>(z, G.nz) * G.nxy)};
+        const PopZ zp(z, G);
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            r[l] = fsrc.template raw<l>(col.template src<l>(), fsrc.zb(zs[1 - CZ[l]]));
+            r[l] = fsrc.template raw<l>(col.template src<l>(), fsrc.zb(zp.v[1 - CZ[l]]));
         });
     };
     // Plane z of the tile, given its gathered populations fr.
@@ -1343,6 +1349,7 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
             const float phic = s_phi[z & 3][0][(ty + 2) * PX + (tx + 2)];
             cell16<MODE>(c, k16, fsrc, gsrc, fdst, gdst, col, me4, zs, fr, nbn, ncx, ncy, ncz, ind, phic);
         } else {
+            const PopZ zp(z, G);
             float curv, Fx, Fy, Fz;
             curvature_force(nbn, c.phys, d, ncx, ncy, ncz, ind, curv, Fx, Fy, Fz);
             const Moments m = moments(fr, c.phys, Fx, Fy, Fz);
@@ -1369,12 +1376,12 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                     phic = phi_f.ld(me4, z1 * 4u);
                     for_links([&](auto lc) {
                         constexpr int l = decltype(lc)::value;
-                        gpre[l] = gsrc.template ldb<l>(col.template src<l>(), gsrc.zb(zs[1 - CZ[l]]));
+                        gpre[l] = gsrc.template ldb<l>(col.template src<l>(), gsrc.zb(zp.v[1 - CZ[l]]));
                     });
                 }
                 for_links([&](auto lc) {
                     constexpr int l = decltype(lc)::value;
-                    fdst.template stb<l>(col.me(), fdst.zb(z1), fluid_post<l>(fc, c.phys, d));
+                    fdst.template stb<l>(col.me(), fdst.zb(zp.v[1]), fluid_post<l>(fc, c.phys, d));
                 });
                 if (MODE == COLLIDE_STEP && c.gm != GM_POPULATIONS) {
                     // Moment form: keep what collisionPhase needs beside the phi
@@ -1395,9 +1402,9 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                 for_links([&](auto lc) {
                     constexpr int l = decltype(lc)::value;
                     if constexpr (MODE == COLLIDE_STEP) {
-                        gdst.template stb<l>(col.me(), gdst.zb(z1), phase_post<l>(pc, c.phys));
+                        gdst.template stb<l>(col.me(), gdst.zb(zp.v[1]), phase_post<l>(pc, c.phys));
                     } else {
-                        gdst.template stb<l>(col.me(), gdst.zb(z1), phase_post_bgk<l>(pc, c.phys, d, gpre[l]));
+                        gdst.template stb<l>(col.me(), gdst.zb(zp.v[1]), phase_post_bgk<l>(pc, c.phys, d, gpre[l]));
                     }
                 });
             }
@@ -1815,7 +1822,7 @@ __global__ __launch_bounds__(TX * TY) void k_phase_batch(const CaseView* __restr
         for (int z = w.z0; z < ze; ++z) {
             const unsigned zs[3] = {(unsigned)(shift<-1>(z, G.nz) * G.nxy), (unsigned)(z * G.nxy),
                                     (unsigned)(shift<1>(z, G.nz) * G.nxy)};
-            float v = phase_sum<S>(c, gp, col, xs, ys, zs);
+            float v = phase_sum<S>(c, gp, col, xs, ys, zs, PopZ(z, G).v);
             if (mass) {
                 v += delta;
                 part += (double)v;
