@@ -149,12 +149,12 @@ int resolve_path(const mcb_params& p) {
 // pass: as asked, or (AUTO) where its tiling gives the pass long z-chunks.
 bool ctx_recomputes_n(const mcb_params& p) {
     if (p.normals != MCB_NORMALS_AUTO) return p.normals == MCB_NORMALS_RECOMPUTED;
-    return phase_recomputes_n(fused_geo(p), choose_tiling_single(p));
+    return phase_recomputes_n(fused_geo(p, true), choose_tiling_single(p));
 }
 
 size_t footprint(const mcb_params& p, int path) {
     // 16-bit: the case plus the batch's ten macro fields.
-    const long long P = path == MCB_PATH_FUSED ? fused_geo(p).plane : plane_stride_cells((long long)p.nx * p.ny * p.nz);
+    const long long P = path == MCB_PATH_FUSED ? fused_geo(p, true).plane : plane_stride_cells((long long)p.nx * p.ny * p.nz);
     if (p.storage != MCB_STORE_FP32) return case_bytes(p) + 10 * (size_t)P * 4;
     size_t floats = 0;
     if (path == MCB_PATH_FUSED && p.f_form == MCB_F_MOMENTS)   // 13 moments A/B (u among them), phi twice, n
@@ -454,7 +454,7 @@ mcb_status mcb_create(const mcb_params* p, void* stream, mcb_ctx** out) {
     c->device = p->device;
     c->phys = host_phys(*p);
     mcb_op_consts_from_params(p, &c->oc);
-    c->geo = fused_geo(*p);
+    c->geo = fused_geo(*p, true);
 
     auto bail = [&](mcb_status s) { mcb_destroy(c); return s; };
     if (hipSetDevice(c->device) != hipSuccess) return bail(MCB_ERR_NO_DEVICE);

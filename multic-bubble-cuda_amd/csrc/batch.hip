@@ -14,7 +14,7 @@ namespace mcb {
 
 namespace {
 
-long long plane_of(const mcb_params& p) { return fused_geo(p).plane; }
+long long plane_of(const mcb_params& p) { return fused_geo(p, false).plane; }
 
 unsigned pop_bytes(int storage) { return storage == MCB_STORE_FP32 ? 4u : 2u; }
 
@@ -312,8 +312,9 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
     c->mode = p.tau_g == 1.0f ? COLLIDE_STEP : COLLIDE_STEP_BGK;
     c->tiling = t;
     // FP32 populations in 64-cell blocks (16-bit ones stay in planes: with
-    // blocks the FP16 batch ran 3% slower).
-    c->geo = fused_geo(p);
+    // blocks the FP16 batch ran 3% slower), rows unpadded: a case's bytes
+    // count against the budgets that admit it.
+    c->geo = fused_geo(p, false);
     c->phys = host_phys(p);
     auto alloc = [&](size_t bytes, void** out) -> mcb_status {
         mcb_status s = dev_alloc(bytes, out);

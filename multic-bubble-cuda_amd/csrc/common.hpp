@@ -13,32 +13,37 @@ namespace mcb {
 // and the layout of its FP32 population buffers (16-bit ones are always in
 // planes).
 //
-// Population layouts (cell r of z plane z, link l, i = z*zpop + r):
+// Population layouts (cell (x, y, z), link l, i = z*zpop + y*pitch + x):
 //   planes (blocked = 0): element l*plane + i, one plane of cells per link,
-//     zpop = nxy;
+//     pitch = nx, zpop = nxy;
 //   blocks (blocked = 1): element (i >> 6)*19*64 + l*64 + (i & 63), groups of
-//     64 consecutive cells holding their 19 links side by side, zpop = nxy
-//     rounded up to 64.
+//     64 consecutive cells holding their 19 links side by side, zpop =
+//     pitch*ny rounded up to 64. pitch is nx rounded up to 32 cells (128
+//     bytes, a cache line) where a context can afford it: otherwise the rows
+//     of a wave start inside lines, and each store leaves two partial lines
+//     to be merged in memory (250^3: 767 us per collide against 553 padded,
+//     150x105x77 66 against 59).
 // A z plane is a whole number of groups, so an offset splits into a
 // wave-uniform z part (z*zpop*19 elements) and a per-lane in-plane part. A
 // cell's 19 links then lie within 19*64 elements instead of 19 planes apart,
 // and a wave's gathers and stores open fewer DRAM pages (256^3: 0.577 -> 0.544
-// ms per FP32 collide, 150x105x77, whose planes end in a partial group:
-// RAGGED).
+// ms per FP32 collide; 200x130x90, whose planes end in a partial group and
+// rows inside lines: 140 -> 123 us, with padded rows 113).
 struct Geo {
     int nx, ny, nz;
     int nxy;          // nx*ny
     long long n;      // nx*ny*nz
     long long plane;  // elements between population planes (>= nz*zpop)
     int blocked = 0;  // FP32 populations in 64-cell blocks (see above)
+    int pitch = 0;    // population cells per row
     int zpop = 0;     // population cells per z plane
 };
 
-// Element offset of link l of cell r of z plane z in a population buffer of
-// layout blk.
-__host__ __device__ __forceinline__ long long pop_index(const Geo& G, int blk, int l, int z, int r) {
-    if (!blk) return l * G.plane + (long long)z * G.nxy + r;
-    const long long i = (long long)z * G.zpop + r;
+// Element offset of link l of cell (x, y, z) in a population buffer of layout
+// blk.
+__host__ __device__ __forceinline__ long long pop_index(const Geo& G, int blk, int l, int x, int y, int z) {
+    if (!blk) return l * G.plane + (long long)z * G.nxy + y * G.nx + x;
+    const long long i = (long long)z * G.zpop + y * G.pitch + x;
     return (i >> 6) * (19 * 64) + l * 64 + (i & 63);
 }
 
@@ -165,22 +170,24 @@ inline long long plane_stride_cells(long long n) { return (n + 255) / 256 * 256 
 // Largest plane stride (cells) the fused kernels address through Planes.
 constexpr long long kMaxFusedPlane = 0xFFFFFFFFLL / (19 * 4);
 
-// Geometry of a lattice on the fused kernels; blocks: FP32 populations in
-// blocks where the padded z planes fit the kernels' 32-bit buffers.
-inline Geo fused_geo(int nx, int ny, int nz, bool blocks) {
-    Geo g{nx, ny, nz, nx * ny, (long long)nx * ny * nz, 0, 0, nx * ny};
+// Geometry of a lattice on the fused kernels: FP32 populations (not f as
+// moments) in blocks, with padded rows if asked for, as far as they fit the
+// kernels' 32-bit buffers.
+inline Geo fused_geo(const mcb_params& p, bool pad_rows) {
+    Geo g{p.nx, p.ny, p.nz, p.nx * p.ny, (long long)p.nx * p.ny * p.nz, 0, 0, p.nx, p.nx * p.ny};
     g.plane = plane_stride_cells(g.n);
-    const int zp = (g.nxy + 63) / 64 * 64;
-    const long long padded = plane_stride_cells((long long)zp * nz);
-    if (blocks && padded <= kMaxFusedPlane) {
+    if (p.storage != MCB_STORE_FP32 || p.f_form != MCB_F_POPULATIONS) return g;
+    for (const int pitch : {(p.nx + 31) / 32 * 32, p.nx}) {
+        if (pitch != p.nx && !pad_rows) continue;
+        const long long zp = ((long long)pitch * p.ny + 63) / 64 * 64, plane = plane_stride_cells(zp * p.nz);
+        if (plane > kMaxFusedPlane) continue;
         g.blocked = 1;
-        g.zpop = zp;
-        g.plane = padded;
+        g.pitch = pitch;
+        g.zpop = (int)zp;
+        g.plane = plane;
+        break;
     }
     return g;
-}
-inline Geo fused_geo(const mcb_params& p) {
-    return fused_geo(p.nx, p.ny, p.nz, p.storage == MCB_STORE_FP32 && p.f_form == MCB_F_POPULATIONS);
 }
 
 inline mcb_status hip_status(hipError_t e) {

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(PBX * PBY) void k_phase(CaseView c, unsigned gx, un
                             (unsigned)(shift<1>(z, G.nz) * G.nxy)};
     const PopPlanes<StoreF32> gp(c.gsrc, G);
     const unsigned me = zs[1] + ys[1] + xs[1];
-    float v = phase_sum<StoreF32>(c, gp, Columns(xs, ys, gp), xs, ys, zs, PopZ(z, G).v);
+    float v = phase_sum<StoreF32>(c, gp, Columns(xs, PopRows(y, G, true).v, gp), xs, ys, zs, PopZ(z, G).v);
     // Ghost-layer faces (moment form): before the first step a face keeps its
     // initial phi, later it takes boundaryConditions' copy.
     if (c.bc == MCB_BC_REFERENCE && ref_face(G, x, y, z))
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(PBX * PBY) void k_init_pull(const float* __restrict
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
         const float w = p.w[WC[l]];
-        const long long at = pop_index(G, G.blocked, l, z, y * G.nx + x);
+        const long long at = pop_index(G, G.blocked, l, x, y, z);
         f[at] = w * 1.0f;
         if (g) g[at] = w * phi[zs[1 + CZ[l]] + ys[1 + CY[l]] + xs[1 + CX[l]]];
     });
@@ -216,12 +216,12 @@ __global__ __launch_bounds__(PBX * PBY) void k_link_shift(const float* __restric
     const int z = blockIdx.z;
     if (x >= G.nx || y >= G.ny) return;
     const int xs[3] = {shift<-1>(x, G.nx), x, shift<1>(x, G.nx)};
-    const int ys[3] = {shift<-1>(y, G.ny) * G.nx, y * G.nx, shift<1>(y, G.ny) * G.nx};
+    const int ys[3] = {shift<-1>(y, G.ny), y, shift<1>(y, G.ny)};
     const int zs[3] = {shift<-1>(z, G.nz), z, shift<1>(z, G.nz)};
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        dst[pop_index(G, dblk, l, z, ys[1] + xs[1])] =
-            src[pop_index(G, sblk, l, zs[1 - SIGN * CZ[l]], ys[1 - SIGN * CY[l]] + xs[1 - SIGN * CX[l]])];
+        dst[pop_index(G, dblk, l, x, y, z)] =
+            src[pop_index(G, sblk, l, xs[1 - SIGN * CX[l]], ys[1 - SIGN * CY[l]], zs[1 - SIGN * CZ[l]])];
     });
 }
 
@@ -231,10 +231,10 @@ template <class T>
 __global__ __launch_bounds__(256) void k_pop_relayout(const T* __restrict__ src, int sblk, T* __restrict__ dst,
                                                       int dblk, Geo G) {
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < G.n; i += (long long)gridDim.x * 256) {
-        const int z = (int)(i / G.nxy), r = (int)(i - (long long)z * G.nxy);
+        const int z = (int)(i / G.nxy), r = (int)(i - (long long)z * G.nxy), y = r / G.nx, x = r - y * G.nx;
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            dst[pop_index(G, dblk, l, z, r)] = src[pop_index(G, sblk, l, z, r)];
+            dst[pop_index(G, dblk, l, x, y, z)] = src[pop_index(G, sblk, l, x, y, z)];
         });
     }
 }

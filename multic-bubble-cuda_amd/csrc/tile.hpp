@@ -187,9 +187,17 @@ struct Field16 {
     }
 };
 
+// Population offsets (cells) of the rows y-1, y, y+1.
+struct PopRows {
+    unsigned v[3];
+    __device__ __forceinline__ PopRows(int y, const Geo& G, bool valid)
+        : v{valid ? (unsigned)(shift<-1>(y, G.ny) * G.pitch) : 0u, (unsigned)(y * G.pitch),
+            valid ? (unsigned)(shift<1>(y, G.ny) * G.pitch) : 0u} {}
+};
+
 // In-plane byte offsets of the 9 columns (x - c_x, y - c_y) that a cell's
 // pull-form gathers read, in the layout of the population buffers (planes'
-// col). They do not depend on z, so a tile computes them once; per plane only
+// col, ys: population row offsets, PopRows). They do not depend on z, so a tile computes them once; per plane only
 // the wave-uniform plane offset (zb) changes, and it goes into the scalar
 // offset of the access.
 struct Columns {
@@ -1278,7 +1286,7 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
                             valid ? (unsigned)shift<1>(x, G.nx) : 0u};
     const unsigned ys[3] = {valid ? (unsigned)(shift<-1>(y, G.ny) * G.nx) : 0u, (unsigned)(y * G.nx),
                             valid ? (unsigned)(shift<1>(y, G.ny) * G.nx) : 0u};
-    const Columns col(xs, ys, fsrc);   // f and g share the layout
+    const Columns col(xs, PopRows(y, G, valid).v, fsrc);   // f and g share the layout
     const unsigned me4 = (ys[1] + xs[1]) * 4u;   // FP32 fields
 
     // Prologue: phi planes zb-2..zb+1, normals of planes zb-1 and zb.
@@ -1813,7 +1821,7 @@ __global__ __launch_bounds__(TX * TY) void k_phase_batch(const CaseView* __restr
     const unsigned ys[3] = {valid ? (unsigned)(shift<-1>(y, G.ny) * G.nx) : 0u, (unsigned)(y * G.nx),
                             valid ? (unsigned)(shift<1>(y, G.ny) * G.nx) : 0u};
     const PopPlanes<S> gp(c.gsrc, G);
-    const Columns col(xs, ys, gp);
+    const Columns col(xs, PopRows(y, G, valid).v, gp);
     const int ze = min(w.z0 + c.zc, G.nz);
     double part = 0.0;
     float delta = 0.0f;
