@@ -40,6 +40,7 @@ struct mcb_ctx {
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     std::vector<hipEvent_t> tev;   // per-kernel timing events
     Tiling tiling{64, 8, 16};
+    bool own_tiling = false;   // set by mcb_set_tiling
     std::string err;
     std::vector<void*> allocs;
 
@@ -580,7 +581,7 @@ mcb_status ctx_init_bubbles_device(mcb_ctx* c, const BubbleSet& s) {
         }
         mcb_status st = batch_status(c, c->batch->add_bubbles(c->p, s.b, s.n, s.width, &c->case_id));
         if (st != MCB_OK) return st;
-        if ((st = batch_status(c, c->batch->set_tiling(c->case_id, c->tiling))) != MCB_OK) return st;
+        if ((st = batch_status(c, c->batch->set_tiling(c->case_id, c->tiling, c->own_tiling))) != MCB_OK) return st;
         c->steps = 0;
         c->initialised = true;
         return MCB_OK;
@@ -631,8 +632,7 @@ mcb_status mcb_init_phi(mcb_ctx* c, const float* phi_host, size_t n) {
         }
         mcb_status st = batch_status(c, c->batch->add(c->p, phi_host, &c->case_id));
         if (st != MCB_OK) return st;
-        Tiling t = c->tiling;
-        if ((st = batch_status(c, c->batch->set_tiling(c->case_id, t))) != MCB_OK) return st;
+        if ((st = batch_status(c, c->batch->set_tiling(c->case_id, c->tiling, c->own_tiling))) != MCB_OK) return st;
         c->steps = 0;
         c->initialised = true;
         return MCB_OK;
@@ -882,6 +882,7 @@ mcb_status mcb_set_tiling(mcb_ctx* c, int tx, int ty, int zc) {
         if (st != MCB_OK) return st;
     }
     c->tiling = t;
+    c->own_tiling = true;
     return MCB_OK;
 }
 

@@ -162,6 +162,9 @@ Tiling choose_tiling_single(const mcb_params& p) {
     // (64x4x16 75), 64^3 64x4x2 22.6 (64x4x16 54).
     Tiling t = choose_tiling(p);
     const bool fp32 = p.storage == MCB_STORE_FP32;
+    // Stored 16-bit g sums its mass in FP64 tile by tile: the tiles of a batch
+    // case, so that a state image continues with the same bits in either.
+    if (!fp32 && p.tau_g != 1.0f) return t;
     auto lanes = [&](const Tiling& q) {
         return (long long)((p.nx + q.tx - 1) / q.tx) * ((p.ny + q.ty - 1) / q.ty) * ((p.nz + q.zc - 1) / q.zc) * q.tx *
                q.ty;
@@ -720,6 +723,7 @@ mcb_status Batch::to_populations(CaseState* c) {
         if (st != MCB_OK) return st;
         c->allocs.emplace_back(q, sizeof(MassCell));
         c->mass = static_cast<MassCell*>(q);
+        if (!c->own_tiling) c->tiling = batch_tiling(c->p);   // see choose_tiling_single
         if ((st = build_own_table(c)) != MCB_OK) return st;   // partial sums
     }
     c->gm = GM_POPULATIONS;
@@ -949,13 +953,15 @@ mcb_status Batch::reduce(int id, double* sum_phi, double* kinetic) {
     return MCB_OK;
 }
 
-mcb_status Batch::set_tiling(int id, const Tiling& t) {
+mcb_status Batch::set_tiling(int id, const Tiling& t, bool by_caller) {
     CaseState* c = get(id);
     if (!c) return fail(MCB_ERR_INVALID_ARG, "no such case");
     if (!supported_for(t, c->storage) || t.zc > c->p.nz) return fail(MCB_ERR_INVALID_ARG, "unsupported tiling");
     B_HIP(hipSetDevice(device_));
     B_HIP(hipStreamSynchronize(stream_));
-    c->tiling = t;
+    // The library's own choice for a moment form does not hold for stored g.
+    c->tiling = !by_caller && c->mass ? batch_tiling(c->p) : t;
+    c->own_tiling = by_caller;
     mcb_status st = build_own_table(c);
     if (st != MCB_OK) return st;
     dirty_ = true;

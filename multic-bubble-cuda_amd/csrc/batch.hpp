@@ -28,6 +28,7 @@ struct CaseState {
     int storage = MCB_STORE_FP32;
     int mode = COLLIDE_STEP;       // COLLIDE_STEP or COLLIDE_STEP_BGK
     Tiling tiling{64, 8, 16};
+    bool own_tiling = false;        // set by the library's caller
     int cur = 0;                    // population buffer of the current state
     int parity_offset = 0;          // cur = batch parity ^ parity_offset
     long long steps = 0;            // steps taken since init
@@ -86,7 +87,7 @@ public:
     mcb_status read(int id, int field, float* host, size_t n);
     mcb_status write(int id, int field, const float* host, size_t n);
     mcb_status reduce(int id, double* sum_phi, double* kinetic);
-    mcb_status set_tiling(int id, const Tiling& t);
+    mcb_status set_tiling(int id, const Tiling& t, bool by_caller = true);
     // State image of a case at a step boundary (state.hpp): size, save, load
     // into a case of the same parameters, or a new case from an image.
     mcb_status state_size(int id, size_t* bytes);

@@ -77,3 +77,27 @@ def test_batch_groups_side_by_side(gpu_lib, storage):
         for cid, p, bub, steps in ids:
             got, want = b.read(cid, "phi"), alone(mcb, p, bub, steps)
             assert np.array_equal(got, want), (p.nx, p.ny, p.nz, int(np.count_nonzero(got != want)))
+
+
+def test_16bit_image_with_written_g_moves_between_context_and_batch(gpu_lib):
+    """A moment-form case whose g was written keeps populations and their FP64 mass sums, tile by tile: the same tiles in a
+    context, whose moment form uses others, and in a batch."""
+    mcb = gpu_lib
+    nx, ny, nz = 60, 24, 40
+    p = mcb.make_params(nx, ny, nz, storage=1, tau_f=0.7, tau_g=1.0)
+    lat = mcb.Lattice(p)
+    lat.init_bubbles([(30.0, 12.0, 20.0, 7.0)], 3.0)
+    lat.step(2)
+    lat.write("g", lat.read("g"))
+    lat.step(1)
+    image = lat.save_state()
+    lat.step(4)
+    with mcb.Batch(1) as b:
+        cid = b.add_state(image)
+        b.step(4)
+        assert np.array_equal(b.read(cid, "phi"), lat.read("phi"))
+    with mcb.Lattice(p) as other:
+        other.load_state(image)
+        other.step(4)
+        assert np.array_equal(other.read("phi"), lat.read("phi"))
+    lat.close()
