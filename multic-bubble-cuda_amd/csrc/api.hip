@@ -156,7 +156,7 @@ bool ctx_recomputes_n(const mcb_params& p) {
 size_t footprint(const mcb_params& p, int path) {
     // 16-bit: the case plus the batch's ten macro fields.
     const long long P = path == MCB_PATH_FUSED ? fused_geo(p, true).plane : plane_stride_cells((long long)p.nx * p.ny * p.nz);
-    if (p.storage != MCB_STORE_FP32) return case_bytes(p) + 10 * (size_t)P * 4;
+    if (p.storage != MCB_STORE_FP32) return case_bytes(p, true) + 10 * (size_t)P * 4;
     size_t floats = 0;
     if (path == MCB_PATH_FUSED && p.f_form == MCB_F_MOMENTS)   // 13 moments A/B (u among them), phi twice, n
         floats = 2 * 13 * (size_t)P + (ctx_recomputes_n(p) ? 12 : 15) * (size_t)P;
@@ -343,9 +343,9 @@ std::vector<StatePart> ctx_state_parts(mcb_ctx* c) {
     }
     if (c->fm)   // the 13 moments (u among them) and the state's phi
         return {{"fm", c->f[c->cur], kFm, N, P, 4, false}, {"phi", c->phis[c->cur ^ 1], 1, N, N, 4, false}};
-    // Images keep populations in planes: with blocked populations they pass
+    // Images keep populations in plain planes: other layouts pass
     // through the idle A/B buffers (pops_image_copy / pops_image_done).
-    const int side = c->geo.blocked ? c->cur ^ 1 : c->cur;
+    const int side = pops_relaid(c->geo) ? c->cur ^ 1 : c->cur;
     std::vector<StatePart> parts{{"f", c->f[side], 19, N, P, 4, false}};
     if (c->gm == GM_POPULATIONS) {
         // With g as populations phi is what the last step reported (phiCalc
@@ -361,7 +361,7 @@ std::vector<StatePart> ctx_state_parts(mcb_ctx* c) {
     return parts;
 }
 
-// Blocked populations around a state image (fused path): the current f (and
+// Populations in another layout around a state image (fused path): the current f (and
 // g populations) into the idle buffers in planes, or back. With ghost-layer
 // faces the idle f's face populations then go back to w_l (a step reads the
 // current buffer and writes every interior cell of the idle one).
@@ -579,7 +579,7 @@ mcb_status ctx_init_bubbles_device(mcb_ctx* c, const BubbleSet& s) {
             if (st != MCB_OK) return st;
             c->case_id = 0;
         }
-        mcb_status st = batch_status(c, c->batch->add_bubbles(c->p, s.b, s.n, s.width, &c->case_id));
+        mcb_status st = batch_status(c, c->batch->add_bubbles(c->p, s.b, s.n, s.width, &c->case_id, true));
         if (st != MCB_OK) return st;
         if ((st = batch_status(c, c->batch->set_tiling(c->case_id, c->tiling, c->own_tiling))) != MCB_OK) return st;
         c->steps = 0;
@@ -630,7 +630,7 @@ mcb_status mcb_init_phi(mcb_ctx* c, const float* phi_host, size_t n) {
             if (st != MCB_OK) return st;
             c->case_id = 0;
         }
-        mcb_status st = batch_status(c, c->batch->add(c->p, phi_host, &c->case_id));
+        mcb_status st = batch_status(c, c->batch->add(c->p, phi_host, &c->case_id, true));
         if (st != MCB_OK) return st;
         if ((st = batch_status(c, c->batch->set_tiling(c->case_id, c->tiling, c->own_tiling))) != MCB_OK) return st;
         c->steps = 0;
@@ -722,7 +722,7 @@ mcb_status mcb_read_field(mcb_ctx* c, int field, float* host, size_t n) {
                 MCB_HIP(c, launch_gm_to_ref(fused_view(c), idle_f, c->stream));
             } else {
                 const float* src = field == MCB_FIELD_F ? c->f[c->cur] : c->g[c->cur];
-                MCB_HIP(c, launch_link_shift(src, c->geo.blocked, field == MCB_FIELD_F ? idle_f : c->g[c->cur ^ 1],
+                MCB_HIP(c, launch_link_shift(src, 1, field == MCB_FIELD_F ? idle_f : c->g[c->cur ^ 1],
                                              0, c->geo, +1, c->stream));
             }
             const float* tmp = field == MCB_FIELD_F || c->gm != GM_POPULATIONS ? idle_f : c->g[c->cur ^ 1];
@@ -780,7 +780,7 @@ mcb_status mcb_write_field(mcb_ctx* c, int field, const float* host, size_t n) {
             for (int l = 0; l < 19; ++l)
                 MCB_HIP(c, hipMemcpyAsync(tmp + (size_t)l * c->geo.plane, host + l * cells, cells * sizeof(float),
                                           hipMemcpyHostToDevice, c->stream));
-            MCB_HIP(c, launch_link_shift(tmp, 0, dst, c->geo.blocked, c->geo, -1, c->stream));
+            MCB_HIP(c, launch_link_shift(tmp, 0, dst, 1, c->geo, -1, c->stream));
             if (c->p.bc_mode == MCB_BC_REFERENCE) {
                 // The written face populations feed the next step once (as
                 // the reference's first momentiCalc reads them); after it they
@@ -1086,7 +1086,7 @@ mcb_status mcb_save_state(mcb_ctx* c, void* buf, size_t bytes) {
     h.path = c->path;
     h.gm = c->path == MCB_PATH_STAGED ? GM_POPULATIONS : c->gm;
     h.steps = c->steps;
-    const bool staged = c->path == MCB_PATH_FUSED && c->geo.blocked;
+    const bool staged = c->path == MCB_PATH_FUSED && pops_relaid(c->geo);
     if (staged) MCB_HIP(c, pops_image_copy(c, true));
     st = state_image_save(c->stream, h, ctx_state_parts(c), buf, bytes, &c->err);
     if (staged) MCB_HIP(c, pops_image_done(c));
@@ -1124,7 +1124,7 @@ mcb_status mcb_load_state(mcb_ctx* c, const void* buf, size_t bytes) {
         c->ref_reset_f = -1;   // the image's face populations are w_l
     }
     if ((st = state_image_load(c->stream, buf, bytes, ctx_state_parts(c), &c->err)) != MCB_OK) return st;
-    if (c->path == MCB_PATH_FUSED && c->geo.blocked) {
+    if (c->path == MCB_PATH_FUSED && pops_relaid(c->geo)) {
         MCB_HIP(c, pops_image_copy(c, false));
         MCB_HIP(c, pops_image_done(c));
         MCB_HIP(c, hipStreamSynchronize(c->stream));

@@ -14,8 +14,6 @@ namespace mcb {
 
 namespace {
 
-long long plane_of(const mcb_params& p) { return fused_geo(p, false).plane; }
-
 unsigned pop_bytes(int storage) { return storage == MCB_STORE_FP32 ? 4u : 2u; }
 
 constexpr int kMacroFields = 10;
@@ -52,8 +50,28 @@ std::vector<WorkItem> xcd_permute(const std::vector<WorkItem>& in) {
 
 }  // namespace
 
-size_t case_bytes(const mcb_params& p) {
-    const size_t P = (size_t)plane_of(p);
+Geo fused_geo(const mcb_params& p, bool pad_rows) {
+    Geo g{p.nx, p.ny, p.nz, p.nx * p.ny, (long long)p.nx * p.ny * p.nz, 0, 0, p.nx, p.nx * p.ny};
+    g.plane = plane_stride_cells(g.n);
+    if (p.f_form != MCB_F_POPULATIONS) return g;
+    const bool fp32 = p.storage == MCB_STORE_FP32;
+    const int group = fp32 ? 64 : 1;
+    if (p.nx < 16 || (!fp32 && tiling_supported16(Tiling{p.nx, 4, 1}))) pad_rows = false;   // at most twice the memory
+    for (const int pitch : {(p.nx + 31) / 32 * 32, p.nx}) {
+        if (pitch != p.nx && !pad_rows) continue;
+        const long long zp = ((long long)pitch * p.ny + group - 1) / group * group, plane = plane_stride_cells(zp * p.nz);
+        if (plane * 19 * pop_bytes(p.storage) > 0xFFFFFFFFLL) continue;
+        g.blocked = fp32;
+        g.pitch = pitch;
+        g.zpop = (int)zp;
+        g.plane = plane;
+        break;
+    }
+    return g;
+}
+
+size_t case_bytes(const mcb_params& p, bool pad_rows) {
+    const size_t P = (size_t)fused_geo(p, pad_rows).plane;
     const bool moments = p.tau_g == 1.0f;
     size_t b = (moments ? 2 : 4) * 19 * P * pop_bytes(p.storage);          // f (and g) A/B
     b += (moments || p.storage != MCB_STORE_FP32 ? 2 : 1) * P * sizeof(float);   // phi
@@ -274,12 +292,13 @@ mcb_status Batch::ensure_partial() {
     return MCB_OK;
 }
 
-mcb_status Batch::add(const mcb_params& p, const float* phi_host, int* id) {
+mcb_status Batch::add(const mcb_params& p, const float* phi_host, int* id, bool pad_rows) {
     if (!phi_host) return fail(MCB_ERR_INVALID_ARG, "null argument");
-    return add_impl(p, phi_host, nullptr, id);
+    return add_impl(p, phi_host, nullptr, id, pad_rows);
 }
 
-mcb_status Batch::add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, int n, float width, int* id) {
+mcb_status Batch::add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, int n, float width, int* id,
+                              bool pad_rows) {
     if (!bubbles || n < 1 || n > kMaxBubbleSet || !(width > 0.0f) || !std::isfinite(width))
         return fail(MCB_ERR_INVALID_ARG, "invalid bubble set");
     BubbleSet s{};
@@ -291,17 +310,19 @@ mcb_status Batch::add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, in
     }
     s.n = n;
     s.width = width;
-    return add_impl(p, nullptr, &s, id);
+    return add_impl(p, nullptr, &s, id, pad_rows);
 }
 
-mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id) {
+mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id,
+                           bool pad_rows) {
     if (!id) return fail(MCB_ERR_INVALID_ARG, "null argument");
     std::string why;
     if (host_validate(&p, &why) != MCB_OK) return fail(MCB_ERR_INVALID_ARG, why);
     if (p.bc_mode != MCB_BC_PERIODIC) return fail(MCB_ERR_UNSUPPORTED, "batched cases are periodic");
     if (p.f_form != MCB_F_POPULATIONS) return fail(MCB_ERR_UNSUPPORTED, "batched cases keep f as populations");
     if (storage_ >= 0 && p.storage != storage_) return fail(MCB_ERR_UNSUPPORTED, "one storage form per batch");
-    const long long P = plane_of(p);
+    const Geo geo = fused_geo(p, pad_rows);
+    const long long P = geo.plane;
     if (19LL * P * pop_bytes(p.storage) > 0xFFFFFFFFLL) return fail(MCB_ERR_UNSUPPORTED, "lattice too large");
     Tiling t = batch_tiling(p);
     if (!supported_for(t, p.storage)) return fail(MCB_ERR_UNSUPPORTED, "no tiling for this lattice");
@@ -315,9 +336,8 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
     c->mode = p.tau_g == 1.0f ? COLLIDE_STEP : COLLIDE_STEP_BGK;
     c->tiling = t;
     // FP32 populations in 64-cell blocks (16-bit ones stay in planes: with
-    // blocks the FP16 batch ran 3% slower), rows unpadded: a case's bytes
-    // count against the budgets that admit it.
-    c->geo = fused_geo(p, false);
+    // blocks the FP16 batch ran 3% slower).
+    c->geo = geo;
     c->phys = host_phys(p);
     auto alloc = [&](size_t bytes, void** out) -> mcb_status {
         mcb_status s = dev_alloc(bytes, out);
@@ -681,7 +701,7 @@ mcb_status Batch::read(int id, int field, float* host, size_t n) {
             e = c->storage == MCB_STORE_FP32 ? launch_gm_to_ref(c->view(c->cur), tmp, stream_)
                                              : launch_ab_to_ref(c->view(c->cur), tmp, stream_);
         else if (c->storage == MCB_STORE_FP32)
-            e = launch_link_shift(static_cast<const float*>(isf ? c->f[c->cur] : c->g[c->cur]), c->geo.blocked, tmp, 0,
+            e = launch_link_shift(static_cast<const float*>(isf ? c->f[c->cur] : c->g[c->cur]), 1, tmp, 0,
                                   c->geo, +1, stream_);
         else
             e = launch_decode16(isf ? c->f[c->cur] : c->g[c->cur], isf ? nullptr : c->phi[c->cur ^ 1], tmp, c->geo,
@@ -744,9 +764,9 @@ mcb_status Batch::to_populations(CaseState* c) {
 std::vector<StatePart> Batch::state_parts(CaseState* c, double* mass) {
     const size_t N = (size_t)c->geo.n, P = (size_t)c->geo.plane;
     const unsigned eb = pop_bytes(c->storage);
-    // Images keep populations in planes: blocked ones pass through the idle
-    // A/B buffers (stage_pops), which the next step overwrites.
-    const int side = c->geo.blocked ? c->cur ^ 1 : c->cur;
+    // Images keep populations in plain planes: other layouts pass through the
+    // idle A/B buffers (stage_pops), which the next step overwrites.
+    const int side = pops_relaid(c->geo) ? c->cur ^ 1 : c->cur;
     std::vector<StatePart> parts;
     parts.push_back({"f", c->f[side], 19, N, P, eb, false});
     if (c->gm == GM_POPULATIONS) parts.push_back({"g", c->g[side], 19, N, P, eb, false});
@@ -793,19 +813,19 @@ mcb_status Batch::save_state(int id, void* buf, size_t bytes) {
     h.path = MCB_PATH_FUSED;
     h.gm = c->gm;
     h.steps = c->steps;
-    if (c->geo.blocked) B_HIP(stage_pops(c, true));
+    if (pops_relaid(c->geo)) B_HIP(stage_pops(c, true));
     return state_image_save(stream_, h, state_parts(c, m5), buf, bytes, &err_);
 }
 
-// Blocked FP32 populations around a state image: the current f (and g
+// Populations in another layout around a state image: the current f (and g
 // populations) into the idle buffers in planes, or back.
 hipError_t Batch::stage_pops(CaseState* c, bool to_image) {
     const int cur = c->cur, idle = c->cur ^ 1;
     void* const* bufs[2] = {c->f, c->gm == GM_POPULATIONS ? c->g : nullptr};
     for (void* const* b : bufs) {
         if (!b) continue;
-        const hipError_t e = to_image ? launch_pop_relayout(b[cur], 1, b[idle], 0, c->geo, 4, stream_)
-                                      : launch_pop_relayout(b[idle], 0, b[cur], 1, c->geo, 4, stream_);
+        const hipError_t e = to_image ? launch_pop_relayout(b[cur], 1, b[idle], 0, c->geo, pop_bytes(c->storage), stream_)
+                                      : launch_pop_relayout(b[idle], 0, b[cur], 1, c->geo, pop_bytes(c->storage), stream_);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -829,7 +849,7 @@ mcb_status Batch::load_state(int id, const void* buf, size_t bytes) {
     c->gm = h.gm;
     double m5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     if ((st = state_image_load(stream_, buf, bytes, state_parts(c, m5), &err_)) != MCB_OK) return st;
-    if (c->geo.blocked) {
+    if (pops_relaid(c->geo)) {
         B_HIP(stage_pops(c, false));
         B_HIP(hipStreamSynchronize(stream_));
     }
@@ -905,7 +925,7 @@ mcb_status Batch::write(int id, int field, const float* host, size_t n) {
             e = hipMemcpyAsync(tmp + l * P, host + l * cells, cells * sizeof(float), hipMemcpyHostToDevice, stream_);
         if (e == hipSuccess) {
             if (c->storage == MCB_STORE_FP32)
-                e = launch_link_shift(tmp, 0, static_cast<float*>(isf ? c->f[c->cur] : c->g[c->cur]), c->geo.blocked,
+                e = launch_link_shift(tmp, 0, static_cast<float*>(isf ? c->f[c->cur] : c->g[c->cur]), 1,
                                       c->geo, -1, stream_);
             else
                 e = launch_encode16(tmp, isf ? nullptr : c->phi[c->cur ^ 1], isf ? c->f[c->cur] : c->g[c->cur], c->geo,

@@ -65,9 +65,16 @@ struct CaseState {
 Phys host_phys(const mcb_params& p);
 mcb_status host_validate(const mcb_params* p, std::string* why);
 
+// Geometry of a lattice on the fused kernels: populations (not f as moments)
+// in blocks (FP32) and, if asked for, in padded rows, as far as they fit the
+// kernels' 32-bit buffers. 16-bit rows that one collide tile spans stay
+// unpadded: the tile is one contiguous piece of memory (FP16, rows padded
+// against not: 176^3 187 against 154 us per step, 144^3 134 against 125).
+Geo fused_geo(const mcb_params& p, bool pad_rows);
+
 // Device bytes of a case with these parameters (populations, phase field(s)
 // and, at tau_g = 1, the moment form of g).
-size_t case_bytes(const mcb_params& p);
+size_t case_bytes(const mcb_params& p, bool pad_rows = false);
 
 class Batch {
 public:
@@ -79,8 +86,12 @@ public:
     // Allocate a case and set its initial state from phi (host, nx*ny*nz
     // floats), or from bubbles on the device (serving; bubble_phi_cell, the
     // bits of the host initialisation).
-    mcb_status add(const mcb_params& p, const float* phi_host, int* id);
-    mcb_status add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, int n, float width, int* id);
+    // pad_rows: populations in line-aligned rows (Geo::pitch), faster where nx
+    // is not a multiple of a line, for case_bytes(p, true) instead of
+    // case_bytes(p) of device memory.
+    mcb_status add(const mcb_params& p, const float* phi_host, int* id, bool pad_rows = false);
+    mcb_status add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, int n, float width, int* id,
+                           bool pad_rows = false);
     mcb_status remove(int id);
     mcb_status step(int nsteps);
     mcb_status macros(int id);
@@ -110,7 +121,7 @@ public:
 
 private:
     mcb_status fail(mcb_status s, const std::string& m);
-    mcb_status add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id);
+    mcb_status add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id, bool pad_rows);
     mcb_status dev_alloc(size_t bytes, void** out);
     void dev_release(void* ptr, size_t bytes);
     mcb_status build_own_table(CaseState* c);

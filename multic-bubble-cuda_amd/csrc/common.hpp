@@ -15,14 +15,16 @@ namespace mcb {
 //
 // Population layouts (cell (x, y, z), link l, i = z*zpop + y*pitch + x):
 //   planes (blocked = 0): element l*plane + i, one plane of cells per link,
-//     pitch = nx, zpop = nxy;
+//     zpop = pitch*ny;
 //   blocks (blocked = 1): element (i >> 6)*19*64 + l*64 + (i & 63), groups of
 //     64 consecutive cells holding their 19 links side by side, zpop =
-//     pitch*ny rounded up to 64. pitch is nx rounded up to 32 cells (128
-//     bytes, a cache line) where a context can afford it: otherwise the rows
-//     of a wave start inside lines, and each store leaves two partial lines
-//     to be merged in memory (250^3: 767 us per collide against 553 padded,
-//     150x105x77 66 against 59).
+//     pitch*ny rounded up to 64.
+// pitch is nx, or nx rounded up to 32 cells (128 or 64 bytes) where the case
+// can afford it (fused_geo): otherwise the rows of a wave start inside cache
+// lines, and each store leaves two partial lines to be merged in memory (FP32
+// 250^3: 767 us per collide against 553 padded, 150x105x77 66 against 59; FP16
+// 250^3: 639 us per step against 424, 150x105x77 72 against 56, 117x90x133 62
+// against 57).
 // A z plane is a whole number of groups, so an offset splits into a
 // wave-uniform z part (z*zpop*19 elements) and a per-lane in-plane part. A
 // cell's 19 links then lie within 19*64 elements instead of 19 planes apart,
@@ -39,13 +41,16 @@ struct Geo {
     int zpop = 0;     // population cells per z plane
 };
 
-// Element offset of link l of cell (x, y, z) in a population buffer of layout
-// blk.
-__host__ __device__ __forceinline__ long long pop_index(const Geo& G, int blk, int l, int x, int y, int z) {
-    if (!blk) return l * G.plane + (long long)z * G.nxy + y * G.nx + x;
+// Element offset of link l of cell (x, y, z) in a population buffer: dev = 1
+// in the layout the kernels step on (above), 0 in plain planes of n cells
+// (readouts, writes and state images).
+__host__ __device__ __forceinline__ long long pop_index(const Geo& G, int dev, int l, int x, int y, int z) {
+    if (!dev) return l * G.plane + (long long)z * G.nxy + y * G.nx + x;
     const long long i = (long long)z * G.zpop + y * G.pitch + x;
-    return (i >> 6) * (19 * 64) + l * 64 + (i & 63);
+    return G.blocked ? (i >> 6) * (19 * 64) + l * 64 + (i & 63) : l * G.plane + i;
 }
+// Whether the two differ.
+inline bool pops_relaid(const Geo& G) { return G.blocked || G.pitch != G.nx; }
 
 __device__ __forceinline__ int wrap_lo(int a, int n) { return a < 0 ? a + n : a; }
 __device__ __forceinline__ int wrap_hi(int a, int n) { return a >= n ? a - n : a; }
@@ -166,29 +171,6 @@ struct Field {
 #define MCB_PLANE_SKEW 256
 #endif
 inline long long plane_stride_cells(long long n) { return (n + 255) / 256 * 256 + MCB_PLANE_SKEW; }
-
-// Largest plane stride (cells) the fused kernels address through Planes.
-constexpr long long kMaxFusedPlane = 0xFFFFFFFFLL / (19 * 4);
-
-// Geometry of a lattice on the fused kernels: FP32 populations (not f as
-// moments) in blocks, with padded rows if asked for, as far as they fit the
-// kernels' 32-bit buffers.
-inline Geo fused_geo(const mcb_params& p, bool pad_rows) {
-    Geo g{p.nx, p.ny, p.nz, p.nx * p.ny, (long long)p.nx * p.ny * p.nz, 0, 0, p.nx, p.nx * p.ny};
-    g.plane = plane_stride_cells(g.n);
-    if (p.storage != MCB_STORE_FP32 || p.f_form != MCB_F_POPULATIONS) return g;
-    for (const int pitch : {(p.nx + 31) / 32 * 32, p.nx}) {
-        if (pitch != p.nx && !pad_rows) continue;
-        const long long zp = ((long long)pitch * p.ny + 63) / 64 * 64, plane = plane_stride_cells(zp * p.nz);
-        if (plane > kMaxFusedPlane) continue;
-        g.blocked = 1;
-        g.pitch = pitch;
-        g.zpop = (int)zp;
-        g.plane = plane;
-        break;
-    }
-    return g;
-}
 
 inline mcb_status hip_status(hipError_t e) {
     if (e == hipSuccess) return MCB_OK;

@@ -149,7 +149,7 @@ __global__ __launch_bounds__(PBX * PBY) void k_init_pull(const float* __restrict
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
         const float w = p.w[WC[l]];
-        const long long at = pop_index(G, G.blocked, l, x, y, z);
+        const long long at = pop_index(G, 1, l, x, y, z);
         f[at] = w * 1.0f;
         if (g) g[at] = w * phi[zs[1 + CZ[l]] + ys[1 + CY[l]] + xs[1 + CX[l]]];
     });
@@ -207,10 +207,10 @@ __global__ __launch_bounds__(PBX * PBY) void k_fm_to_ref(CaseView c, float* __re
     });
 }
 
-// dst_l(x) = src_l(x - SIGN c_l), src in layout sblk and dst in dblk.
+// dst_l(x) = src_l(x - SIGN c_l), src in layout sdev and dst in ddev (pop_index).
 template <int SIGN>
-__global__ __launch_bounds__(PBX * PBY) void k_link_shift(const float* __restrict__ src, int sblk,
-                                                          float* __restrict__ dst, int dblk, Geo G) {
+__global__ __launch_bounds__(PBX * PBY) void k_link_shift(const float* __restrict__ src, int sdev,
+                                                          float* __restrict__ dst, int ddev, Geo G) {
     const int x = blockIdx.x * PBX + threadIdx.x;
     const int y = blockIdx.y * PBY + threadIdx.y;
     const int z = blockIdx.z;
@@ -220,21 +220,21 @@ __global__ __launch_bounds__(PBX * PBY) void k_link_shift(const float* __restric
     const int zs[3] = {shift<-1>(z, G.nz), z, shift<1>(z, G.nz)};
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        dst[pop_index(G, dblk, l, x, y, z)] =
-            src[pop_index(G, sblk, l, xs[1 - SIGN * CX[l]], ys[1 - SIGN * CY[l]], zs[1 - SIGN * CZ[l]])];
+        dst[pop_index(G, ddev, l, x, y, z)] =
+            src[pop_index(G, sdev, l, xs[1 - SIGN * CX[l]], ys[1 - SIGN * CY[l]], zs[1 - SIGN * CZ[l]])];
     });
 }
 
-// dst (layout dblk) = src (layout sblk): the 19 links of every cell, as raw
+// dst (layout ddev) = src (layout sdev): the 19 links of every cell, as raw
 // elements of T (4-byte FP32 or 2-byte 16-bit populations).
 template <class T>
-__global__ __launch_bounds__(256) void k_pop_relayout(const T* __restrict__ src, int sblk, T* __restrict__ dst,
-                                                      int dblk, Geo G) {
+__global__ __launch_bounds__(256) void k_pop_relayout(const T* __restrict__ src, int sdev, T* __restrict__ dst,
+                                                      int ddev, Geo G) {
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < G.n; i += (long long)gridDim.x * 256) {
         const int z = (int)(i / G.nxy), r = (int)(i - (long long)z * G.nxy), y = r / G.nx, x = r - y * G.nx;
         for_links([&](auto lc) {
             constexpr int l = decltype(lc)::value;
-            dst[pop_index(G, dblk, l, x, y, z)] = src[pop_index(G, sblk, l, x, y, z)];
+            dst[pop_index(G, ddev, l, x, y, z)] = src[pop_index(G, sdev, l, x, y, z)];
         });
     }
 }
@@ -557,23 +557,23 @@ hipError_t launch_gm_to_ref(const CaseView& c, float* dst, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_link_shift(const float* src, int sblk, float* dst, int dblk, const Geo& geo, int sign,
+hipError_t launch_link_shift(const float* src, int sdev, float* dst, int ddev, const Geo& geo, int sign,
                              hipStream_t s) {
     const dim3 grid = cell_grid(geo), block(PBX, PBY, 1);
-    if (sign > 0) hipLaunchKernelGGL(k_link_shift<1>, grid, block, 0, s, src, sblk, dst, dblk, geo);
-    else hipLaunchKernelGGL(k_link_shift<-1>, grid, block, 0, s, src, sblk, dst, dblk, geo);
+    if (sign > 0) hipLaunchKernelGGL(k_link_shift<1>, grid, block, 0, s, src, sdev, dst, ddev, geo);
+    else hipLaunchKernelGGL(k_link_shift<-1>, grid, block, 0, s, src, sdev, dst, ddev, geo);
     return hipGetLastError();
 }
 
-hipError_t launch_pop_relayout(const void* src, int sblk, void* dst, int dblk, const Geo& geo, unsigned elem_bytes,
+hipError_t launch_pop_relayout(const void* src, int sdev, void* dst, int ddev, const Geo& geo, unsigned elem_bytes,
                                hipStream_t s) {
     const unsigned blocks = (unsigned)std::min<long long>((geo.n + 255) / 256, 256LL * 16);
     if (elem_bytes == 4)
         hipLaunchKernelGGL(k_pop_relayout<unsigned>, dim3(blocks), dim3(256), 0, s, static_cast<const unsigned*>(src),
-                           sblk, static_cast<unsigned*>(dst), dblk, geo);
+                           sdev, static_cast<unsigned*>(dst), ddev, geo);
     else
         hipLaunchKernelGGL(k_pop_relayout<unsigned short>, dim3(blocks), dim3(256), 0, s,
-                           static_cast<const unsigned short*>(src), sblk, static_cast<unsigned short*>(dst), dblk, geo);
+                           static_cast<const unsigned short*>(src), sdev, static_cast<unsigned short*>(dst), ddev, geo);
     return hipGetLastError();
 }
 

@@ -28,6 +28,25 @@ struct Offs {
     }
 };
 
+// Population offsets (within a link's plane) of a cell and of its neighbour
+// x + SIGN c_l.
+struct PopOffs {
+    unsigned x[3], y[3], z[3];
+    __device__ PopOffs(int i, int j, int k, const Geo& G) {
+        const PopRows r(j, G, true);
+        const PopZ p(k, G);
+        x[0] = (unsigned)shift<-1>(i, G.nx); x[1] = (unsigned)i; x[2] = (unsigned)shift<1>(i, G.nx);
+        for (int a = 0; a < 3; ++a) {
+            y[a] = r.v[a];
+            z[a] = p.v[a];
+        }
+    }
+    template <int L, int SIGN> __device__ unsigned nb() const {
+        return z[1 + SIGN * CZ[L]] + y[1 + SIGN * CY[L]] + x[1 + SIGN * CX[L]];
+    }
+    __device__ unsigned me() const { return nb<0, 1>(); }
+};
+
 // Initial pull-form state: f*_l = w_l (offset 0); g*_l(y) = w_l * phi(y + c_l)
 // with anchor phi(y) when g is stored as populations (g null: moment form).
 template <class S>
@@ -38,11 +57,11 @@ __global__ __launch_bounds__(PBX * PBY) void k_init16(const float* __restrict__ 
     const int z = blockIdx.z;
     if (x >= G.nx || y >= G.ny) return;
     const Offs o(x, y, z, G);
-    const unsigned me = o.me();
+    const unsigned me = PopOffs(x, y, z, G).me();
     const PopPlanes<S> fp(f, G), gp(g, G);
     for_links([&](auto lc) { fp.template st<decltype(lc)::value>(me, 0.0f); });
     if (!g) return;
-    const float ph = phi[me];
+    const float ph = phi[o.me()];
     float rg = 0.0f;
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
@@ -63,11 +82,12 @@ __global__ __launch_bounds__(PBX * PBY) void k_decode16(const void* src, const f
     const int z = blockIdx.z;
     if (x >= G.nx || y >= G.ny) return;
     const Offs o(x, y, z, G);
+    const PopOffs po(x, y, z, G);
     const PopPlanes<S> sp(src, G);
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        const unsigned s = o.template nb<l, -1>();
-        dst[(size_t)l * G.plane + o.me()] = pop_from_offset<l>(p, anchor ? anchor[s] : 1.0f, sp.template ld<l>(s));
+        dst[(size_t)l * G.plane + o.me()] = pop_from_offset<l>(p, anchor ? anchor[o.template nb<l, -1>()] : 1.0f,
+                                                               sp.template ld<l>(po.template nb<l, -1>()));
     });
 }
 
@@ -81,7 +101,7 @@ __global__ __launch_bounds__(PBX * PBY) void k_encode16(const float* __restrict_
     const int z = blockIdx.z;
     if (x >= G.nx || y >= G.ny) return;
     const Offs o(x, y, z, G);
-    const unsigned me = o.me();
+    const unsigned me = o.me(), pme = PopOffs(x, y, z, G).me();
     const PopPlanes<S> dp(dst, G);
     const float a = anchor ? anchor[me] : 1.0f;
     float r = 0.0f;
@@ -89,10 +109,10 @@ __global__ __launch_bounds__(PBX * PBY) void k_encode16(const float* __restrict_
         constexpr int l = decltype(lc)::value;
         if constexpr (l != 0) {
             const float s = offset_of_pop<l>(p, a, src[(size_t)l * G.plane + o.template nb<l, 1>()]);
-            r += (s - dp.template st<l>(me, s)) * off_unscale(WC[l]);
+            r += (s - dp.template st<l>(pme, s)) * off_unscale(WC[l]);
         }
     });
-    dp.template st<0>(me, offset_of_pop<0>(p, a, src[me] + r));
+    dp.template st<0>(pme, offset_of_pop<0>(p, a, src[me] + r));
 }
 
 // (phi, B) moment form -> reference layout: dst_l(x) = w_l (phi + c_l.B)(x - c_l),

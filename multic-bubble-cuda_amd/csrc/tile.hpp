@@ -1090,9 +1090,10 @@ __device__ __forceinline__ void phase_tile_ab(const CaseView& c, int x0, int y0,
 template <int MODE, class S, class NBN>
 __device__ __forceinline__ void cell16(const CaseView& c, const fast::Consts& k, const PopPlanes<S>& fsrc,
                                        const PopPlanes<S>& gsrc, const PopPlanes<S>& fdst,
-                                       const PopPlanes<S>& gdst, const Columns& col, unsigned me4,
-                                       const unsigned (&zs)[3], const unsigned short (&fr)[Q], NBN&& nbn,
-                                       float ncx, float ncy, float ncz, float ind, float phic) {
+                                       const PopPlanes<S>& gdst, const Columns& col, const unsigned (&xs)[3],
+                                       const unsigned (&ys)[3], const unsigned (&zs)[3], const PopZ& zp,
+                                       const unsigned short (&fr)[Q], NBN&& nbn, float ncx, float ncy, float ncz,
+                                       float ind, float phic) {
     float Fx, Fy, Fz;
     fast::curvature_force(nbn, k, ncx, ncy, ncz, ind, Fx, Fy, Fz);
     float tv[Q];   // f_l - w_l
@@ -1100,13 +1101,13 @@ __device__ __forceinline__ void cell16(const CaseView& c, const fast::Consts& k,
         constexpr int l = decltype(lc)::value;
         tv[l] = S::dec(fr[l]) * off_unscale(WC[l]);
     });
-    const unsigned z1 = zs[1];
+    const unsigned z1 = zs[1], me4 = (ys[1] + xs[1]) * 4u;
     const unsigned fb = (unsigned)(c.geo.n * 4);   // bytes of one FP32 field
     // Stores the 16-bit form of t = offset * K and adds its rounding residual
     // (population units) to r.
     auto put = [&](auto lc, const PopPlanes<S>& dst, float t, float& r) {
         constexpr int l = decltype(lc)::value;
-        r += (t - dst.template stb<l>(col.me(), z1 * 2u, t)) * off_unscale(WC[l]);
+        r += (t - dst.template stb<l>(col.me(), dst.zb(zp.v[1]), t)) * off_unscale(WC[l]);
     };
     float rf = 0.0f;
     auto emit = [&](auto lc, float x) {   // x = f*_l / w_l - 1
@@ -1127,16 +1128,18 @@ __device__ __forceinline__ void cell16(const CaseView& c, const fast::Consts& k,
         Field(c.ny, fb).st(me4, z1 * 4u, ncy);
         Field(c.nz, fb).st(me4, z1 * 4u, ncz);
     } else {
-        fdst.template stb<0>(col.me(), z1 * 2u, (k.w0 * x0 + rf) * off_scale(0));
+        fdst.template stb<0>(col.me(), fdst.zb(zp.v[1]), (k.w0 * x0 + rf) * off_scale(0));
 
         const float phin = k.sharp_c * phic * (1.0f - phic);
         if (MODE == COLLIDE_STEP && c.gm != GM_POPULATIONS) {
             // Moment form of g (tau_g = 1): B = 3 phi u + phi_n n (phase_tile_ab).
+            // Which product is fused is written out: the compiler's own choice
+            // changes with the code around it, and a state with it.
             const float p3 = 3.0f * phic;
             const unsigned fb2 = (unsigned)(c.geo.n * 2);
-            Field16(c.gm_u[0], fb2).st(col.me(), z1 * 2u, enc_b(p3 * ux + phin * ncx));
-            Field16(c.gm_u[1], fb2).st(col.me(), z1 * 2u, enc_b(p3 * uy + phin * ncy));
-            Field16(c.gm_u[2], fb2).st(col.me(), z1 * 2u, enc_b(p3 * uz + phin * ncz));
+            Field16(c.gm_u[0], fb2).st(me4 / 2u, z1 * 2u, enc_b(__builtin_fmaf(p3, ux, phin * ncx)));
+            Field16(c.gm_u[1], fb2).st(me4 / 2u, z1 * 2u, enc_b(__builtin_fmaf(phin, ncy, p3 * uy)));
+            Field16(c.gm_u[2], fb2).st(me4 / 2u, z1 * 2u, enc_b(__builtin_fmaf(phin, ncz, p3 * uz)));
             return;
         }
         // g offset of link l after the phase collision, from its odd part.
@@ -1147,9 +1150,11 @@ __device__ __forceinline__ void cell16(const CaseView& c, const fast::Consts& k,
             } else {
                 // (1 - omega_g)(g_pre - w phi) + omega_g (+-odd), with
                 // g_pre - w phi = w (anchor - phi) + t / K.
-                const unsigned vb = col.template src<l>(), zb = zs[1 - CZ[l]];
-                const float pre = __builtin_fmaf(k.template w<l>(), Field(c.phi_prev, fb).ld(vb * 2u, zb * 4u) - phic,
-                                                 gsrc.template ldb<l>(vb, zb * 2u) * off_unscale(WC[l]));
+                const float anchor =
+                    Field(c.phi_prev, fb).ld((ys[1 - CY[l]] + xs[1 - CX[l]]) * 4u, zs[1 - CZ[l]] * 4u);
+                const float pre = __builtin_fmaf(
+                    k.template w<l>(), anchor - phic,
+                    gsrc.template ldb<l>(col.template src<l>(), gsrc.zb(zp.v[1 - CZ[l]])) * off_unscale(WC[l]));
                 return k.one_m_omega_g * pre + k.omega_g * odd;
             }
         };
@@ -1162,7 +1167,7 @@ __device__ __forceinline__ void cell16(const CaseView& c, const fast::Consts& k,
                 put(LinkC<l + 1>{}, gdst, g_off(LinkC<l + 1>{}, -odd) * off_scale(WC[l]), rg);
             }
         });
-        gdst.template stb<0>(col.me(), z1 * 2u, (g_off(LinkC<0>{}, 0.0f) + rg) * off_scale(0));
+        gdst.template stb<0>(col.me(), gdst.zb(zp.v[1]), (g_off(LinkC<0>{}, 0.0f) + rg) * off_scale(0));
     }
 }
 
@@ -1355,7 +1360,7 @@ __device__ __forceinline__ void collide_tile(const CaseView& c, int x0, int y0, 
         };
         if constexpr (S::kAnchored) {
             const float phic = s_phi[z & 3][0][(ty + 2) * PX + (tx + 2)];
-            cell16<MODE>(c, k16, fsrc, gsrc, fdst, gdst, col, me4, zs, fr, nbn, ncx, ncy, ncz, ind, phic);
+            cell16<MODE>(c, k16, fsrc, gsrc, fdst, gdst, col, xs, ys, zs, PopZ(z, G), fr, nbn, ncx, ncy, ncz, ind, phic);
         } else {
             const PopZ zp(z, G);
             float curv, Fx, Fy, Fz;
