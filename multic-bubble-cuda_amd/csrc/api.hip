@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "batch.hpp"
+#include "readback.hpp"
 #include "state.hpp"
 #include "common.hpp"
 #include "fused.hpp"
@@ -38,6 +39,7 @@ struct mcb_ctx {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    std::shared_ptr<Readback> readback = Readback::shared();
     std::vector<hipEvent_t> tev;   // per-kernel timing events
     Tiling tiling{64, 8, 16};
     bool own_tiling = false;   // set by mcb_set_tiling
@@ -704,7 +706,7 @@ mcb_status mcb_read_field(mcb_ctx* c, int field, float* host, size_t n) {
         if (n != 19 * cells) return fail(c, MCB_ERR_INVALID_ARG, "population buffer must hold 19*nx*ny*nz floats");
         if (c->path == MCB_PATH_STAGED) {
             const float* src = field == MCB_FIELD_F ? c->sf : c->sg;
-            MCB_HIP(c, hipMemcpyAsync(host, src, 19 * cells * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+            MCB_HIP(c, Readback::copy(c->readback.get(), host, src, 19 * cells * sizeof(float), c->stream));
         } else {
             if (field == MCB_FIELD_G && c->p.bc_mode == MCB_BC_REFERENCE)
                 return fail(c, MCB_ERR_UNSUPPORTED,
@@ -727,8 +729,8 @@ mcb_status mcb_read_field(mcb_ctx* c, int field, float* host, size_t n) {
             }
             const float* tmp = field == MCB_FIELD_F || c->gm != GM_POPULATIONS ? idle_f : c->g[c->cur ^ 1];
             for (int l = 0; l < 19; ++l)
-                MCB_HIP(c, hipMemcpyAsync(host + l * cells, tmp + (size_t)l * c->geo.plane, cells * sizeof(float),
-                                          hipMemcpyDeviceToHost, c->stream));
+                MCB_HIP(c, Readback::copy(c->readback.get(), host + l * cells, tmp + (size_t)l * c->geo.plane, cells * sizeof(float),
+                                             c->stream));
             if (c->p.bc_mode == MCB_BC_REFERENCE)   // restore the idle buffer's face populations (w_l)
                 MCB_HIP(c, launch_init_pull(c->phi, c->f[c->cur ^ 1], nullptr, c->geo, c->phys, c->stream));
         }
@@ -736,8 +738,7 @@ mcb_status mcb_read_field(mcb_ctx* c, int field, float* host, size_t n) {
         const float* src = scalar_field(c, field);
         if (!src) return fail(c, MCB_ERR_INVALID_ARG, "unknown field");
         if (n != cells) return fail(c, MCB_ERR_INVALID_ARG, "field buffer must hold nx*ny*nz floats");
-        MCB_HIP(c, hipMemcpyAsync(host, src, cells * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-        MCB_HIP(c, hipStreamSynchronize(c->stream));
+        MCB_HIP(c, Readback::copy(c->readback.get(), host, src, cells * sizeof(float), c->stream));
         if (field == MCB_FIELD_PHI && c->path == MCB_PATH_FUSED && c->p.bc_mode == MCB_BC_REFERENCE &&
             c->gm == GM_MOMENTS && src == c->phis[c->cur ^ 1])
             reference_faces_from_interior(c->p, host);

@@ -707,8 +707,7 @@ mcb_status Batch::read(int id, int field, float* host, size_t n) {
             e = launch_decode16(isf ? c->f[c->cur] : c->g[c->cur], isf ? nullptr : c->phi[c->cur ^ 1], tmp, c->geo,
                                 c->phys, c->storage, stream_);
         for (int l = 0; l < 19 && e == hipSuccess; ++l)
-            e = hipMemcpyAsync(host + l * cells, tmp + l * P, cells * sizeof(float), hipMemcpyDeviceToHost, stream_);
-        if (e == hipSuccess) e = hipStreamSynchronize(stream_);
+            e = Readback::copy(readback_.get(), host + l * cells, tmp + l * P, cells * sizeof(float), stream_);
         (void)hipFree(tmp);
         B_HIP(e);
         return MCB_OK;
@@ -723,8 +722,7 @@ mcb_status Batch::read(int id, int field, float* host, size_t n) {
     } else {
         return fail(MCB_ERR_INVALID_ARG, "unknown field");
     }
-    B_HIP(hipMemcpyAsync(host, src, cells * sizeof(float), hipMemcpyDeviceToHost, stream_));
-    B_HIP(hipStreamSynchronize(stream_));
+    B_HIP(Readback::copy(readback_.get(), host, src, cells * sizeof(float), stream_));
     return MCB_OK;
 }
 

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "fused.hpp"
+#include "readback.hpp"
 #include "state.hpp"
 
 namespace mcb {
@@ -146,6 +147,7 @@ private:
 
     int device_;
     hipStream_t stream_;
+    std::shared_ptr<Readback> readback_ = Readback::shared();
     std::string err_;
     std::map<int, std::unique_ptr<CaseState>> cases_;
     std::vector<int> order_;          // case ids in view-array order (by group)
