@@ -50,13 +50,24 @@ std::vector<WorkItem> xcd_permute(const std::vector<WorkItem>& in) {
 
 }  // namespace
 
+// Whether a 16-bit lattice alone steps on tiles of whole rows (plain rows, then;
+// see fused_geo): where one is instantiated, rows are not whole lines, and its
+// workgroups fill 11 of a CU's 16 waves (48, 80, 112, 176: 80x230x160 106 us per
+// step against 120 with the next best tile, 176^3 155 against 187; not 144, one
+// 9-wave workgroup a CU: 125 against 116 with 64x4).
+static bool keeps_row_tile16(int nx) {
+    const int waves = nx / 16;
+    return tiling_supported16(Tiling{nx, 4, 1}) && nx % 32 != 0 && 16 / waves * waves >= 11;
+}
+
 Geo fused_geo(const mcb_params& p, bool pad_rows) {
     Geo g{p.nx, p.ny, p.nz, p.nx * p.ny, (long long)p.nx * p.ny * p.nz, 0, 0, p.nx, p.nx * p.ny};
     g.plane = plane_stride_cells(g.n);
     if (p.f_form != MCB_F_POPULATIONS) return g;
     const bool fp32 = p.storage == MCB_STORE_FP32;
     const int group = fp32 ? 64 : 1;
-    if (p.nx < 16 || (!fp32 && tiling_supported16(Tiling{p.nx, 4, 1}))) pad_rows = false;   // at most twice the memory
+    const bool row = p.tau_g == 1.0f ? keeps_row_tile16(p.nx) : tiling_supported16(Tiling{p.nx, 4, 1});
+    if (p.nx < 16 || (!fp32 && row)) pad_rows = false;   // at most twice the memory
     for (const int pitch : {(p.nx + 31) / 32 * 32, p.nx}) {
         if (pitch != p.nx && !pad_rows) continue;
         const long long zp = ((long long)pitch * p.ny + group - 1) / group * group, plane = plane_stride_cells(zp * p.nz);
@@ -172,28 +183,55 @@ Tiling choose_tiling_single(const mcb_params& p) {
         auto it = g_tuned.find(std::make_tuple(p.nx, p.ny, p.nz, p.storage));
         if (it != g_tuned.end()) return it->second;
     }
-    // A lattice alone on the device: shorter z-chunks until its workgroups
-    // have 16 waves for every CU (256 CUs; what 128 VGPRs allow), whatever the
-    // tile. FP32 (us per collide): the reference preset (64x64x256) 64x8x4,
-    // 64^3 64x8x1 20.2 (64x4x4: 25.6). 16 bits (us per step): 117x90x133
-    // 64x4x4 65 (64x8x32, sized for a full device, 147), 128^3 64x4x8 64
-    // (64x4x16 75), 64^3 64x4x2 22.6 (64x4x16 54).
     Tiling t = choose_tiling(p);
     const bool fp32 = p.storage == MCB_STORE_FP32;
     // Stored 16-bit g sums its mass in FP64 tile by tile: the tiles of a batch
     // case, so that a state image continues with the same bits in either.
     if (!fp32 && p.tau_g != 1.0f) return t;
+    // A lattice alone on the device (us per step, this rule against 64x8x16,
+    // 16 bits 32x8x32 and 64x8x32): 4-row tiles, so that twice the workgroups
+    // share the CUs, and short chunks, so that the planes that neighbouring
+    // chunks read twice are still in L2. FP32 64x4x8 192^3 298 (319), 180^3 279
+    // (300); stored g, with twice the planes, 64x4x2 250^3 1152 (1265), 180^3
+    // 459 (524), 96x220x200 308 (356). 16 bits 64x4x8 240x250x100 170 (207),
+    // 200^3 264 (304), 180^3 167 (186); 16 planes once they fill the device four
+    // times over (256^3 397, 8 planes 406).
+    const int pad64 = (p.nx + 63) / 64 * 64, pad32 = (p.nx + 31) / 32 * 32;
+    const bool moments = p.tau_g == 1.0f;
+    bool row = false;
+    if (p.nx > 32 && p.f_form == MCB_F_POPULATIONS) {
+        row = !fp32 && keeps_row_tile16(p.nx);
+        // 32-wide tiles where 64-wide ones would pad more lanes: FP32 80x230x160
+        // 156 against 204, 160^3 196 against 226, 224^3 453 against 501; in 16
+        // bits, whose 64 lanes of a row are two lines, only where they pad a
+        // fourth, or a sixth with whole 32-cell rows (96^3 41 against 42, 160^3
+        // 128 against 137, but 150x105x77 56 against 54, 224^3 331 against 319).
+        const bool narrow =
+            p.nx > 64 && (fp32 ? pad32 < pad64 : pad32 * 6 < pad64 * 5 + (p.nx % 32 == 0 ? 1 : 0));
+        if (row) t = Tiling{p.nx, 4, 16};
+        else if (narrow) t = Tiling{32, 8, fp32 ? (moments ? 4 : 2) : 16};
+        else t = Tiling{64, 4, fp32 ? (moments ? 8 : 2) : 16};
+        t.zc = std::min(t.zc, p.nz);
+    }
     auto lanes = [&](const Tiling& q) {
         return (long long)((p.nx + q.tx - 1) / q.tx) * ((p.ny + q.ty - 1) / q.ty) * ((p.nz + q.zc - 1) / q.zc) * q.tx *
                q.ty;
     };
-    while (t.zc > (fp32 ? 1 : 2) && lanes(t) < 256 * 16 * 64) t.zc /= 2;
-    // Where the chunks are down to 4 planes, 4-row tiles give twice the
-    // workgroups for the same halo restaging per plane (the reference
-    // preset: 64x4x4 43.9 us per collide against 46.4 with 64x8x4); with one
-    // or two planes a tile's own halo weighs more (64^3: 64x8x1 20.2, 64x4x1
-    // 22.4; 16 bits keep 4 rows, 2 planes being their least).
-    if (t.zc <= 4 && (t.zc > 2 || !fp32) && t.tx == 64 && t.ty == 8) t.ty = 4;
+    const long long wave_per_cu = 256 * 64;   // lanes: one wave on each of 256 CUs
+    if (!fp32 && !row && t.zc > 8 && lanes(t) < 4 * 16 * wave_per_cu) t.zc = 8;
+    // Shorter chunks until most of a CU's 16 waves (what 128 VGPRs allow) are
+    // there: 13 in FP32 (112^3 64x4x8, 12.3 waves, 85.7 us, 4 planes 79; 96^3
+    // 32x8x4, 13.5 waves, 50.8, 2 planes 52.7), 11 in 16 bits (117x90x133 8
+    // planes, 12.2 waves, 54.8, 4 planes 56.1) and before single planes
+    // (40x100x60 64x4x2, 11.7 waves, 25.9, 1 plane 31); 7 with whole rows, whose
+    // halo is small (112^3 8 planes 58.9, 4 planes 60.8). One plane is the
+    // least, 2 in 16 bits.
+    auto want = [&] { return (row ? 7 : (fp32 && t.zc > 2 ? 13 : 11)) * wave_per_cu; };
+    while (t.zc > (fp32 ? 1 : 2) && lanes(t) < want()) t.zc /= 2;
+    // Single planes restage their own halo: 8 rows where they pad no more
+    // (64^3 with stored g 23.2 against 25.6), in 32-wide tiles where 64 lanes
+    // do not fill (48^3 18.2 against 19.1).
+    if (t.zc == 1 && t.tx == 64 && t.ty == 4 && p.ny % 8 == 0) t = Tiling{p.nx % 64 == 0 ? 64 : 32, 8, 1};
     return t;
 }
 

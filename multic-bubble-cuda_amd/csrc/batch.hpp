@@ -192,8 +192,8 @@ private:
 // Tile shape for a lattice: the autotuned choice for (nx, ny, nz, storage)
 // when one exists, else a size rule.
 Tiling choose_tiling(const mcb_params& p);
-// The tiling of a single-case context: as choose_tiling, with z-chunks short
-// enough that a small lattice alone still fills the device.
+// The tiling of a single-case context: the autotuned choice, else a rule for a
+// lattice that has the device to itself.
 Tiling choose_tiling_single(const mcb_params& p);
 // The tiling of a batch case, where the batch fills the device: by row length
 // in FP32, the 16-bit rule of choose_tiling otherwise.

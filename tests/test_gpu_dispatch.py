@@ -135,3 +135,23 @@ def test_16bit_image_with_written_g_moves_between_context_and_batch(gpu_lib):
         other.step(4)
         assert np.array_equal(other.read("phi"), lat.read("phi"))
     lat.close()
+
+
+@pytest.mark.parametrize("storage,tau_g,nx,ny,nz", [
+    (0, 1.0, 33, 24, 60), (0, 0.8, 72, 33, 20), (0, 0.8, 48, 16, 9), (0, 1.0, 160, 64, 40), (0, 0.8, 130, 70, 33),
+    (1, 1.0, 96, 40, 24), (1, 1.0, 144, 36, 30), (1, 1.0, 112, 20, 50), (1, 1.0, 40, 30, 20), (2, 1.0, 200, 90, 70)])
+def test_tiles_of_a_lattice_alone(gpu_lib, storage, tau_g, nx, ny, nz):
+    """The tile that a context picks against tiles of 16x16x3: no cell's arithmetic depends on its tile."""
+    mcb = gpu_lib
+    p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.7, tau_g=tau_g)
+    got = []
+    for tiling in (None, (16, 16, 3)):
+        lat = mcb.Lattice(p)
+        if tiling:
+            lat.set_tiling(*tiling)
+        lat.init_bubbles([(0.4 * nx, 0.5 * ny, 0.5 * nz, 0.3 * min(nx, ny, nz))], 3.0)
+        lat.step(6)
+        got.append((lat.read("phi"), lat.read("f")))
+        lat.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
