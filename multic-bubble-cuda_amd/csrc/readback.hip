@@ -20,8 +20,8 @@ namespace {
 // chunks for large reads (64 MiB in 2 MiB chunks 1.8 ms), 2 MiB below (4 MiB
 // 155 us against 190 with twice the threads and 247 direct, 8 MiB 275 against
 // 490).
-constexpr size_t kSlots = 4, kSlice = 256u << 10, kMaxChunk = 4u << 20, kLarge = 16u << 20;
-constexpr size_t chunk_of(size_t bytes) { return bytes >= kLarge ? kMaxChunk : 2u << 20; }
+constexpr size_t kSlots = 4, kSlice = 256u << 10, kLarge = 16u << 20;
+constexpr size_t chunk_of(size_t bytes) { return bytes >= kLarge ? 4u << 20 : 2u << 20; }
 constexpr unsigned threads_of(size_t bytes) { return bytes >= kLarge ? 8 : 4; }
 // Below this the direct copy is about as fast (2 MiB: 123 us), and starting
 // threads costs what it could gain.
@@ -62,12 +62,20 @@ Readback::~Readback() {
     if (ring_) (void)hipHostFree(ring_);
 }
 
-bool Readback::ready() {
-    if (!ring_ && hipHostMalloc(reinterpret_cast<void**>(&ring_), kSlots * kMaxChunk, hipHostMallocPortable) != hipSuccess) {
+// Room for a read of `bytes`; pinning costs 30 us per MiB and more.
+bool Readback::ready(size_t bytes) {
+    const size_t chunk = chunk_of(bytes), need = std::min((bytes + chunk - 1) / chunk, kSlots) * chunk;
+    if (ring_bytes_ >= need) return true;
+    if (ring_) (void)hipHostFree(ring_);
+    ring_ = nullptr;
+    ring_bytes_ = 0;
+    if (hipHostMalloc(reinterpret_cast<void**>(&ring_), need, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
         ring_ = nullptr;
+        return false;
     }
-    return ring_ != nullptr;
+    ring_bytes_ = need;
+    return true;
 }
 
 hipError_t Readback::copy(Readback* r, void* host, const void* dev, size_t bytes, hipStream_t stream) {
@@ -75,7 +83,7 @@ hipError_t Readback::copy(Readback* r, void* host, const void* dev, size_t bytes
     if (r && bytes >= kMinBytes && pageable(host) && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
         cs == hipStreamCaptureStatusNone) {
         std::unique_lock<std::mutex> lk(r->mu_, std::try_to_lock);
-        if (lk.owns_lock() && r->ready())
+        if (lk.owns_lock() && r->ready(bytes))
             return r->staged(static_cast<char*>(host), static_cast<const char*>(dev), bytes, stream);
     }
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream);

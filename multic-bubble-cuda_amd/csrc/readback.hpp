@@ -10,9 +10,9 @@
 namespace mcb {
 
 // A ring of pinned memory that large copies pass through. Contexts and
-// batches share one ring: it is allocated by the first large read, serves one
-// read at a time (a second one meanwhile copies without it) and is freed with
-// the last context or batch.
+// batches share one ring: it grows to what the largest read needs (16 MiB at
+// most), serves one read at a time (a second one meanwhile copies without it)
+// and is freed with the last context or batch.
 class Readback {
 public:
     static std::shared_ptr<Readback> shared() noexcept;   // null where memory is short
@@ -23,11 +23,12 @@ public:
     static hipError_t copy(Readback* r, void* host, const void* dev, size_t bytes, hipStream_t stream);
 
 private:
-    bool ready();
+    bool ready(size_t bytes);
     hipError_t staged(char* host, const char* dev, size_t bytes, hipStream_t stream);
 
     std::mutex mu_;
     char* ring_ = nullptr;
+    size_t ring_bytes_ = 0;
 };
 
 }  // namespace mcb
