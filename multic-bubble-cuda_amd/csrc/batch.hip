@@ -66,8 +66,7 @@ Geo fused_geo(const mcb_params& p, bool pad_rows) {
     if (p.f_form != MCB_F_POPULATIONS) return g;
     const bool fp32 = p.storage == MCB_STORE_FP32;
     const int group = fp32 ? 64 : 1;
-    const bool row = p.tau_g == 1.0f ? keeps_row_tile16(p.nx) : tiling_supported16(Tiling{p.nx, 4, 1});
-    if (p.nx < 16 || (!fp32 && row)) pad_rows = false;   // at most twice the memory
+    if (p.nx < 16 || (!fp32 && keeps_row_tile16(p.nx))) pad_rows = false;   // at most twice the memory
     for (const int pitch : {(p.nx + 31) / 32 * 32, p.nx}) {
         if (pitch != p.nx && !pad_rows) continue;
         const long long zp = ((long long)pitch * p.ny + group - 1) / group * group, plane = plane_stride_cells(zp * p.nz);
@@ -97,6 +96,9 @@ CaseView CaseState::view(int q) const {
     v.zc = tiling.zc;
     v.tx = tiling.tx;
     v.ty = tiling.ty;
+    v.stx = sum.tx;
+    v.sty = sum.ty;
+    v.szc = sum.zc;
     v.fsrc = f[q];
     v.fdst = f[q ^ 1];
     v.gsrc = g[q];
@@ -185,9 +187,6 @@ Tiling choose_tiling_single(const mcb_params& p) {
     }
     Tiling t = choose_tiling(p);
     const bool fp32 = p.storage == MCB_STORE_FP32;
-    // Stored 16-bit g sums its mass in FP64 tile by tile: the tiles of a batch
-    // case, so that a state image continues with the same bits in either.
-    if (!fp32 && p.tau_g != 1.0f) return t;
     // A lattice alone on the device (us per step, this rule against 64x8x16,
     // 16 bits 32x8x32 and 64x8x32): 4-row tiles, so that twice the workgroups
     // share the CUs, and short chunks, so that the planes that neighbouring
@@ -195,7 +194,9 @@ Tiling choose_tiling_single(const mcb_params& p) {
     // (300); stored g, with twice the planes, 64x4x2 250^3 1152 (1265), 180^3
     // 459 (524), 96x220x200 308 (356). 16 bits 64x4x8 240x250x100 170 (207),
     // 200^3 264 (304), 180^3 167 (186); 16 planes once they fill the device four
-    // times over (256^3 397, 8 planes 406).
+    // times over (256^3 397, 8 planes 406). 16-bit stored g, whose sums have
+    // tiles of their own (build_own_table): 117x90x133 121 (315), 64^3 30 (101),
+    // 200^3 756 (987).
     const int pad64 = (p.nx + 63) / 64 * 64, pad32 = (p.nx + 31) / 32 * 32;
     const bool moments = p.tau_g == 1.0f;
     bool row = false;
@@ -373,6 +374,7 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
     c->storage = p.storage;
     c->mode = p.tau_g == 1.0f ? COLLIDE_STEP : COLLIDE_STEP_BGK;
     c->tiling = t;
+    c->alone = pad_rows;
     // FP32 populations in 64-cell blocks (16-bit ones stay in planes: with
     // blocks the FP16 batch ran 3% slower).
     c->geo = geo;
@@ -463,6 +465,12 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
 mcb_status Batch::build_own_table(CaseState* c) {
     auto own = xcd_permute(tiles_of(*c, 0));
     c->n_work = (unsigned)own.size();
+    // Stored 16-bit g adds its FP64 sums tile by tile. In a context they
+    // keep the tiles of a batch case, whatever the context steps on: a state
+    // image continues with the same bits in either.
+    c->sum = c->alone && c->mass && !c->own_tiling ? batch_tiling(c->p) : c->tiling;
+    auto over = [](int n, int t) { return (size_t)((n + t - 1) / t); };
+    const size_t sums = over(c->p.nx, c->sum.tx) * over(c->p.ny, c->sum.ty) * over(c->p.nz, c->sum.zc);
     if (own.size() > c->work_cap) {
         if (c->d_work) B_HIP(hipFree(c->d_work));
         c->d_work = nullptr;
@@ -471,12 +479,13 @@ mcb_status Batch::build_own_table(CaseState* c) {
         c->work_cap = own.size();
     }
     B_HIP(hipMemcpyAsync(c->d_work, own.data(), own.size() * sizeof(WorkItem), hipMemcpyHostToDevice, stream_));
-    if ((c->mass || c->massq) && c->n_work > c->partial_cap) {
+    const size_t parts = std::max<size_t>(c->n_work, sums);
+    if ((c->mass || c->massq) && parts > c->partial_cap) {
         if (c->partial) B_HIP(hipFree(c->partial));
         c->partial = nullptr;
         c->partial_cap = 0;
-        B_HIP(hipMalloc(reinterpret_cast<void**>(&c->partial), c->n_work * sizeof(double)));
-        c->partial_cap = c->n_work;
+        B_HIP(hipMalloc(reinterpret_cast<void**>(&c->partial), parts * sizeof(double)));
+        c->partial_cap = parts;
     }
     B_HIP(hipStreamSynchronize(stream_));   // own is a host temporary
     return MCB_OK;
@@ -593,6 +602,10 @@ mcb_status Batch::rebuild() {
         gr.t = Tiling{c0->tiling.tx, c0->tiling.ty, 0};
         gr.mode = c0->mode;
         gr.mass = false;
+        gr.sum = c0->sum;   // of its own: a case alone (a context) only
+        if (!c0->alone || !c0->mass || (c0->sum.tx == c0->tiling.tx && c0->sum.ty == c0->tiling.ty && c0->sum.zc == c0->tiling.zc))
+            gr.sum.zc = 0;
+        gr.geo = c0->geo;
         std::vector<WorkItem> items;
         long long work = 0;
         for (size_t i = start[k]; i < end; ++i) {
@@ -650,6 +663,7 @@ mcb_status Batch::launch_steps(int q, int n) {
             const Group& gr = groups_[i];
             const hipStream_t s = fork && gr.lane ? lane_[gr.lane - 1] : stream_;
             e = launch_phase_batch(d_views_[q], gr.d_work, gr.n, gr.t, storage_, s);
+            if (e == hipSuccess && gr.sum.zc) e = launch_mass_sum(d_views_[q] + gr.first, gr.geo, gr.sum, s);
             if (e == hipSuccess && gr.mass) e = launch_mass_finish(d_views_[q] + gr.first, gr.cases, s);
             if (e == hipSuccess) e = launch_collide_batch(d_views_[q], gr.d_work, gr.n, gr.t, gr.mode, storage_, s);
         }
@@ -779,7 +793,6 @@ mcb_status Batch::to_populations(CaseState* c) {
         if (st != MCB_OK) return st;
         c->allocs.emplace_back(q, sizeof(MassCell));
         c->mass = static_cast<MassCell*>(q);
-        if (!c->own_tiling) c->tiling = batch_tiling(c->p);   // see choose_tiling_single
         if ((st = build_own_table(c)) != MCB_OK) return st;   // partial sums
     }
     c->gm = GM_POPULATIONS;
@@ -1015,8 +1028,7 @@ mcb_status Batch::set_tiling(int id, const Tiling& t, bool by_caller) {
     if (!supported_for(t, c->storage) || t.zc > c->p.nz) return fail(MCB_ERR_INVALID_ARG, "unsupported tiling");
     B_HIP(hipSetDevice(device_));
     B_HIP(hipStreamSynchronize(stream_));
-    // The library's own choice for a moment form does not hold for stored g.
-    c->tiling = !by_caller && c->mass ? batch_tiling(c->p) : t;
+    c->tiling = t;
     c->own_tiling = by_caller;
     mcb_status st = build_own_table(c);
     if (st != MCB_OK) return st;

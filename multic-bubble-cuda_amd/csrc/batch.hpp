@@ -30,6 +30,8 @@ struct CaseState {
     int mode = COLLIDE_STEP;       // COLLIDE_STEP or COLLIDE_STEP_BGK
     Tiling tiling{64, 8, 16};
     bool own_tiling = false;        // set by the library's caller
+    bool alone = false;             // a context's only case
+    Tiling sum{64, 8, 16};          // tiles of the sum of phi of stored 16-bit g (build_own_table)
     int cur = 0;                    // population buffer of the current state
     int parity_offset = 0;          // cur = batch parity ^ parity_offset
     long long steps = 0;            // steps taken since init
@@ -168,6 +170,8 @@ private:
         size_t cap = 0;
         unsigned n = 0;
         unsigned first = 0, cases = 0;
+        Tiling sum{};                    // zc > 0: its only case sums phi on tiles of its own (launch_mass_sum)
+        Geo geo{};                       // of that case
         bool mass = false;               // a case keeps a mass-drift correction (MassCell or MassQ)
         int lane = 0;                    // 0: stream_, i: lane_[i - 1]
     };

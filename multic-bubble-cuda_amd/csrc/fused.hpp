@@ -38,7 +38,8 @@ struct Tiling {
 
 // Mass bookkeeping of a case with 16-bit populations (device memory). The
 // phase pass adds delta[q] to every phi it computes at case parity q and
-// writes one FP64 partial sum of phi per work item; after the pass
+// writes one FP64 partial sum of phi per work item (or launch_mass_sum, for
+// tiles of its own, after it); after the pass
 // launch_mass_finish sums the partials in a fixed order and stores
 // delta[q ^ 1] = (target - sum phi) / cells for the next step.
 struct MassCell {
@@ -75,6 +76,7 @@ struct CaseView {
     Phys phys;
     int zc;                 // z planes per collide workgroup
     int tx, ty;             // tile of the case's work items
+    int stx, sty, szc;      // tiles of the sum of phi (mass): the work items', or launch_mass_sum's own
     int mslot;              // parity of the case's state: delta slot the phase pass reads
     MassCell* mass;         // 16-bit storage only
     MassQ* massq;           // 16-bit storage in moment form only
@@ -187,6 +189,9 @@ hipError_t launch_pop_relayout(const void* src, int sdev, void* dst, int ddev, c
 
 // ---- batched (many cases, one launch per pass), any storage form
 // storage: MCB_STORE_FP32 / FP16 / BF16; work: device array of n_work items.
+// After the phase pass of a stored-g case whose sum of phi has tiles of its own
+// (view; sum: the same tile): its FP64 partials of the phi the pass wrote.
+hipError_t launch_mass_sum(const CaseView* view, const Geo& geo, const Tiling& sum, hipStream_t s);
 // After a batch's phase pass: the mass-drift corrections of its 16-bit
 // cases (MassCell for stored g, MassQ for the moment form), one workgroup
 // per case of the view array.

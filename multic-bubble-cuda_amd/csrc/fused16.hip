@@ -193,6 +193,29 @@ bool tiling_supported16(const Tiling& t) {
 }
 
 namespace {
+// launch_mass_sum: the partial that k_phase_batch writes with the tiles szc
+// planes long, from the phi it stored (the same additions in the same order).
+// Stored g is summed on the tiles of a batch case, so that its bits do not
+// depend on where it runs; a lattice alone steps on shorter ones. 4 bytes a
+// cell, most of them still in L2.
+template <int TX, int TY>
+__global__ __launch_bounds__(TX * TY) void k_mass_sum(const CaseView* __restrict__ view) {
+    const CaseView c = *view;
+    const Geo& G = c.geo;
+    const unsigned gx = (unsigned)(G.nx + TX - 1) / TX, gy = (unsigned)(G.ny + TY - 1) / TY;
+    const unsigned tile = blockIdx.x, row = tile / gx;
+    const int x = (int)(tile % gx) * TX + (int)threadIdx.x, y = (int)(row % gy) * TY + (int)threadIdx.y;
+    const int z0 = (int)(row / gy) * c.szc, ze = min(z0 + c.szc, G.nz);
+    double part = 0.0;
+    if (x < G.nx && y < G.ny) {
+        const float* phi = c.phi + (long long)y * G.nx + x;
+#pragma unroll 8
+        for (int z = z0; z < ze; ++z) part += (double)phi[(long long)z * G.nxy];
+    }
+    const double s = block_sum<TX * TY>(part);
+    if (threadIdx.y == 0 && threadIdx.x == 0) c.partial[tile] = s;
+}
+
 // launch_mass_finish: one workgroup per case of the view array.
 constexpr int kFinishThreads = 256;
 __global__ __launch_bounds__(kFinishThreads) void k_mass_finish(const CaseView* __restrict__ cases) {
@@ -201,8 +224,10 @@ __global__ __launch_bounds__(kFinishThreads) void k_mass_finish(const CaseView* 
     const unsigned n_tiles = (unsigned)((G.nx + c.tx - 1) / c.tx) * (unsigned)((G.ny + c.ty - 1) / c.ty) *
                              (unsigned)((G.nz + c.zc - 1) / c.zc);
     if (c.mass && c.gm == GM_POPULATIONS) {   // stored 16-bit g: FP64 partials, fixed order
+        const unsigned n_sums = (unsigned)((G.nx + c.stx - 1) / c.stx) * (unsigned)((G.ny + c.sty - 1) / c.sty) *
+                                (unsigned)((G.nz + c.szc - 1) / c.szc);
         double acc = 0.0;
-        for (unsigned i = threadIdx.x; i < n_tiles; i += kFinishThreads) acc += c.partial[i];
+        for (unsigned i = threadIdx.x; i < n_sums; i += kFinishThreads) acc += c.partial[i];
         const double total = block_sum<kFinishThreads>(acc);
         if (threadIdx.x == 0) c.mass->delta[c.mslot ^ 1] = (c.mass->target - total) / (double)G.n;
         return;
@@ -224,6 +249,19 @@ __global__ __launch_bounds__(kFinishThreads) void k_mass_finish(const CaseView* 
     }
 }
 }  // namespace
+
+hipError_t launch_mass_sum(const CaseView* view, const Geo& geo, const Tiling& sum, hipStream_t s) {
+    const unsigned tiles = (unsigned)((geo.nx + sum.tx - 1) / sum.tx) * (unsigned)((geo.ny + sum.ty - 1) / sum.ty) *
+                           (unsigned)((geo.nz + sum.zc - 1) / sum.zc);
+#define MCB_TILE_CASE(TX, TY)                                                                     \
+    if (sum.tx == TX && sum.ty == TY) {                                                           \
+        hipLaunchKernelGGL((k_mass_sum<TX, TY>), dim3(tiles), dim3(TX, TY, 1), 0, s, view);       \
+        return hipGetLastError();                                                                 \
+    }
+    MCB_TILES_16(MCB_TILE_CASE)
+#undef MCB_TILE_CASE
+    return hipErrorInvalidValue;
+}
 
 hipError_t launch_mass_finish(const CaseView* cases, unsigned n_cases, hipStream_t s) {
     if (n_cases == 0) return hipSuccess;

@@ -1843,7 +1843,7 @@ __global__ __launch_bounds__(TX * TY) void k_phase_batch(const CaseView* __restr
             st32(c.phi, zs[1] + ys[1] + xs[1], v);
         }
     }
-    if (mass) mass_partial<TX, TY>(c, w, part);
+    if (mass && c.stx == c.tx && c.sty == c.ty && c.szc == c.zc) mass_partial<TX, TY>(c, w, part);
 }
 
 // 16-bit collide with more than 10 waves per workgroup (the 176 x 4 tile):

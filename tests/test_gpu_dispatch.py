@@ -155,3 +155,21 @@ def test_tiles_of_a_lattice_alone(gpu_lib, storage, tau_g, nx, ny, nz):
         lat.close()
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", [1, 2])
+@pytest.mark.parametrize("nx,ny,nz", [(33, 13, 70), (64, 64, 33), (80, 9, 40), (112, 10, 17), (130, 66, 35), (20, 18, 50)])
+def test_mass_sum_of_stored_g_alone(gpu_lib, storage, nx, ny, nz):
+    """A context sums phi on a batch case's tiles whatever tiles it steps on: the bits of the correction are the same."""
+    mcb = gpu_lib
+    p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.6, tau_g=0.8)
+    bubble = [(0.4 * nx, 0.5 * ny, 0.5 * nz, 0.3 * min(nx, ny, nz))]
+    with mcb.Lattice(p) as lat, mcb.Batch(storage) as b:
+        lat.init_bubbles(bubble, 3.0)
+        lat.step(8)
+        phi0 = lat.read("phi")
+        cid = b.add_state(lat.save_state())
+        lat.step(8)
+        b.step(8)
+        assert np.array_equal(b.read(cid, "phi"), lat.read("phi"))
+        assert abs(float(lat.read("phi").sum(dtype=np.float64)) - float(phi0.sum(dtype=np.float64))) <= 1e-3
