@@ -198,8 +198,8 @@ mcb_status mcb_autotune(const mcb_params* p, int* tx, int* ty, int* zc, double* 
 
 /* ---- Batches: many independent periodic cases resident on one device ----
  * A batch step advances every case by one step with one launch per pass for
- * all cases (grouped by tile shape); two steps at a time are replayed from a
- * captured hipGraph. All cases of a batch share one storage form. Cases never
+ * all cases of a tile shape; the groups run side by side on up to four
+ * streams, joined to the batch's stream by events. All cases of a batch share one storage form. Cases never
  * exchange data: a case's results do not depend on the rest of the batch.
  * No reference counterpart (the reference runs one lattice per process). */
 typedef struct mcb_batch mcb_batch;
