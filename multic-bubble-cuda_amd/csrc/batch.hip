@@ -32,9 +32,8 @@ constexpr long long kGroupCells = 1LL << 20;
 // the list (against xcd_order, where each XCD walks its own range: the 64
 // FP32 'batch' presets 22.0k -> 22.4k MLUPS, FP16 at 256^3 41.5k -> 42.7k,
 // 128^3 and 144^3 within 0.5%; without renumbering FP16 ran 2-7% slower).
-std::vector<WorkItem> tiles_of(const CaseState& c, int slot) {
+std::vector<WorkItem> tiles_of(const CaseState& c, int slot, const Tiling& t) {
     std::vector<WorkItem> v;
-    const Tiling& t = c.tiling;
     for (int z0 = 0; z0 < c.p.nz; z0 += t.zc)
         for (int y0 = 0; y0 < c.p.ny; y0 += t.ty)
             for (int x0 = 0; x0 < c.p.nx; x0 += t.tx) v.push_back(WorkItem{slot, x0, y0, z0});
@@ -80,6 +79,22 @@ Geo fused_geo(const mcb_params& p, bool pad_rows) {
     return g;
 }
 
+// Tiles of the 16-bit (phi, B) phase pass of a lattice alone that collides on
+// t. The pass stages a halo of one cell: 4-row tiles of 64 stage 1.55 cells for
+// each of theirs, 8 rows 1.29 (256^3: 37 against 28 LDS instructions a cell),
+// while the collide pass wants the many small workgroups. Where 8 rows and
+// longer chunks leave three workgroups a CU: 100 steps and a read of 256^3 FP16
+// 41.0 ms against 42.2, 192^3 BF16 18.7 against 18.6; below that 4 rows keep more
+// of the device busy (117x90x133 57 us per step against 59). The fixed-point
+// sums of phi do not depend on the tiles.
+static Tiling phase_tiling16(const mcb_params& p, const Tiling& t) {
+    if (t.tx != 64 || t.ty != 4) return t;
+    auto groups = [&](int zc) { return (long long)((p.nx + 63) / 64) * ((p.ny + 7) / 8) * ((p.nz + zc - 1) / zc); };
+    for (int zc = std::min(32, p.nz); zc > t.zc; zc /= 2)
+        if (groups(zc) >= 768) return Tiling{64, 8, zc};
+    return t;
+}
+
 size_t case_bytes(const mcb_params& p, bool pad_rows) {
     const size_t P = (size_t)fused_geo(p, pad_rows).plane;
     const bool moments = p.tau_g == 1.0f;
@@ -96,6 +111,9 @@ CaseView CaseState::view(int q) const {
     v.zc = tiling.zc;
     v.tx = tiling.tx;
     v.ty = tiling.ty;
+    v.ptx = phase.tx;
+    v.pty = phase.ty;
+    v.pzc = phase.zc;
     v.stx = sum.tx;
     v.sty = sum.ty;
     v.szc = sum.zc;
@@ -463,14 +481,16 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
 // The case's own work table (case index 0, used with the case's entry of the
 // view arrays as the base) and its partial-sum buffer, for its tiling.
 mcb_status Batch::build_own_table(CaseState* c) {
-    auto own = xcd_permute(tiles_of(*c, 0));
+    auto own = xcd_permute(tiles_of(*c, 0, c->tiling));
     c->n_work = (unsigned)own.size();
     // Stored 16-bit g adds its FP64 sums tile by tile. In a context they
     // keep the tiles of a batch case, whatever the context steps on: a state
     // image continues with the same bits in either.
     c->sum = c->alone && c->mass && !c->own_tiling ? batch_tiling(c->p) : c->tiling;
+    c->phase = c->alone && c->massq && !c->mass && !c->own_tiling ? phase_tiling16(c->p, c->tiling) : c->tiling;
     auto over = [](int n, int t) { return (size_t)((n + t - 1) / t); };
-    const size_t sums = over(c->p.nx, c->sum.tx) * over(c->p.ny, c->sum.ty) * over(c->p.nz, c->sum.zc);
+    auto count = [&](const Tiling& t) { return over(c->p.nx, t.tx) * over(c->p.ny, t.ty) * over(c->p.nz, t.zc); };
+    const size_t sums = std::max(count(c->sum), count(c->phase));
     if (own.size() > c->work_cap) {
         if (c->d_work) B_HIP(hipFree(c->d_work));
         c->d_work = nullptr;
@@ -537,10 +557,10 @@ mcb_status Batch::rebuild() {
     B_HIP(hipStreamSynchronize(stream_));
     mcb_status st = ensure_macro_scratch();
     if (st != MCB_OK) return st;
-    // Cases in the order of their groups (tile shape and collide mode).
+    // Cases in the order of their groups (tile shapes and collide mode).
     auto key = [&](int id) {
         const CaseState* c = cases_[id].get();
-        return std::make_tuple(c->tiling.tx, c->tiling.ty, c->mode);
+        return std::make_tuple(c->tiling.tx, c->tiling.ty, c->mode, c->phase.tx, c->phase.ty);
     };
     order_.clear();
     for (auto& kv : cases_) order_.push_back(kv.first);
@@ -600,22 +620,33 @@ mcb_status Batch::rebuild() {
         gr.cases = (unsigned)(end - start[k]);
         const CaseState* c0 = cases_[order_[start[k]]].get();
         gr.t = Tiling{c0->tiling.tx, c0->tiling.ty, 0};
+        gr.pt = Tiling{c0->phase.tx, c0->phase.ty, 0};
         gr.mode = c0->mode;
         gr.mass = false;
         gr.sum = c0->sum;   // of its own: a case alone (a context) only
         if (!c0->alone || !c0->mass || (c0->sum.tx == c0->tiling.tx && c0->sum.ty == c0->tiling.ty && c0->sum.zc == c0->tiling.zc))
             gr.sum.zc = 0;
         gr.geo = c0->geo;
-        std::vector<WorkItem> items;
+        std::vector<WorkItem> items, phase;
+        bool differ = false;
         long long work = 0;
         for (size_t i = start[k]; i < end; ++i) {
             const CaseState* c = cases_[order_[i]].get();
             if (c->massq || c->mass) gr.mass = true;
-            const auto tl = tiles_of(*c, (int)i);
+            const auto tl = tiles_of(*c, (int)i, c->tiling), pl = tiles_of(*c, (int)i, c->phase);
             items.insert(items.end(), tl.begin(), tl.end());
+            phase.insert(phase.end(), pl.begin(), pl.end());
+            differ |= c->phase.tx != c->tiling.tx || c->phase.ty != c->tiling.ty || c->phase.zc != c->tiling.zc;
             work += c->geo.n;
         }
         items = xcd_permute(items);
+        gr.n = (unsigned)items.size();
+        gr.n_phase = 0;
+        if (differ) {
+            phase = xcd_permute(phase);
+            gr.n_phase = (unsigned)phase.size();
+            items.insert(items.end(), phase.begin(), phase.end());
+        }
         if (items.size() > gr.cap) {
             if (gr.d_work) B_HIP(hipFree(gr.d_work));
             gr.d_work = nullptr;
@@ -624,7 +655,6 @@ mcb_status Batch::rebuild() {
             B_HIP(hipMalloc(reinterpret_cast<void**>(&gr.d_work), cap * sizeof(WorkItem)));
             gr.cap = cap;
         }
-        gr.n = (unsigned)items.size();
         B_HIP(hipMemcpyAsync(gr.d_work, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, stream_));
         B_HIP(hipStreamSynchronize(stream_));   // items is a host temporary
         load.emplace_back(work + kGroupCells, k);
@@ -662,7 +692,8 @@ mcb_status Batch::launch_steps(int q, int n) {
         for (size_t i = 0; i < n_groups_ && e == hipSuccess; ++i) {
             const Group& gr = groups_[i];
             const hipStream_t s = fork && gr.lane ? lane_[gr.lane - 1] : stream_;
-            e = launch_phase_batch(d_views_[q], gr.d_work, gr.n, gr.t, storage_, s);
+            e = gr.n_phase ? launch_phase_batch(d_views_[q], gr.d_work + gr.n, gr.n_phase, gr.pt, storage_, s)
+                           : launch_phase_batch(d_views_[q], gr.d_work, gr.n, gr.t, storage_, s);
             if (e == hipSuccess && gr.sum.zc) e = launch_mass_sum(d_views_[q] + gr.first, gr.geo, gr.sum, s);
             if (e == hipSuccess && gr.mass) e = launch_mass_finish(d_views_[q] + gr.first, gr.cases, s);
             if (e == hipSuccess) e = launch_collide_batch(d_views_[q], gr.d_work, gr.n, gr.t, gr.mode, storage_, s);

@@ -31,6 +31,7 @@ struct CaseState {
     Tiling tiling{64, 8, 16};
     bool own_tiling = false;        // set by the library's caller
     bool alone = false;             // a context's only case
+    Tiling phase{64, 8, 16};        // tiles of the phase pass (phase_tiling16)
     Tiling sum{64, 8, 16};          // tiles of the sum of phi of stored 16-bit g (build_own_table)
     int cur = 0;                    // population buffer of the current state
     int parity_offset = 0;          // cur = batch parity ^ parity_offset
@@ -164,11 +165,11 @@ private:
     // Cases of one tile shape and collide mode: views [first, first + cases) of
     // the arrays, one work table, one lane.
     struct Group {
-        Tiling t{};
+        Tiling t{}, pt{};                // tiles of the collide and phase passes
         int mode = COLLIDE_STEP;
-        WorkItem* d_work = nullptr;
+        WorkItem* d_work = nullptr;      // [0, n) collide, [n, n + n_phase) phase where its tiles differ
         size_t cap = 0;
-        unsigned n = 0;
+        unsigned n = 0, n_phase = 0;
         unsigned first = 0, cases = 0;
         Tiling sum{};                    // zc > 0: its only case sums phi on tiles of its own (launch_mass_sum)
         Geo geo{};                       // of that case

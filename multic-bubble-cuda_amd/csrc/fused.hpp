@@ -76,6 +76,7 @@ struct CaseView {
     Phys phys;
     int zc;                 // z planes per collide workgroup
     int tx, ty;             // tile of the case's work items
+    int ptx, pty, pzc;      // tiles of its batch phase pass (phase_tiling16)
     int stx, sty, szc;      // tiles of the sum of phi (mass): the work items', or launch_mass_sum's own
     int mslot;              // parity of the case's state: delta slot the phase pass reads
     MassCell* mass;         // 16-bit storage only

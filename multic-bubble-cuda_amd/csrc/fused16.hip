@@ -221,8 +221,8 @@ constexpr int kFinishThreads = 256;
 __global__ __launch_bounds__(kFinishThreads) void k_mass_finish(const CaseView* __restrict__ cases) {
     const CaseView c = cases[blockIdx.x];
     const Geo& G = c.geo;
-    const unsigned n_tiles = (unsigned)((G.nx + c.tx - 1) / c.tx) * (unsigned)((G.ny + c.ty - 1) / c.ty) *
-                             (unsigned)((G.nz + c.zc - 1) / c.zc);
+    const unsigned n_tiles = (unsigned)((G.nx + c.ptx - 1) / c.ptx) * (unsigned)((G.ny + c.pty - 1) / c.pty) *
+                             (unsigned)((G.nz + c.pzc - 1) / c.pzc);
     if (c.mass && c.gm == GM_POPULATIONS) {   // stored 16-bit g: FP64 partials, fixed order
         const unsigned n_sums = (unsigned)((G.nx + c.stx - 1) / c.stx) * (unsigned)((G.ny + c.sty - 1) / c.sty) *
                                 (unsigned)((G.nz + c.szc - 1) / c.szc);

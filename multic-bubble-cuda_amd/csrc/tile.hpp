@@ -912,7 +912,7 @@ template <int TX, int TY>
 __device__ __forceinline__ void massq_partial(const CaseView& c, int x0, int y0, int z0, long long part) {
     const Geo& G = c.geo;
     const unsigned gx = (unsigned)(G.nx + TX - 1) / TX, gy = (unsigned)(G.ny + TY - 1) / TY;
-    const unsigned tile = ((unsigned)(z0 / c.zc) * gy + (unsigned)(y0 / TY)) * gx + (unsigned)(x0 / TX);
+    const unsigned tile = ((unsigned)(z0 / c.pzc) * gy + (unsigned)(y0 / TY)) * gx + (unsigned)(x0 / TX);
     const long long s = block_sum_q<TX * TY>(part);
     if (threadIdx.y == 0 && threadIdx.x == 0) reinterpret_cast<long long*>(c.partial)[tile] = s;
 }
@@ -1812,8 +1812,8 @@ __global__ __launch_bounds__(TX * TY) void k_phase_batch(const CaseView* __restr
     const CaseView c = cases[w.c];
     const Geo& G = c.geo;
     if (c.gm == GM_MOMENTS) {   // uniform per workgroup
-        if constexpr (S::kAnchored) phase_tile_ab<TX, TY>(c, w.x0, w.y0, w.z0, min(w.z0 + c.zc, G.nz));
-        else phase_tile_gm<TX, TY>(c, w.x0, w.y0, w.z0, min(w.z0 + c.zc, G.nz));
+        if constexpr (S::kAnchored) phase_tile_ab<TX, TY>(c, w.x0, w.y0, w.z0, min(w.z0 + c.pzc, G.nz));
+        else phase_tile_gm<TX, TY>(c, w.x0, w.y0, w.z0, min(w.z0 + c.pzc, G.nz));
         return;
     }
     // 16-bit phase populations carry the mass bookkeeping (a barrier inside).
@@ -1827,7 +1827,7 @@ __global__ __launch_bounds__(TX * TY) void k_phase_batch(const CaseView* __restr
                             valid ? (unsigned)(shift<1>(y, G.ny) * G.nx) : 0u};
     const PopPlanes<S> gp(c.gsrc, G);
     const Columns col(xs, PopRows(y, G, valid).v, gp);
-    const int ze = min(w.z0 + c.zc, G.nz);
+    const int ze = min(w.z0 + c.pzc, G.nz);
     double part = 0.0;
     float delta = 0.0f;
     if (mass) delta = (float)c.mass->delta[c.mslot];

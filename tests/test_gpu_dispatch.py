@@ -173,3 +173,26 @@ def test_mass_sum_of_stored_g_alone(gpu_lib, storage, nx, ny, nz):
         b.step(8)
         assert np.array_equal(b.read(cid, "phi"), lat.read("phi"))
         assert abs(float(lat.read("phi").sum(dtype=np.float64)) - float(phi0.sum(dtype=np.float64))) <= 1e-3
+
+
+@pytest.mark.parametrize("storage,nx,ny,nz", [(1, 64, 8, 33), (2, 65, 9, 20), (1, 130, 31, 17), (2, 64, 7, 24), (1, 256, 200, 130),
+                                              (2, 128, 64, 48)])
+def test_phase_tiles_of_16_bit_cases(gpu_lib, storage, nx, ny, nz):
+    """The phase pass of a large lattice alone on 8-row tiles with longer chunks (256x200x130), against 4 rows and a batch."""
+    mcb = gpu_lib
+    p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.6)
+    bubble = [(0.4 * nx, 0.5 * ny, 0.5 * nz, 0.3 * min(nx, ny, nz))]
+    got = []
+    for tiling in (None, (64, 4, 16)):
+        with mcb.Lattice(p) as lat, mcb.Batch(storage) as b:
+            cid = b.add(p, bubble, 3.0)
+            lat.init_bubbles(bubble, 3.0)
+            if tiling:
+                lat.set_tiling(*tiling)
+                b.set_tiling(cid, *tiling)
+            lat.step(6)
+            b.step(6)
+            got += [lat.read("phi"), lat.read("f"), b.read(cid, "phi"), b.read(cid, "f")]
+    for a, b in zip(got[:4], got[4:]):
+        assert np.array_equal(a, b)
+    assert np.array_equal(got[0], got[2])
