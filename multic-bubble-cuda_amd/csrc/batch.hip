@@ -81,10 +81,11 @@ Geo fused_geo(const mcb_params& p, bool pad_rows) {
 
 // Tiles of the 16-bit (phi, B) phase pass of a lattice alone that collides on
 // t. The pass stages a halo of one cell: 4-row tiles of 64 stage 1.55 cells for
-// each of theirs, 8 rows 1.29 (256^3: 37 against 28 LDS instructions a cell),
+// each of theirs, 8 rows 1.29 (256^3 FP16: 117 against 103 VALU and 37 against 34
+// LDS instructions a cell, 92 us a pass against 85),
 // while the collide pass wants the many small workgroups. Where 8 rows and
 // longer chunks leave three workgroups a CU: 100 steps and a read of 256^3 FP16
-// 41.0 ms against 42.2, 192^3 BF16 18.7 against 18.6; below that 4 rows keep more
+// 41.1 ms against 42.2, 192^3 BF16 18.7 against 18.6; below that 4 rows keep more
 // of the device busy (117x90x133 57 us per step against 59). The fixed-point
 // sums of phi do not depend on the tiles.
 static Tiling phase_tiling16(const mcb_params& p, const Tiling& t) {
