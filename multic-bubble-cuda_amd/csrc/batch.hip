@@ -26,6 +26,8 @@ constexpr long long kSplitCells = 8LL << 20;
 // cells (about 25 us).
 constexpr long long kGroupCells = 1LL << 20;
 
+bool same_tiling(const Tiling& a, const Tiling& b) { return a.tx == b.tx && a.ty == b.ty && a.zc == b.zc; }
+
 // Work items of a case (x fastest, then y, then z chunks), renumbered by
 // xcd_runs: each XCD takes runs of 8 consecutive tiles, so x-neighbouring
 // tiles meet in one L2 while the device works on one contiguous stretch of
@@ -480,15 +482,22 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
 }
 
 // The case's own work table (case index 0, used with the case's entry of the
-// view arrays as the base) and its partial-sum buffer, for its tiling.
+// view arrays as the base) and its partial-sum buffer, for its tiling: the
+// collide pass's items, then the phase pass's where its tiles differ.
 mcb_status Batch::build_own_table(CaseState* c) {
-    auto own = xcd_permute(tiles_of(*c, 0, c->tiling));
-    c->n_work = (unsigned)own.size();
     // Stored 16-bit g adds its FP64 sums tile by tile. In a context they
     // keep the tiles of a batch case, whatever the context steps on: a state
     // image continues with the same bits in either.
     c->sum = c->alone && c->mass && !c->own_tiling ? batch_tiling(c->p) : c->tiling;
     c->phase = c->alone && c->massq && !c->mass && !c->own_tiling ? phase_tiling16(c->p, c->tiling) : c->tiling;
+    auto own = xcd_permute(tiles_of(*c, 0, c->tiling));
+    c->n_work = (unsigned)own.size();
+    c->n_phase = 0;
+    if (!same_tiling(c->phase, c->tiling)) {
+        const auto phase = xcd_permute(tiles_of(*c, 0, c->phase));
+        c->n_phase = (unsigned)phase.size();
+        own.insert(own.end(), phase.begin(), phase.end());
+    }
     auto over = [](int n, int t) { return (size_t)((n + t - 1) / t); };
     auto count = [&](const Tiling& t) { return over(c->p.nx, t.tx) * over(c->p.ny, t.ty) * over(c->p.nz, t.zc); };
     const size_t sums = std::max(count(c->sum), count(c->phase));
@@ -625,8 +634,7 @@ mcb_status Batch::rebuild() {
         gr.mode = c0->mode;
         gr.mass = false;
         gr.sum = c0->sum;   // of its own: a case alone (a context) only
-        if (!c0->alone || !c0->mass || (c0->sum.tx == c0->tiling.tx && c0->sum.ty == c0->tiling.ty && c0->sum.zc == c0->tiling.zc))
-            gr.sum.zc = 0;
+        if (!c0->alone || !c0->mass || same_tiling(c0->sum, c0->tiling)) gr.sum.zc = 0;
         gr.geo = c0->geo;
         std::vector<WorkItem> items, phase;
         bool differ = false;
@@ -637,7 +645,7 @@ mcb_status Batch::rebuild() {
             const auto tl = tiles_of(*c, (int)i, c->tiling), pl = tiles_of(*c, (int)i, c->phase);
             items.insert(items.end(), tl.begin(), tl.end());
             phase.insert(phase.end(), pl.begin(), pl.end());
-            differ |= c->phase.tx != c->tiling.tx || c->phase.ty != c->tiling.ty || c->phase.zc != c->tiling.zc;
+            differ |= !same_tiling(c->phase, c->tiling);
             work += c->geo.n;
         }
         items = xcd_permute(items);
@@ -762,7 +770,9 @@ mcb_status Batch::macros(int id) {
     }
     // The case's own table indexes case 0 of a view array based at its slot.
     const CaseView* views = d_views_[parity_] + c->slot;
-    B_HIP(launch_phase_batch(views, c->d_work, c->n_work, c->tiling, storage_, stream_));
+    const bool own_phase = c->n_phase != 0;
+    B_HIP(launch_phase_batch(views, own_phase ? c->d_work + c->n_work : c->d_work, own_phase ? c->n_phase : c->n_work,
+                             c->phase, storage_, stream_));
     B_HIP(launch_collide_batch(views, c->d_work, c->n_work, c->tiling, COLLIDE_MACROS, storage_, stream_));
     c->phi_last = c->phi[c->cur];
     macro_id_ = id;

@@ -50,9 +50,11 @@ struct CaseState {
     std::vector<std::pair<void*, size_t>> allocs;   // device blocks and their sizes
     size_t bytes = 0;
     int slot = 0;                   // index in the batch's view arrays
-    WorkItem* d_work = nullptr;     // this case's tiles with case index 0 (its macro pass)
+    // This case's tiles with case index 0 (its macro pass): [0, n_work) collide,
+    // [n_work, n_work + n_phase) phase where its tiles differ.
+    WorkItem* d_work = nullptr;
     size_t work_cap = 0;
-    unsigned n_work = 0;
+    unsigned n_work = 0, n_phase = 0;
 
     // Buffers seen by the kernels at A/B parity q (q = cur before a step).
     CaseView view(int q) const;

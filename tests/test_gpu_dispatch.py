@@ -196,3 +196,27 @@ def test_phase_tiles_of_16_bit_cases(gpu_lib, storage, nx, ny, nz):
     for a, b in zip(got[:4], got[4:]):
         assert np.array_equal(a, b)
     assert np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("storage,nx,ny,nz", [(1, 256, 200, 130), (2, 200, 200, 150), (1, 64, 8, 33)])
+def test_macros_of_a_case_with_phase_tiles_of_its_own(gpu_lib, storage, nx, ny, nz):
+    """The macro pass runs its phase pass on the case's phase tiles, each cell once (200x200x150 and 256x200x130 have tiles
+    of their own, 64x8x33 has not): the fields, and the steps and mass corrections after it, are those of 64x4 tiles."""
+    mcb = gpu_lib
+    p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.6)
+    bubble = [(0.4 * nx, 0.5 * ny, 0.5 * nz, 0.3 * min(nx, ny, nz))]
+    got = []
+    for tiling in (None, (64, 4, 16)):
+        with mcb.Lattice(p) as lat:
+            if tiling:
+                lat.set_tiling(*tiling)
+            lat.init_bubbles(bubble, 3.0)
+            out = [lat.observables()]     # before the first step: phi from the initial populations
+            for steps in (1, 4, 3):
+                lat.step(steps)
+                out.append(lat.observables())
+            out.append({"f": lat.read("f")})
+            got.append(out)
+    for a, b in zip(*got):
+        for k in a:
+            assert np.array_equal(a[k], b[k]), (k, int(np.count_nonzero(a[k] != b[k])))
