@@ -330,8 +330,8 @@ mcb_status any_step(mcb_ctx* c, int nsteps) {
 // iteration to the next, so they are state too; fused FP32, f of the current
 // buffer and g as populations (with the phi the last step reported) or in
 // moment form (the state's phi and u; n is gradCalc of that phi, rebuilt on
-// loading where the context stores it).
-std::vector<StatePart> ctx_state_parts(mcb_ctx* c) {
+// loading where the context stores it). gm: the form of g.
+std::vector<StatePart> ctx_state_parts(mcb_ctx* c, int gm) {
     const size_t N = (size_t)c->geo.n, P = (size_t)c->geo.plane;
     if (c->path == MCB_PATH_STAGED) {
         std::vector<StatePart> parts{{"f", c->sf, 19, N, N, 4, false}, {"g", c->sg, 19, N, N, 4, false}};
@@ -349,7 +349,7 @@ std::vector<StatePart> ctx_state_parts(mcb_ctx* c) {
     // through the idle A/B buffers (pops_image_copy / pops_image_done).
     const int side = pops_relaid(c->geo) ? c->cur ^ 1 : c->cur;
     std::vector<StatePart> parts{{"f", c->f[side], 19, N, P, 4, false}};
-    if (c->gm == GM_POPULATIONS) {
+    if (gm == GM_POPULATIONS) {
         // With g as populations phi is what the last step reported (phiCalc
         // of the populations before that step's collision): not given back
         // by the state's populations, so kept for a read after loading.
@@ -1073,7 +1073,7 @@ mcb_status mcb_state_size(mcb_ctx* c, size_t* bytes) {
     if (st != MCB_OK) return st;
     if (!bytes) return fail(c, MCB_ERR_INVALID_ARG, "null size pointer");
     if (c->batch) return batch_status(c, c->batch->state_size(c->case_id, bytes));
-    *bytes = state_image_bytes(ctx_state_parts(c));
+    *bytes = state_image_bytes(ctx_state_parts(c, c->gm));
     return MCB_OK;
 }
 
@@ -1089,7 +1089,7 @@ mcb_status mcb_save_state(mcb_ctx* c, void* buf, size_t bytes) {
     h.steps = c->steps;
     const bool staged = c->path == MCB_PATH_FUSED && pops_relaid(c->geo);
     if (staged) MCB_HIP(c, pops_image_copy(c, true));
-    st = state_image_save(c->stream, h, ctx_state_parts(c), buf, bytes, &c->err);
+    st = state_image_save(c->stream, h, ctx_state_parts(c, c->gm), buf, bytes, &c->err);
     if (staged) MCB_HIP(c, pops_image_done(c));
     MCB_HIP(c, hipStreamSynchronize(c->stream));
     return st;
@@ -1103,7 +1103,7 @@ mcb_status mcb_load_state(mcb_ctx* c, const void* buf, size_t bytes) {
     if (!same_state_params(h.params, c->p) || h.path != c->path)
         return fail(c, MCB_ERR_INVALID_ARG, "state image of another lattice, parameter set or path");
     if (h.gm < GM_POPULATIONS || h.gm > GM_INITIAL || (h.gm != GM_POPULATIONS && c->p.tau_g != 1.0f) ||
-        (c->path == MCB_PATH_STAGED && h.gm != GM_POPULATIONS))
+        (c->path == MCB_PATH_STAGED && h.gm != GM_POPULATIONS) || (c->fm && h.gm == GM_POPULATIONS))
         return fail(c, MCB_ERR_INVALID_ARG, "state image with an invalid g form");
     if (!c->initialised) {
         // Any initial state gives the context its buffers (and, for 16 bits,
@@ -1114,6 +1114,8 @@ mcb_status mcb_load_state(mcb_ctx* c, const void* buf, size_t bytes) {
     if ((st = check_ready(c)) != MCB_OK) return st;
     if (c->batch) return batch_status(c, c->batch->load_state(c->case_id, buf, bytes));
     MCB_HIP(c, hipStreamSynchronize(c->stream));
+    // A refused image leaves the context as it was.
+    if ((st = state_image_check(buf, bytes, ctx_state_parts(c, h.gm), &c->err)) != MCB_OK) return st;
     if (c->path == MCB_PATH_FUSED) {
         if (h.gm == GM_POPULATIONS && c->gm != GM_POPULATIONS) {
             // As writing G: from here on g is kept as populations.
@@ -1124,7 +1126,7 @@ mcb_status mcb_load_state(mcb_ctx* c, const void* buf, size_t bytes) {
         c->gm = h.gm;
         c->ref_reset_f = -1;   // the image's face populations are w_l
     }
-    if ((st = state_image_load(c->stream, buf, bytes, ctx_state_parts(c), &c->err)) != MCB_OK) return st;
+    if ((st = state_image_load(c->stream, buf, bytes, ctx_state_parts(c, c->gm), &c->err)) != MCB_OK) return st;
     if (c->path == MCB_PATH_FUSED && pops_relaid(c->geo)) {
         MCB_HIP(c, pops_image_copy(c, false));
         MCB_HIP(c, pops_image_done(c));

@@ -127,7 +127,7 @@ CaseView CaseState::view(int q) const {
     v.phi = phi[q];
     v.phi_prev = phi[q ^ 1];
     v.mslot = q;
-    v.mass = mass;
+    v.mass = gm == GM_POPULATIONS ? mass : nullptr;
     v.massq = massq;
     v.partial = partial;
     // Moment form: only the parity of the initial state (cur = 0 before the
@@ -488,8 +488,9 @@ mcb_status Batch::build_own_table(CaseState* c) {
     // Stored 16-bit g adds its FP64 sums tile by tile. In a context they
     // keep the tiles of a batch case, whatever the context steps on: a state
     // image continues with the same bits in either.
-    c->sum = c->alone && c->mass && !c->own_tiling ? batch_tiling(c->p) : c->tiling;
-    c->phase = c->alone && c->massq && !c->mass && !c->own_tiling ? phase_tiling16(c->p, c->tiling) : c->tiling;
+    const bool holds_g = c->gm == GM_POPULATIONS, ruled = c->alone && !c->own_tiling && c->storage != MCB_STORE_FP32;
+    c->sum = ruled && holds_g ? batch_tiling(c->p) : c->tiling;
+    c->phase = ruled && !holds_g ? phase_tiling16(c->p, c->tiling) : c->tiling;
     auto own = xcd_permute(tiles_of(*c, 0, c->tiling));
     c->n_work = (unsigned)own.size();
     c->n_phase = 0;
@@ -634,7 +635,7 @@ mcb_status Batch::rebuild() {
         gr.mode = c0->mode;
         gr.mass = false;
         gr.sum = c0->sum;   // of its own: a case alone (a context) only
-        if (!c0->alone || !c0->mass || same_tiling(c0->sum, c0->tiling)) gr.sum.zc = 0;
+        if (c0->gm != GM_POPULATIONS || same_tiling(c0->sum, c0->tiling)) gr.sum.zc = 0;
         gr.geo = c0->geo;
         std::vector<WorkItem> items, phase;
         bool differ = false;
@@ -822,24 +823,34 @@ mcb_status Batch::read(int id, int field, float* host, size_t n) {
 
 mcb_status Batch::to_populations(CaseState* c) {
     B_HIP(hipStreamSynchronize(stream_));
+    // A case that went back to the moment form (load_state) still has these.
     const size_t pops = 19 * (size_t)c->geo.plane * pop_bytes(c->storage);
     for (int b = 0; b < 2; ++b) {
-        mcb_status st = dev_alloc(pops, &c->g[b]);
+        if (c->g[b]) continue;
+        void* q = nullptr;
+        mcb_status st = dev_alloc(pops, &q);
         if (st != MCB_OK) return st;
-        c->allocs.emplace_back(c->g[b], pops);
+        c->g[b] = q;
+        c->allocs.emplace_back(q, pops);
         c->bytes += pops;
     }
-    if (c->storage != MCB_STORE_FP32) {
+    if (c->storage != MCB_STORE_FP32 && !c->mass) {
         void* q = nullptr;
         mcb_status st = dev_alloc(sizeof(MassCell), &q);
         if (st != MCB_OK) return st;
         c->allocs.emplace_back(q, sizeof(MassCell));
         c->mass = static_cast<MassCell*>(q);
-        if ((st = build_own_table(c)) != MCB_OK) return st;   // partial sums
     }
-    c->gm = GM_POPULATIONS;
+    return set_form(c, GM_POPULATIONS);
+}
+
+// The form of g that the case's next step reads; its phase and sum tiles go
+// with it.
+mcb_status Batch::set_form(CaseState* c, int gm) {
+    const bool other = (gm == GM_POPULATIONS) != (c->gm == GM_POPULATIONS);
+    c->gm = gm;
     dirty_ = true;
-    return MCB_OK;
+    return other ? build_own_table(c) : MCB_OK;
 }
 
 // --------------------------------------------------------------- state
@@ -851,8 +862,9 @@ mcb_status Batch::to_populations(CaseState* c) {
 // give back); the 16-bit mass target and the correction pending for the next
 // phase pass. n is not part of an image: it is gradCalc of the state's phi,
 // rebuilt on loading. FP32 images have the parts of a single context's (same
-// form), so either resumes in the other.
-std::vector<StatePart> Batch::state_parts(CaseState* c, double* mass) {
+// form), so either resumes in the other. gm: the form of g, which alone decides
+// the parts (a case may hold buffers of the other form besides).
+std::vector<StatePart> Batch::state_parts(CaseState* c, int gm, double* mass) {
     const size_t N = (size_t)c->geo.n, P = (size_t)c->geo.plane;
     const unsigned eb = pop_bytes(c->storage);
     // Images keep populations in plain planes: other layouts pass through the
@@ -860,14 +872,14 @@ std::vector<StatePart> Batch::state_parts(CaseState* c, double* mass) {
     const int side = pops_relaid(c->geo) ? c->cur ^ 1 : c->cur;
     std::vector<StatePart> parts;
     parts.push_back({"f", c->f[side], 19, N, P, eb, false});
-    if (c->gm == GM_POPULATIONS) parts.push_back({"g", c->g[side], 19, N, P, eb, false});
+    if (gm == GM_POPULATIONS) parts.push_back({"g", c->g[side], 19, N, P, eb, false});
     parts.push_back({"phi", c->phi[c->cur ^ 1], 1, N, N, 4, false});
-    if (c->gm != GM_POPULATIONS) {
+    if (gm != GM_POPULATIONS) {
         static const char* const un[3] = {"u0", "u1", "u2"};
         for (int k = 0; k < 3; ++k)
             if (c->gmu[k]) parts.push_back({un[k], c->gmu[k], 1, N, N, c->storage == MCB_STORE_FP32 ? 4u : 2u, false});
     }
-    if (c->mass) parts.push_back({"mass", mass, 1, 2, 2, 8, true});
+    if (c->storage != MCB_STORE_FP32 && gm == GM_POPULATIONS) parts.push_back({"mass", mass, 1, 2, 2, 8, true});
     if (c->massq) parts.push_back({"massq", mass + 2, 1, 3, 3, 8, true});
     return parts;
 }
@@ -876,7 +888,7 @@ mcb_status Batch::state_size(int id, size_t* bytes) {
     CaseState* c = get(id);
     if (!c || !bytes) return fail(MCB_ERR_INVALID_ARG, "no such case or null size pointer");
     double m5[5];
-    *bytes = state_image_bytes(state_parts(c, m5));
+    *bytes = state_image_bytes(state_parts(c, c->gm, m5));
     return MCB_OK;
 }
 
@@ -886,7 +898,7 @@ mcb_status Batch::save_state(int id, void* buf, size_t bytes) {
     B_HIP(hipSetDevice(device_));
     B_HIP(hipStreamSynchronize(stream_));
     double m5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (c->mass) {
+    if (c->mass && c->gm == GM_POPULATIONS) {
         MassCell m;
         B_HIP(hipMemcpy(&m, c->mass, sizeof(m), hipMemcpyDeviceToHost));
         m5[0] = m.target;
@@ -905,7 +917,7 @@ mcb_status Batch::save_state(int id, void* buf, size_t bytes) {
     h.gm = c->gm;
     h.steps = c->steps;
     if (pops_relaid(c->geo)) B_HIP(stage_pops(c, true));
-    return state_image_save(stream_, h, state_parts(c, m5), buf, bytes, &err_);
+    return state_image_save(stream_, h, state_parts(c, c->gm, m5), buf, bytes, &err_);
 }
 
 // Populations in another layout around a state image: the current f (and g
@@ -934,17 +946,18 @@ mcb_status Batch::load_state(int id, const void* buf, size_t bytes) {
         return fail(MCB_ERR_INVALID_ARG, "state image with an invalid g form");
     B_HIP(hipSetDevice(device_));
     B_HIP(hipStreamSynchronize(stream_));
-    if (h.gm == GM_POPULATIONS && c->gm != GM_POPULATIONS && (st = to_populations(c)) != MCB_OK) return st;
+    // A refused image leaves the case as it was.
+    double m5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if ((st = state_image_check(buf, bytes, state_parts(c, h.gm, m5), &err_)) != MCB_OK) return st;
     // A case that holds populations and gets a moment-form image keeps its
     // g buffers (unused) and reads the moment fields again.
-    c->gm = h.gm;
-    double m5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if ((st = state_image_load(stream_, buf, bytes, state_parts(c, m5), &err_)) != MCB_OK) return st;
+    if ((st = h.gm == GM_POPULATIONS ? to_populations(c) : set_form(c, h.gm)) != MCB_OK) return st;
+    if ((st = state_image_load(stream_, buf, bytes, state_parts(c, h.gm, m5), &err_)) != MCB_OK) return st;
     if (pops_relaid(c->geo)) {
         B_HIP(stage_pops(c, false));
         B_HIP(hipStreamSynchronize(stream_));
     }
-    if (c->mass) {
+    if (c->mass && c->gm == GM_POPULATIONS) {
         MassCell m{m5[0], {0.0, 0.0}};
         m.delta[c->cur] = m5[1];
         B_HIP(hipMemcpy(c->mass, &m, sizeof(m), hipMemcpyHostToDevice));

@@ -139,11 +139,12 @@ private:
     // Keep g as populations from here on (arbitrary g has no moment form):
     // allocates the g buffers and, for 16 bits, the mass-drift state.
     mcb_status to_populations(CaseState* c);
+    mcb_status set_form(CaseState* c, int gm);
     // The arrays of a case's state image; mass receives / supplies (5 slots)
     // the 16-bit mass target and pending correction of stored g (0, 1) and
     // of the moment form (2: fixed-point target, 3: target recorded, 4:
     // pending correction).
-    std::vector<StatePart> state_parts(CaseState* c, double* mass);
+    std::vector<StatePart> state_parts(CaseState* c, int gm, double* mass);
     hipError_t stage_pops(CaseState* c, bool to_image);
     // One set of macro fields per batch, sized for its largest case; it holds
     // the observables of the case of the most recent macros() call.

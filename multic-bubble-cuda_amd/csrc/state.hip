@@ -76,8 +76,7 @@ mcb_status state_image_header(const void* buf, size_t bytes, StateHeader* h, std
     return MCB_OK;
 }
 
-mcb_status state_image_load(hipStream_t s, const void* buf, size_t bytes, const std::vector<StatePart>& parts,
-                            std::string* err) {
+mcb_status state_image_check(const void* buf, size_t bytes, const std::vector<StatePart>& parts, std::string* err) {
     StateHeader h;
     mcb_status st = state_image_header(buf, bytes, &h, err);
     if (st != MCB_OK) return st;
@@ -85,7 +84,6 @@ mcb_status state_image_load(hipStream_t s, const void* buf, size_t bytes, const 
         return bad(err, "state image does not match this lattice's state layout");
     const char* in = static_cast<const char*>(buf);
     size_t off = sizeof(StateHeader);
-    // Check every part before copying any.
     for (const StatePart& p : parts) {
         StatePartHeader ph;
         std::memcpy(&ph, in + off, sizeof(ph));
@@ -94,7 +92,16 @@ mcb_status state_image_load(hipStream_t s, const void* buf, size_t bytes, const 
             return bad(err, std::string("state image part mismatch at '") + p.name + "'");
         off += sizeof(ph) + part_data_bytes(p);
     }
-    off = sizeof(StateHeader);
+    return MCB_OK;
+}
+
+mcb_status state_image_load(hipStream_t s, const void* buf, size_t bytes, const std::vector<StatePart>& parts,
+                            std::string* err) {
+    // Every part is checked before any is copied.
+    const mcb_status st = state_image_check(buf, bytes, parts, err);
+    if (st != MCB_OK) return st;
+    const char* in = static_cast<const char*>(buf);
+    size_t off = sizeof(StateHeader);
     for (const StatePart& p : parts) {
         off += sizeof(StatePartHeader);
         const size_t w = p.row_elems * p.elem_bytes;

@@ -56,8 +56,11 @@ mcb_status state_image_save(hipStream_t s, const StateHeader& info, const std::v
 // Checks the header of an image (magic, version, size) and returns it.
 mcb_status state_image_header(const void* buf, size_t bytes, StateHeader* h, std::string* err);
 
-// Copies the image's parts into parts, which must match the image's part
-// list (names, shapes, element sizes) in order.
+// Whether the image's part list is parts (names, shapes, element sizes, in
+// order); their pointers are not used.
+mcb_status state_image_check(const void* buf, size_t bytes, const std::vector<StatePart>& parts, std::string* err);
+
+// Copies the image's parts into parts, after that check.
 mcb_status state_image_load(hipStream_t s, const void* buf, size_t bytes, const std::vector<StatePart>& parts,
                             std::string* err);
 

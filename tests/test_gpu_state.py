@@ -7,6 +7,8 @@ The reference has no restart (it writes phi snapshots only, src/main.cu:184-189)
 the property pinned here is the definition of a checkpoint: save, load,
 continue == continue.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -295,3 +297,81 @@ def test_state_images_of_other_cases_are_refused(gpu_lib):
         with pytest.raises(mcb.McbError):
             b.add_state(image)                    # FP32 image into an FP16 batch
     a.close()
+
+
+def with_form(mcb, image, gm):
+    """The image with another g form in its header (after magic, version, part count, size, parameters and path)."""
+    at = 8 + 4 + 4 + 8 + ctypes.sizeof(mcb.Params) + 4
+    return image[:at] + gm.to_bytes(4, "little") + image[at + 4:]
+
+
+@pytest.mark.parametrize("shape", [SHAPE, (256, 200, 130)])     # the second has phase tiles of its own in 16 bits
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("where", ["context", "batch"])
+def test_moment_form_image_into_a_case_with_written_g(gpu_lib, where, storage, shape):
+    """A case that keeps g as populations (it was written) takes an image of the moment form and continues like the run
+    that never stopped; g can be written again."""
+    mcb = gpu_lib
+    p = params(mcb, storage, 1.0, shape=shape)
+    with mcb.Lattice(p) as a:
+        a.init_bubbles(BUB, 3.0)
+        a.step(4)
+        image = a.save_state()
+        if where == "context":
+            b = mcb.Lattice(p)
+            b.init_bubbles(BUB[:1], 3.0)
+            b.step(3)
+            b.write("g", b.read("g"))
+            b.step(2)
+            b.load_state(image)
+            assert b.save_state() == image
+            step, read, write = b.step, b.read, b.write
+        else:
+            b = mcb.Batch(storage)
+            cid = b.add(p, BUB[:1], 3.0)
+            b.step(3)
+            b.write(cid, "g", b.read(cid, "g"))
+            b.step(2)
+            b.load_state(cid, image)
+            assert b.save_state(cid) == image
+            step, read, write = b.step, lambda k: b.read(cid, k), lambda k, v: b.write(cid, k, v)
+        a.step(5)
+        step(5)
+        for k in ("phi", "f", "g"):
+            assert np.array_equal(a.read(k), read(k)), (k, "after the image")
+        g = a.read("g")
+        a.write("g", g)
+        write("g", g)
+        a.step(3)
+        step(3)
+        for k in ("phi", "f", "g"):
+            assert np.array_equal(a.read(k), read(k)), (k, "after writing g again")
+        b.close()
+
+
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("where", ["context", "batch"])
+def test_refused_image_leaves_the_case_as_it_was(gpu_lib, where, storage):
+    mcb = gpu_lib
+    p = params(mcb, storage, 1.0)
+    with mcb.Lattice(p) as a, mcb.Batch(storage) as b:
+        a.init_bubbles(BUB, 3.0)
+        a.step(4)
+        cid = b.add_state(a.save_state())
+        image = with_form(mcb, a.save_state(), 0)          # says populations, holds the moment form
+        with pytest.raises(mcb.McbError):
+            a.load_state(image) if where == "context" else b.load_state(cid, image)
+        a.step(5)
+        b.step(5)
+        for k in ("phi", "f", "g"):
+            assert np.array_equal(a.read(k), b.read(cid, k)), k
+
+
+def test_f_moments_image_that_says_populations_is_refused(gpu_lib):
+    mcb = gpu_lib
+    p = mcb.make_params(*SHAPE, tau_f=0.6, f_form=mcb.F_MOMENTS, path=mcb.PATH_FUSED)
+    with mcb.Lattice(p) as a:
+        a.init_bubbles(BUB, 3.0)
+        a.step(2)
+        with pytest.raises(mcb.McbError):
+            a.load_state(with_form(mcb, a.save_state(), 0))
