@@ -61,15 +61,31 @@ static bool keeps_row_tile16(int nx) {
     return tiling_supported16(Tiling{nx, 4, 1}) && nx % 32 != 0 && 16 / waves * waves >= 11;
 }
 
+// Rows of a lattice alone that are worth padding to whole lines (us per step,
+// plain against padded). Above 64 cells: FP32 65x200x150 157 against 132,
+// 65x256x256 388 against 261, 200x256x256 815 against 596; FP16 84x256x256 288
+// against 204, 200x256x256 583 against 401. Shorter rows fill few lines, and
+// what the padding adds is read and written with them: FP32 tau_g 0.8
+// 20x256x256 173 against 267, 50x256x256 260 against 402, FP16 tau_g 0.8
+// 33x256x256 234 against 314; only rows just below 32 gain (FP32 30x256x256 147
+// against 121). 16 bits with stored g, whose traffic is mostly populations, gain
+// up to a sixth of padding (144 of 160: 413 against 406, 200x200x150 624
+// against 581; 65x200x150 224 against 235, 98x200x150 259 against 273).
+static bool pads_rows(const mcb_params& p) {
+    const int pitch = (p.nx + 31) / 32 * 32;
+    if (p.nx <= 64) return p.nx < 32 && pitch - p.nx <= 2;
+    if (p.storage == MCB_STORE_FP32) return true;
+    return !keeps_row_tile16(p.nx) && (p.tau_g == 1.0f || 5 * pitch <= 6 * p.nx);
+}
+
 Geo fused_geo(const mcb_params& p, bool pad_rows) {
     Geo g{p.nx, p.ny, p.nz, p.nx * p.ny, (long long)p.nx * p.ny * p.nz, 0, 0, p.nx, p.nx * p.ny};
     g.plane = plane_stride_cells(g.n);
     if (p.f_form != MCB_F_POPULATIONS) return g;
     const bool fp32 = p.storage == MCB_STORE_FP32;
     const int group = fp32 ? 64 : 1;
-    if (p.nx < 16 || (!fp32 && keeps_row_tile16(p.nx))) pad_rows = false;   // at most twice the memory
     for (const int pitch : {(p.nx + 31) / 32 * 32, p.nx}) {
-        if (pitch != p.nx && !pad_rows) continue;
+        if (pitch != p.nx && !(pad_rows && pads_rows(p))) continue;
         const long long zp = ((long long)pitch * p.ny + group - 1) / group * group, plane = plane_stride_cells(zp * p.nz);
         if (plane * 19 * pop_bytes(p.storage) > 0xFFFFFFFFLL) continue;
         g.blocked = fp32;
@@ -221,6 +237,10 @@ Tiling choose_tiling_single(const mcb_params& p) {
     const int pad64 = (p.nx + 63) / 64 * 64, pad32 = (p.nx + 31) / 32 * 32;
     const bool moments = p.tau_g == 1.0f;
     bool row = false;
+    // One 32-wide tile for rows that two of 16 would half fill (plain rows, 16x16
+    // against this: FP32 28x256x256 125 against 93, tau_g 0.8 252 against 141;
+    // FP16 24x256x256 86 against 61).
+    if (p.nx > 16 && p.nx < 32 && p.f_form == MCB_F_POPULATIONS) t = Tiling{32, 8, t.zc};
     if (p.nx > 32 && p.f_form == MCB_F_POPULATIONS) {
         row = !fp32 && keeps_row_tile16(p.nx);
         // 32-wide tiles where 64-wide ones would pad more lanes: FP32 80x230x160

@@ -72,8 +72,8 @@ Phys host_phys(const mcb_params& p);
 mcb_status host_validate(const mcb_params* p, std::string* why);
 
 // Geometry of a lattice on the fused kernels: populations (not f as moments)
-// in blocks (FP32) and, if asked for, in padded rows, as far as they fit the
-// kernels' 32-bit buffers. 16-bit rows that one collide tile spans stay
+// in blocks (FP32) and, if asked for and worth it (pads_rows), in padded rows,
+// as far as they fit the kernels' 32-bit buffers. 16-bit rows that one collide tile spans stay
 // unpadded: the tile is one contiguous piece of memory (FP16, rows padded
 // against not: 176^3 187 against 154 us per step, 144^3 134 against 125).
 Geo fused_geo(const mcb_params& p, bool pad_rows);

@@ -19,8 +19,8 @@ namespace mcb {
 //   blocks (blocked = 1): element (i >> 6)*19*64 + l*64 + (i & 63), groups of
 //     64 consecutive cells holding their 19 links side by side, zpop =
 //     pitch*ny rounded up to 64.
-// pitch is nx, or nx rounded up to 32 cells (128 or 64 bytes) where the case
-// can afford it (fused_geo): otherwise the rows of a wave start inside cache
+// pitch is nx, or nx rounded up to 32 cells (128 or 64 bytes) in contexts whose
+// rows are long enough (pads_rows): otherwise the rows of a wave start inside cache
 // lines, and each store leaves two partial lines to be merged in memory (FP32
 // 250^3: 767 us per collide against 553 padded, 150x105x77 66 against 59; FP16
 // 250^3: 639 us per step against 424, 150x105x77 72 against 56, 117x90x133 62

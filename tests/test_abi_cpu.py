@@ -263,3 +263,16 @@ def test_state_calls_without_a_device_report_status():
     assert mcb.lib().mcb_state_size(None, ctypes.byref(n)) == mcb.ERR_INVALID_ARG
     assert mcb.lib().mcb_load_state(None, None, 0) == mcb.ERR_INVALID_ARG
     assert mcb.lib().mcb_batch_add_state(None, None, 0, None) == mcb.ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("kw", [dict(tau_g=0.8), dict(tau_g=1.0, normals=1), dict(tau_g=0.8, storage=1),
+                                dict(tau_g=1.0, storage=2)])
+def test_short_rows_are_not_padded(kw):
+    """A context of short rows takes what the same cells take in rows of 64, one of longer rows at most half as much again."""
+    def footprint(nx, ny):
+        return mcb.lib().mcb_footprint_bytes(ctypes.byref(mcb.make_params(nx, ny, 256, **kw)))
+
+    for nx in (16, 20, 28, 33, 40, 50, 63):
+        assert footprint(nx, 256) <= 1.01 * footprint(64, 4 * nx), nx
+    for nx in (65, 100, 150):
+        assert footprint(nx, 256) <= 1.5 * footprint(64, 4 * nx), nx

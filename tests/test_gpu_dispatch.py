@@ -220,3 +220,22 @@ def test_macros_of_a_case_with_phase_tiles_of_its_own(gpu_lib, storage, nx, ny, 
     for a, b in zip(*got):
         for k in a:
             assert np.array_equal(a[k], b[k]), (k, int(np.count_nonzero(a[k] != b[k])))
+
+
+@pytest.mark.parametrize("nx", [15, 17, 29, 30, 34, 63, 64, 66, 97, 128])
+@pytest.mark.parametrize("storage,tau_g", [(0, 1.0), (0, 0.8), (1, 0.8), (2, 1.0)])
+def test_rows_around_the_padding_rule(gpu_lib, storage, tau_g, nx):
+    """Contexts with padded rows and with plain ones against a batch case, whose rows are plain, and its own tiles."""
+    mcb = gpu_lib
+    p = mcb.make_params(nx, 11, 19, storage=storage, tau_f=0.65, tau_g=tau_g)
+    bubble = [(0.4 * nx, 5.0, 9.0, 3.3)]
+    with mcb.Lattice(p) as lat, mcb.Batch(storage) as b:
+        lat.init_bubbles(bubble, 3.0)
+        cid = b.add(p, bubble, 3.0)
+        lat.step(7)
+        b.step(7)
+        for k in ("phi", "f", "g"):
+            assert np.array_equal(lat.read(k), b.read(cid, k)), k
+        got, want = lat.observables(), b.observables(cid)
+        for k in FIELDS:
+            assert np.array_equal(got[k], want[k]), k
