@@ -156,25 +156,58 @@ bool ctx_recomputes_n(const mcb_params& p) {
 }
 
 size_t footprint(const mcb_params& p, int path) {
+    // Populations take P elements a link, fields S.
+    const size_t S = (size_t)plane_stride_cells((long long)p.nx * p.ny * p.nz);
+    const size_t P = path == MCB_PATH_FUSED ? (size_t)fused_geo(p, true).plane : S;
     // 16-bit: the case plus the batch's ten macro fields.
-    const long long P = path == MCB_PATH_FUSED ? fused_geo(p, true).plane : plane_stride_cells((long long)p.nx * p.ny * p.nz);
-    if (p.storage != MCB_STORE_FP32) return case_bytes(p, true) + 10 * (size_t)P * 4;
+    if (p.storage != MCB_STORE_FP32) return case_bytes(p, true) + 10 * S * 4;
     size_t floats = 0;
     if (path == MCB_PATH_FUSED && p.f_form == MCB_F_MOMENTS)   // 13 moments A/B (u among them), phi twice, n
-        floats = 2 * 13 * (size_t)P + (ctx_recomputes_n(p) ? 12 : 15) * (size_t)P;
+        floats = 2 * 13 * P + (ctx_recomputes_n(p) ? 12 : 15) * S;
     else if (path == MCB_PATH_FUSED && p.tau_g == 1.0f)   // g in moment form: phi twice, u, and n unless recomputed
-        floats = 2 * 19 * (size_t)P + (ctx_recomputes_n(p) ? 15 : 18) * (size_t)P;
-    else if (path == MCB_PATH_FUSED) floats = 4 * 19 * (size_t)P + 11 * (size_t)P;
-    else floats = 3 * 19 * (size_t)P + 19 * (size_t)P;
+        floats = 2 * 19 * P + (ctx_recomputes_n(p) ? 15 : 18) * S;
+    else if (path == MCB_PATH_FUSED) floats = 4 * 19 * P + 11 * S;
+    else floats = 3 * 19 * P + 19 * S;
     return floats * sizeof(float) + (2 * kReduceBlocks + 2) * sizeof(double);
 }
 
 mcb_status alloc(mcb_ctx* c, float** out, size_t floats) {
     void* ptr = nullptr;
     hipError_t e = hipMalloc(&ptr, floats * sizeof(float));
-    if (e != hipSuccess) return hip_fail(c, e, "hipMalloc");
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return hip_fail(c, e, "hipMalloc");
+    }
     c->allocs.push_back(ptr);
     *out = static_cast<float*>(ptr);
+    return MCB_OK;
+}
+
+// The device buffers of a fused FP32 context, for its geometry. At tau_g = 1 g
+// is kept in moment form: phi (two buffers), u and n (or n recomputed by the
+// phase pass) instead of two sets of 19 planes.
+mcb_status fused_buffers(mcb_ctx* c) {
+    const bool moments = c->p.tau_g == 1.0f;
+    const size_t P = (size_t)c->geo.plane, S = (size_t)plane_stride_cells(c->geo.n);
+    mcb_status st;
+    for (int b = 0; b < 2; ++b) {
+        if ((st = alloc(c, &c->f[b], (c->fm ? kFm : 19) * P)) != MCB_OK) return st;
+        if (!moments && (st = alloc(c, &c->g[b], 19 * P)) != MCB_OK) return st;
+    }
+    float** scal[] = {&c->phi, &c->rho, &c->ux, &c->uy, &c->uz, &c->ffx, &c->ffy, &c->ffz,
+                      &c->normx, &c->normy, &c->normz};
+    for (auto* q : scal)
+        if ((st = alloc(c, q, S)) != MCB_OK) return st;
+    if (!moments) return MCB_OK;
+    c->gm = GM_INITIAL;
+    c->phis[0] = c->phi;
+    float** gmf[] = {&c->phis[1], &c->gmu[0], &c->gmu[1], &c->gmu[2]};
+    for (auto* q : gmf)   // with f in moment form u is among its planes
+        if ((q == &c->phis[1] || !c->fm) && (st = alloc(c, q, S)) != MCB_OK) return st;
+    // n is stored beside u unless the phase pass recomputes it.
+    if (!ctx_recomputes_n(c->p))
+        for (int k = 0; k < 3; ++k)
+            if ((st = alloc(c, &c->gmn[k], S)) != MCB_OK) return st;
     return MCB_OK;
 }
 
@@ -223,7 +256,7 @@ void fused_init_target(mcb_ctx* c) {
 // w_l phi0(y + c_l) in pull form or nothing (initDist is implied by
 // GM_INITIAL) in moment form; the macro fields start at zero.
 hipError_t fused_init_state(mcb_ctx* c) {
-    const size_t pbytes = (size_t)c->geo.plane * sizeof(float);
+    const size_t pbytes = (size_t)c->geo.n * sizeof(float);
     float* zero[] = {c->rho, c->ux, c->uy, c->uz, c->ffx, c->ffy, c->ffz, c->normx, c->normy, c->normz};
     for (float* q : zero) {
         hipError_t e = hipMemsetAsync(q, 0, pbytes, c->stream);
@@ -470,35 +503,23 @@ mcb_status mcb_create(const mcb_params* p, void* stream, mcb_ctx** out) {
     for (auto& e : c->ev)
         if (hipEventCreate(&e) != hipSuccess) return bail(MCB_ERR_HIP);
 
-    const long long n = c->geo.n, P = c->geo.plane;
+    const long long n = c->geo.n;
     if (p->storage != MCB_STORE_FP32) {
         c->batch.reset(new (std::nothrow) Batch(c->device, c->stream));
         if (!c->batch) return bail(MCB_ERR_OUT_OF_MEMORY);
         c->tiling = choose_tiling_single(*p);
     } else if (path == MCB_PATH_FUSED) {
-        // At tau_g = 1 g is kept in moment form: phi (two buffers), u and n
-        // (or n recomputed by the phase pass) instead of two sets of 19 planes.
-        const bool moments = p->tau_g == 1.0f;
         c->fm = p->f_form == MCB_F_MOMENTS;
-        for (int b = 0; b < 2; ++b) {
-            if ((st = alloc(c, &c->f[b], (c->fm ? kFm : 19) * (size_t)P)) != MCB_OK) return bail(st);
-            if (!moments && (st = alloc(c, &c->g[b], 19 * (size_t)P)) != MCB_OK) return bail(st);
+        st = fused_buffers(c);
+        if (st == MCB_ERR_OUT_OF_MEMORY && c->geo.pitch != p->nx) {
+            // Plain rows, which take less, where padded ones do not fit.
+            for (void* q : c->allocs) (void)hipFree(q);
+            c->allocs.clear();
+            c->err.clear();
+            c->geo = fused_geo(*p, false);
+            st = fused_buffers(c);
         }
-        float** scal[] = {&c->phi, &c->rho, &c->ux, &c->uy, &c->uz, &c->ffx, &c->ffy, &c->ffz,
-                          &c->normx, &c->normy, &c->normz};
-        for (auto* q : scal)
-            if ((st = alloc(c, q, (size_t)P)) != MCB_OK) return bail(st);
-        if (moments) {
-            c->gm = GM_INITIAL;
-            c->phis[0] = c->phi;
-            float** gmf[] = {&c->phis[1], &c->gmu[0], &c->gmu[1], &c->gmu[2]};
-            for (auto* q : gmf)   // with f in moment form u is among its planes
-                if ((q == &c->phis[1] || !c->fm) && (st = alloc(c, q, (size_t)P)) != MCB_OK) return bail(st);
-            // n is stored beside u unless the phase pass recomputes it.
-            if (!ctx_recomputes_n(*p))
-                for (int k = 0; k < 3; ++k)
-                    if ((st = alloc(c, &c->gmn[k], (size_t)P)) != MCB_OK) return bail(st);
-        }
+        if (st != MCB_OK) return bail(st);
         if (p->bc_mode == MCB_BC_REFERENCE) {
             // Face cells never collide: their f*_l stay w_l in both buffers
             // (fgBoundary's rho(e) w_l with the face rho of 1) and their u and
@@ -507,8 +528,8 @@ mcb_status mcb_create(const mcb_params* p, void* stream, mcb_ctx** out) {
                 if (launch_init_pull(c->phi, c->f[b], nullptr, c->geo, c->phys, c->stream) != hipSuccess)
                     return bail(MCB_ERR_HIP);
             for (int k = 0; k < 3; ++k)
-                if (hipMemsetAsync(c->gmu[k], 0, (size_t)P * sizeof(float), c->stream) != hipSuccess ||
-                    (c->gmn[k] && hipMemsetAsync(c->gmn[k], 0, (size_t)P * sizeof(float), c->stream) != hipSuccess))
+                if (hipMemsetAsync(c->gmu[k], 0, (size_t)n * sizeof(float), c->stream) != hipSuccess ||
+                    (c->gmn[k] && hipMemsetAsync(c->gmn[k], 0, (size_t)n * sizeof(float), c->stream) != hipSuccess))
                     return bail(MCB_ERR_HIP);
             if (hipStreamSynchronize(c->stream) != hipSuccess) return bail(MCB_ERR_HIP);
         }

@@ -116,10 +116,11 @@ static Tiling phase_tiling16(const mcb_params& p, const Tiling& t) {
 
 size_t case_bytes(const mcb_params& p, bool pad_rows) {
     const size_t P = (size_t)fused_geo(p, pad_rows).plane;
+    const size_t S = (size_t)plane_stride_cells((long long)p.nx * p.ny * p.nz);
     const bool moments = p.tau_g == 1.0f;
     size_t b = (moments ? 2 : 4) * 19 * P * pop_bytes(p.storage);          // f (and g) A/B
-    b += (moments || p.storage != MCB_STORE_FP32 ? 2 : 1) * P * sizeof(float);   // phi
-    if (moments) b += p.storage == MCB_STORE_FP32 ? 6 * P * sizeof(float) : 3 * P * 2;   // u, n (FP32) or B (FP16)
+    b += (moments || p.storage != MCB_STORE_FP32 ? 2 : 1) * S * sizeof(float);   // phi
+    if (moments) b += p.storage == MCB_STORE_FP32 ? 6 * S * sizeof(float) : 3 * S * 2;   // u, n (FP32) or B (FP16)
     return b;
 }
 
@@ -372,13 +373,13 @@ mcb_status Batch::ensure_partial() {
     return MCB_OK;
 }
 
-mcb_status Batch::add(const mcb_params& p, const float* phi_host, int* id, bool pad_rows) {
+mcb_status Batch::add(const mcb_params& p, const float* phi_host, int* id, bool alone) {
     if (!phi_host) return fail(MCB_ERR_INVALID_ARG, "null argument");
-    return add_impl(p, phi_host, nullptr, id, pad_rows);
+    return add_impl(p, phi_host, nullptr, id, alone);
 }
 
 mcb_status Batch::add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, int n, float width, int* id,
-                              bool pad_rows) {
+                              bool alone) {
     if (!bubbles || n < 1 || n > kMaxBubbleSet || !(width > 0.0f) || !std::isfinite(width))
         return fail(MCB_ERR_INVALID_ARG, "invalid bubble set");
     BubbleSet s{};
@@ -390,10 +391,18 @@ mcb_status Batch::add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, in
     }
     s.n = n;
     s.width = width;
-    return add_impl(p, nullptr, &s, id, pad_rows);
+    return add_impl(p, nullptr, &s, id, alone);
 }
 
-mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id,
+mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id, bool alone) {
+    mcb_status st = add_case(p, phi_host, bubbles, id, alone, alone);
+    // Plain rows, which take less, where padded ones do not fit.
+    if (st == MCB_ERR_OUT_OF_MEMORY && alone && fused_geo(p, true).pitch != p.nx)
+        st = add_case(p, phi_host, bubbles, id, alone, false);
+    return st;
+}
+
+mcb_status Batch::add_case(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id, bool alone,
                            bool pad_rows) {
     if (!id) return fail(MCB_ERR_INVALID_ARG, "null argument");
     std::string why;
@@ -415,7 +424,7 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
     c->storage = p.storage;
     c->mode = p.tau_g == 1.0f ? COLLIDE_STEP : COLLIDE_STEP_BGK;
     c->tiling = t;
-    c->alone = pad_rows;
+    c->alone = alone;
     // FP32 populations in 64-cell blocks (16-bit ones stay in planes: with
     // blocks the FP16 batch ran 3% slower).
     c->geo = geo;
@@ -428,7 +437,7 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
         return MCB_OK;
     };
     mcb_status st;
-    const size_t pops = 19 * (size_t)P * pop_bytes(p.storage);
+    const size_t pops = 19 * (size_t)P * pop_bytes(p.storage), S = (size_t)plane_stride_cells(geo.n);
     // At tau_g = 1 g is kept in moment form instead of two sets of 19
     // planes, for every storage form.
     const bool moments = c->mode == COLLIDE_STEP;
@@ -437,11 +446,11 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
         if (!moments && (st = alloc(pops, &c->g[b])) != MCB_OK) return st;
     }
     void* q = nullptr;
-    if ((st = alloc((size_t)P * sizeof(float), &q)) != MCB_OK) return st;
+    if ((st = alloc(S * sizeof(float), &q)) != MCB_OK) return st;
     c->phi[0] = c->phi[1] = static_cast<float*>(q);
     if (moments || p.storage != MCB_STORE_FP32) {
         // phi[1] holds the state's phi (moment form) or the g anchor (16 bits).
-        if ((st = alloc((size_t)P * sizeof(float), &q)) != MCB_OK) return st;
+        if ((st = alloc(S * sizeof(float), &q)) != MCB_OK) return st;
         c->phi[1] = static_cast<float*>(q);
     }
     if (moments) {
@@ -451,7 +460,7 @@ mcb_status Batch::add_impl(const mcb_params& p, const float* phi_host, const Bub
         // (phase_tile_ab).
         const bool fp32 = p.storage == MCB_STORE_FP32;
         for (int k = 0; k < (fp32 ? 6 : 3); ++k) {
-            if ((st = alloc((size_t)P * (fp32 ? sizeof(float) : 2), &q)) != MCB_OK) return st;
+            if ((st = alloc(S * (fp32 ? sizeof(float) : 2), &q)) != MCB_OK) return st;
             (k < 3 ? c->gmu[k] : c->gmn[k - 3]) = static_cast<float*>(q);
         }
         if (!fp32) {
@@ -566,7 +575,7 @@ mcb_status Batch::set_mass_target(CaseState* c, double target) {
 
 mcb_status Batch::ensure_macro_scratch() {
     size_t need = 0;
-    for (auto& kv : cases_) need = std::max(need, (size_t)kv.second->geo.plane);
+    for (auto& kv : cases_) need = std::max(need, (size_t)plane_stride_cells(kv.second->geo.n));
     if (need <= macro_plane_) return MCB_OK;
     for (void* q : macro_bufs_) B_HIP(hipFree(q));
     macro_bufs_.clear();

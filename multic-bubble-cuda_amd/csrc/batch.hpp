@@ -92,12 +92,12 @@ public:
     // Allocate a case and set its initial state from phi (host, nx*ny*nz
     // floats), or from bubbles on the device (serving; bubble_phi_cell, the
     // bits of the host initialisation).
-    // pad_rows: populations in line-aligned rows (Geo::pitch), faster where nx
-    // is not a multiple of a line, for case_bytes(p, true) instead of
-    // case_bytes(p) of device memory.
-    mcb_status add(const mcb_params& p, const float* phi_host, int* id, bool pad_rows = false);
+    // alone: a context's only case, on the tiles and rows of a lattice that has
+    // the device to itself; case_bytes(p, true) of device memory where its rows
+    // are padded (Geo::pitch), case_bytes(p) otherwise and where that does not fit.
+    mcb_status add(const mcb_params& p, const float* phi_host, int* id, bool alone = false);
     mcb_status add_bubbles(const mcb_params& p, const mcb_bubble* bubbles, int n, float width, int* id,
-                           bool pad_rows = false);
+                           bool alone = false);
     mcb_status remove(int id);
     mcb_status step(int nsteps);
     mcb_status macros(int id);
@@ -127,7 +127,9 @@ public:
 
 private:
     mcb_status fail(mcb_status s, const std::string& m);
-    mcb_status add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id, bool pad_rows);
+    mcb_status add_impl(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id, bool alone);
+    mcb_status add_case(const mcb_params& p, const float* phi_host, const BubbleSet* bubbles, int* id, bool alone,
+                        bool pad_rows);
     mcb_status dev_alloc(size_t bytes, void** out);
     void dev_release(void* ptr, size_t bytes);
     mcb_status build_own_table(CaseState* c);
