@@ -202,15 +202,19 @@ Tiling choose_tiling(const mcb_params& p) {
 }
 
 Tiling batch_tiling(const mcb_params& p) {
-    // FP32, measured on batches of equal cubes (k MLUPS): 64x8 tiles with
-    // 8-plane chunks where they pad rows by less than half a tile (64: 23.3,
-    // 128: 23.5), 32x8 where they would (32: 23.2 against 16.0, 96: 21.8
-    // against 20.3), whole rows of 48 (22.8 against 20.4). The shapes of a
-    // batch run side by side (launch_steps).
+    // FP32, batches of equal cubes (k MLUPS, tau_g 1 and 0.8), all in 8-plane
+    // chunks: 64x8 tiles (64: 23.3); 32x8 where rows are too short for them (24:
+    // 21.1 against 12.8 and 12.9 against 9.7) or end in half of one (32: 24.3
+    // against 17.5, 96: 22.7 against 21.8, 160: 22.6 against 21.9, 224: 13.8
+    // against 13.3), but not where they end in less (72: 12.0 against 14.4 with
+    // 64x8, 136: 12.8 against 15.8, 144: 19.5 against 20.5); whole rows that are
+    // odd multiples of 16 (48: 23.6 against 21.7, 80: 20.9 against 18.6, 112: 22.8
+    // against 21.6), of which the long ones pay with stored g only (144: 19.7
+    // against 20.5, but 13.3 against 12.6; 176: 20.9 against 22.0, 13.6 against 12.9).
     if (p.storage == MCB_STORE_FP32) {
-        const int over = p.nx % 64;
-        Tiling t = over > 0 && over <= 32 && p.nx < 192 ? Tiling{32, 8, 8} : Tiling{64, 8, 8};
-        if (p.nx == 48) t = Tiling{48, 4, 8};
+        Tiling t = p.nx <= 32 || p.nx % 64 == 32 ? Tiling{32, 8, 8} : Tiling{64, 8, 8};
+        const Tiling row{p.nx, 4, 8};
+        if (p.nx >= 48 && p.nx % 32 == 16 && (p.nx < 128 || p.tau_g != 1.0f) && tiling_supported(row)) t = row;
         t.zc = std::min(t.zc, p.nz);
         return t;
     }
@@ -597,10 +601,28 @@ mcb_status Batch::rebuild() {
     B_HIP(hipStreamSynchronize(stream_));
     mcb_status st = ensure_macro_scratch();
     if (st != MCB_OK) return st;
+    // FP32 cases whose rules name different shapes all step on 64x8 tiles: one
+    // launch per pass for a mode. Groups of their own, side by side, gained 8% at
+    // best (16 cubes of 32 to 64 cells, 100 steps a call: 120 against 111 us; 32
+    // of 32 to 128: 897 against 905) and cost a call of one step the events that
+    // join them (16, 32, 48 and 64: 50 against 84 us).
+    // (All the rules' chunks are 8 planes, so the views serve either shape.)
+    auto ruled = [&](const CaseState* c) { return storage_ == MCB_STORE_FP32 && !c->own_tiling; };
+    bool mixed = false;
+    const CaseState* first = nullptr;
+    for (auto& kv : cases_) {
+        const CaseState* c = kv.second.get();
+        if (!ruled(c)) continue;
+        if (!first) first = c;
+        mixed |= c->tiling.tx != first->tiling.tx || c->tiling.ty != first->tiling.ty;
+    }
+    auto shape = [&](const CaseState* c) { return mixed && ruled(c) ? Tiling{64, 8, c->tiling.zc} : c->tiling; };
+    auto phase_shape = [&](const CaseState* c) { return mixed && ruled(c) ? shape(c) : c->phase; };
     // Cases in the order of their groups (tile shapes and collide mode).
     auto key = [&](int id) {
         const CaseState* c = cases_[id].get();
-        return std::make_tuple(c->tiling.tx, c->tiling.ty, c->mode, c->phase.tx, c->phase.ty);
+        const Tiling t = shape(c), pt = phase_shape(c);
+        return std::make_tuple(t.tx, t.ty, c->mode, pt.tx, pt.ty);
     };
     order_.clear();
     for (auto& kv : cases_) order_.push_back(kv.first);
@@ -659,8 +681,8 @@ mcb_status Batch::rebuild() {
         gr.first = (unsigned)start[k];
         gr.cases = (unsigned)(end - start[k]);
         const CaseState* c0 = cases_[order_[start[k]]].get();
-        gr.t = Tiling{c0->tiling.tx, c0->tiling.ty, 0};
-        gr.pt = Tiling{c0->phase.tx, c0->phase.ty, 0};
+        gr.t = shape(c0);
+        gr.pt = phase_shape(c0);
         gr.mode = c0->mode;
         gr.mass = false;
         gr.sum = c0->sum;   // of its own: a case alone (a context) only
@@ -672,10 +694,10 @@ mcb_status Batch::rebuild() {
         for (size_t i = start[k]; i < end; ++i) {
             const CaseState* c = cases_[order_[i]].get();
             if (c->massq || c->mass) gr.mass = true;
-            const auto tl = tiles_of(*c, (int)i, c->tiling), pl = tiles_of(*c, (int)i, c->phase);
+            const auto tl = tiles_of(*c, (int)i, shape(c)), pl = tiles_of(*c, (int)i, phase_shape(c));
             items.insert(items.end(), tl.begin(), tl.end());
             phase.insert(phase.end(), pl.begin(), pl.end());
-            differ |= !same_tiling(c->phase, c->tiling);
+            differ |= !same_tiling(phase_shape(c), shape(c));
             work += c->geo.n;
         }
         items = xcd_permute(items);

@@ -239,3 +239,29 @@ def test_rows_around_the_padding_rule(gpu_lib, storage, tau_g, nx):
         got, want = lat.observables(), b.observables(cid)
         for k in FIELDS:
             assert np.array_equal(got[k], want[k]), k
+
+
+@pytest.mark.parametrize("tau_g", [1.0, 0.8])
+@pytest.mark.parametrize("sides,other", [((32, 32), 48), ((80, 80), 33), ((48, 144), 176), ((24, 24), 96), ((112, 112), 16)])
+def test_fp32_batch_shapes_change_as_cases_join_and_leave(gpu_lib, sides, other, tau_g):
+    """A batch of one tile shape, with a case of another shape for some steps, and one whose tile the caller sets."""
+    mcb = gpu_lib
+
+    def case(n):
+        return mcb.make_params(n, 20, 18, tau_f=0.6, tau_g=tau_g), (0.4 * n, 10.0, 9.0, 5.0)
+
+    with mcb.Batch(0) as b:
+        ids = [b.add(case(n)[0], [case(n)[1]], 3.0) for n in sides]
+        b.step(3)
+        extra = b.add(case(other)[0], [case(other)[1]], 3.0)
+        b.step(2)
+        b.set_tiling(ids[0], 16, 16, 5)
+        b.step(2)
+        got = {"extra": b.read(extra, "phi")}
+        want = {"extra": alone(mcb, case(other)[0], case(other)[1], 4)}
+        b.remove(extra)
+        b.step(4)
+        for i, n in zip(ids, sides):
+            got[i], want[i] = b.read(i, "phi"), alone(mcb, case(n)[0], case(n)[1], 11)
+        for k in got:
+            assert np.array_equal(got[k], want[k]), k
