@@ -18,10 +18,17 @@ unsigned pop_bytes(int storage) { return storage == MCB_STORE_FP32 ? 4u : 2u; }
 
 constexpr int kMacroFields = 10;
 
-// Smallest group that is split for overlap (see rebuild): below, each half is
-// a chain of launches too short to fill the device (a batch of 5.8M cells in
-// FP16 with its largest group split: 199 us per step against 155).
-constexpr long long kSplitCells = 8LL << 20;
+// A batch of one group steps as two halves side by side, in calls of two steps
+// or more, from kSplitCells on: below, each half is a chain of launches too short
+// to fill the device (5.8M cells in FP16: 199 us per step against 155). FP32 up
+// to 24M cells, 16M with stored g (us per step, halves against whole, tau_g 1: 20
+// cubes of 80 493 against 523, 32 of 32 to 128, 18M cells, 777 against 793, 13 of
+// 144 1914 against 1884; tau_g 0.8: 775 against 811, 1357 against 1359, 10 of 128
+// 1527 against 1508); FP16 13 of 144 1254 and 3824 against 1327 and 3908. A call
+// of one step pays for the join (33 cubes of 72: 888 against 875), and next to
+// other groups the halves of the largest one hold up the rest (16 FP16 cubes of
+// 48 to 128: 467 against 433).
+constexpr long long kSplitCells = 8LL << 20, kSplitCellsFp32 = 24LL << 20, kSplitCellsFp32Bgk = 16LL << 20;
 // What a group's launches of a step cost on their lane beside its cells, in
 // cells (about 25 us).
 constexpr long long kGroupCells = 1LL << 20;
@@ -653,34 +660,36 @@ mcb_status Batch::rebuild() {
     }
     for (int q = 0; q < 2; ++q)
         if (n) B_HIP(hipMemcpyAsync(d_views_[q], hv_[q].data(), n * sizeof(CaseView), hipMemcpyHostToDevice, stream_));
-    // Groups, and [start[k], start[k + 1]) their cases. One with more than half
-    // of the work is cut in two, so that there are chains to overlap.
-    auto cells = [&](size_t i) { return cases_[order_[i]]->geo.n; };
-    std::vector<size_t> start;
-    long long total = 0;
+    // Groups: [start[k], start[k + 1]) are the cases of group k. Behind them the
+    // halves of a single large one.
+    std::vector<std::pair<size_t, size_t>> range;
     for (size_t i = 0; i < n; ++i) {
-        if (i == 0 || key(order_[i]) != key(order_[i - 1])) start.push_back(i);
-        total += cells(i);
+        if (i == 0 || key(order_[i]) != key(order_[i - 1])) range.emplace_back(i, i);
+        range.back().second = i + 1;
     }
-    for (size_t k = 0; k < start.size(); ++k) {
-        const size_t end = k + 1 < start.size() ? start[k + 1] : n;
+    n_groups_ = range.size();
+    n_halves_ = 0;
+    if (n_groups_ == 1 && n > 1) {
+        auto cells = [&](size_t i) { return cases_[order_[i]]->geo.n; };
         long long work = 0, half = 0;
-        for (size_t i = start[k]; i < end; ++i) work += cells(i);
-        if (2 * work <= total || work < kSplitCells || end - start[k] < 2) continue;
-        size_t cut = start[k];
-        while (cut < end - 1 && 2 * half < work) half += cells(cut++);
-        start.insert(start.begin() + (long)k + 1, cut);
-        break;
+        for (size_t i = 0; i < n; ++i) work += cells(i);
+        const long long most = cases_[order_[0]]->mode == COLLIDE_STEP ? kSplitCellsFp32 : kSplitCellsFp32Bgk;
+        if (work >= kSplitCells && (storage_ != MCB_STORE_FP32 || work < most)) {
+            size_t cut = 0;
+            while (cut < n - 1 && 2 * half < work) half += cells(cut++);
+            range.emplace_back(0, cut);
+            range.emplace_back(cut, n);
+            n_halves_ = 2;
+        }
     }
-    n_groups_ = n ? start.size() : 0;
-    if (groups_.size() < n_groups_) groups_.resize(n_groups_);
+    if (groups_.size() < range.size()) groups_.resize(range.size());
     std::vector<std::pair<long long, size_t>> load;   // cost and index of a group
-    for (size_t k = 0; k < n_groups_; ++k) {
+    for (size_t k = 0; k < range.size(); ++k) {
         Group& gr = groups_[k];
-        const size_t end = k + 1 < n_groups_ ? start[k + 1] : n;
-        gr.first = (unsigned)start[k];
-        gr.cases = (unsigned)(end - start[k]);
-        const CaseState* c0 = cases_[order_[start[k]]].get();
+        const size_t begin = range[k].first, end = range[k].second;
+        gr.first = (unsigned)begin;
+        gr.cases = (unsigned)(end - begin);
+        const CaseState* c0 = cases_[order_[begin]].get();
         gr.t = shape(c0);
         gr.pt = phase_shape(c0);
         gr.mode = c0->mode;
@@ -691,7 +700,7 @@ mcb_status Batch::rebuild() {
         std::vector<WorkItem> items, phase;
         bool differ = false;
         long long work = 0;
-        for (size_t i = start[k]; i < end; ++i) {
+        for (size_t i = begin; i < end; ++i) {
             const CaseState* c = cases_[order_[i]].get();
             if (c->massq || c->mass) gr.mass = true;
             const auto tl = tiles_of(*c, (int)i, shape(c)), pl = tiles_of(*c, (int)i, phase_shape(c));
@@ -718,7 +727,8 @@ mcb_status Batch::rebuild() {
         }
         B_HIP(hipMemcpyAsync(gr.d_work, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, stream_));
         B_HIP(hipStreamSynchronize(stream_));   // items is a host temporary
-        load.emplace_back(work + kGroupCells, k);
+        if (k < n_groups_) load.emplace_back(work + kGroupCells, k);
+        else gr.lane = (int)(k - n_groups_);
     }
     B_HIP(hipStreamSynchronize(stream_));   // the copies of hv_
     // Lanes: each group to the least loaded one, largest first.
@@ -730,8 +740,9 @@ mcb_status Batch::rebuild() {
         groups_[l.second].lane = at;
         lane_load[at] += l.first;
     }
-    if (lanes_ > 1 && !fork_) B_HIP(hipEventCreateWithFlags(&fork_, hipEventDisableTiming));
-    for (int i = 0; i + 1 < lanes_; ++i) {
+    const int lanes = std::max(lanes_, n_halves_);
+    if (lanes > 1 && !fork_) B_HIP(hipEventCreateWithFlags(&fork_, hipEventDisableTiming));
+    for (int i = 0; i + 1 < lanes; ++i) {
         if (!lane_[i]) B_HIP(hipStreamCreateWithFlags(&lane_[i], hipStreamNonBlocking));
         if (!join_[i]) B_HIP(hipEventCreateWithFlags(&join_[i], hipEventDisableTiming));
     }
@@ -741,16 +752,19 @@ mcb_status Batch::rebuild() {
 
 mcb_status Batch::launch_steps(int q, int n) {
     // A caller capturing stream_ gets everything recorded there.
+    int lanes = n > 1 ? std::max(lanes_, n_halves_) : lanes_;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (lanes_ > 1) B_HIP(hipStreamIsCapturing(stream_, &cap));
-    const bool fork = lanes_ > 1 && cap == hipStreamCaptureStatusNone;
+    if (lanes > 1) B_HIP(hipStreamIsCapturing(stream_, &cap));
+    if (cap != hipStreamCaptureStatusNone) lanes = 1;
+    const bool fork = lanes > 1, halves = fork && n_halves_ > 0;
+    const size_t first = halves ? n_groups_ : 0, last = halves ? n_groups_ + (size_t)n_halves_ : n_groups_;
     if (fork) {
         B_HIP(hipEventRecord(fork_, stream_));
-        for (int i = 0; i + 1 < lanes_; ++i) B_HIP(hipStreamWaitEvent(lane_[i], fork_, 0));
+        for (int i = 0; i + 1 < lanes; ++i) B_HIP(hipStreamWaitEvent(lane_[i], fork_, 0));
     }
     hipError_t e = hipSuccess;
     for (int k = 0; k < n && e == hipSuccess; ++k, q ^= 1)
-        for (size_t i = 0; i < n_groups_ && e == hipSuccess; ++i) {
+        for (size_t i = first; i < last && e == hipSuccess; ++i) {
             const Group& gr = groups_[i];
             const hipStream_t s = fork && gr.lane ? lane_[gr.lane - 1] : stream_;
             e = gr.n_phase ? launch_phase_batch(d_views_[q], gr.d_work + gr.n, gr.n_phase, gr.pt, storage_, s)
@@ -760,9 +774,11 @@ mcb_status Batch::launch_steps(int q, int n) {
             if (e == hipSuccess) e = launch_collide_batch(d_views_[q], gr.d_work, gr.n, gr.t, gr.mode, storage_, s);
         }
     // Also after an error: whatever was launched is ordered before stream_'s next work.
-    for (int i = 0; fork && i + 1 < lanes_; ++i) {
-        B_HIP(hipEventRecord(join_[i], lane_[i]));
-        B_HIP(hipStreamWaitEvent(stream_, join_[i], 0));
+    for (int i = 0; fork && i + 1 < lanes; ++i) {
+        hipError_t j = hipEventRecord(join_[i], lane_[i]);
+        if (j == hipSuccess) j = hipStreamWaitEvent(stream_, join_[i], 0);
+        if (j != hipSuccess) (void)hipStreamSynchronize(lane_[i]);
+        if (e == hipSuccess) e = j;
     }
     B_HIP(e);
     return MCB_OK;

@@ -181,8 +181,9 @@ private:
         bool mass = false;               // a case keeps a mass-drift correction (MassCell or MassQ)
         int lane = 0;                    // 0: stream_, i: lane_[i - 1]
     };
-    std::vector<Group> groups_;          // the first n_groups_ are in use (tables are kept for reuse)
+    std::vector<Group> groups_;          // the first n_groups_ + n_halves_ are in use (tables are kept for reuse)
     size_t n_groups_ = 0;
+    int n_halves_ = 0;                   // 2: behind a single group stand its halves (kSplitCells)
     static constexpr int kLanes = 4;     // hardware queues of a process
     hipStream_t lane_[kLanes - 1] = {};  // created when a batch first needs them
     hipEvent_t fork_ = nullptr, join_[kLanes - 1] = {};

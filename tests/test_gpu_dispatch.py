@@ -4,6 +4,8 @@ FP32: bit for bit against the oracle, on lattices whose phase pass runs single
 planes, partial tiles, chunks that do not divide the lattice, and one or more
 full rounds of workgroups.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -265,3 +267,55 @@ def test_fp32_batch_shapes_change_as_cases_join_and_leave(gpu_lib, sides, other,
             got[i], want[i] = b.read(i, "phi"), alone(mcb, case(n)[0], case(n)[1], 11)
         for k in got:
             assert np.array_equal(got[k], want[k]), k
+
+
+@pytest.mark.parametrize("storage,sides", [(1, [(192, 160, 150)] * 2), (0, [(192, 160, 150), (160, 150, 200)]),
+                                           (0, [(192, 160, 150)] * 6)])
+def test_large_batch_as_halves_and_whole(gpu_lib, storage, sides):
+    """Calls of one step run the batch whole, longer ones as two halves side by side (the last is too large for that)."""
+    mcb = gpu_lib
+    with mcb.Batch(storage) as b:
+        cases = []
+        for i, (nx, ny, nz) in enumerate(sides):
+            p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.55 + 0.02 * i)
+            bub = ((0.4 + 0.05 * i) * nx, 0.5 * ny, 0.6 * nz, 0.28 * min(nx, ny, nz))
+            cases.append((b.add(p, [bub], 3.0), p, bub))
+        for steps in (2, 1, 3, 1, 1, 4):
+            b.step(steps)
+        for cid, p, bub in cases:
+            assert np.array_equal(b.read(cid, "phi"), alone(mcb, p, bub, 12)), cid
+
+
+@pytest.mark.parametrize("storage,sides", [(1, [32, 48, 33, 64, 80]), (1, [(192, 160, 150)] * 2), (0, [32, 48, 70])])
+def test_batch_steps_inside_a_caller_graph(gpu_lib, storage, sides):
+    """A caller that captures the batch's stream gets every group and every half recorded there; replays, with the batch's
+    own steps and reads between them, advance it like the same steps launched directly."""
+    mcb = gpu_lib
+    hip = ctypes.CDLL("libamdhip64.so")
+    vp = ctypes.c_void_p
+    stream, graph, exe = vp(), vp(), vp()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    with mcb.Batch(storage, stream=stream) as g, mcb.Batch(storage) as e:
+        ids = []
+        for i, n in enumerate(sides):
+            nx, ny, nz = (n, 20, 18) if isinstance(n, int) else n
+            p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.6, tau_g=0.8 if i % 2 else 1.0)
+            bub = [(0.4 * nx, 0.5 * ny, 0.5 * nz, 0.3 * min(nx, ny, nz))]
+            ids.append((g.add(p, bub, 3.0), e.add(p, bub, 3.0)))
+        g.step(1)
+        e.step(1)
+        g.synchronize()
+        assert hip.hipStreamBeginCapture(stream, 1) == 0          # thread-local mode
+        g.step(2)                                                 # recorded, not run
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+        for replay in range(4):
+            assert hip.hipGraphLaunch(exe, stream) == 0
+            g.step(2)
+            e.step(4)
+            for a, b in ids:
+                x, y = g.read(a, "phi"), e.read(b, "phi")
+                assert np.array_equal(x, y), (replay, a, int(np.count_nonzero(x != y)))
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+    hip.hipStreamDestroy(stream)
