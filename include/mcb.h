@@ -190,10 +190,12 @@ mcb_status mcb_get_tiling(const mcb_ctx* ctx, int* tx, int* ty, int* zc);
 int mcb_tiling_count(void);
 mcb_status mcb_tiling_at(int i, int* tx, int* ty);
 
-/* Time every supported tile shape and z-chunk on a scratch lattice with these
- * parameters (on p->device) and remember the fastest; later contexts and
- * batch cases of the same sides and storage use it. No reference counterpart
- * (the reference launches fixed 8x8x8 blocks, src/main.cu:43-46). */
+/* Time every supported tile shape and z-chunk on a scratch context with these
+ * parameters (on p->device) and remember the fastest; later contexts of the
+ * same sides, storage and form of g (tau_g = 1 or not) use it. With 16-bit
+ * storage and tau_g = 1 a batch case is tuned beside it, for later batch
+ * cases. No reference counterpart (the reference launches fixed 8x8x8 blocks,
+ * src/main.cu:43-46). */
 mcb_status mcb_autotune(const mcb_params* p, int* tx, int* ty, int* zc, double* ms_per_step);
 
 /* ---- Batches: many independent periodic cases resident on one device ----

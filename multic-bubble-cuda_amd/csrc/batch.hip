@@ -173,20 +173,28 @@ CaseState::~CaseState() {
 // ---------------------------------------------------------------- tilings
 
 namespace {
+// Tuned tiles by sides, storage, form of g and whether the lattice is alone.
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int, int>, Tiling> g_tuned;
+using TuneKey = std::tuple<int, int, int, int, bool, bool>;
+std::map<TuneKey, Tiling> g_tuned;
+
+TuneKey tune_key(const mcb_params& p, bool alone) {
+    return TuneKey{p.nx, p.ny, p.nz, p.storage, p.tau_g == 1.0f, alone};
+}
+
+bool tuned(const mcb_params& p, bool alone, Tiling* t) {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    auto it = g_tuned.find(tune_key(p, alone));
+    if (it != g_tuned.end()) *t = it->second;
+    return it != g_tuned.end();
+}
 
 bool supported_for(const Tiling& t, int storage) {
     return storage == MCB_STORE_FP32 ? tiling_supported(t) : tiling_supported16(t);
 }
 }  // namespace
 
-Tiling choose_tiling(const mcb_params& p) {
-    {
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        auto it = g_tuned.find(std::make_tuple(p.nx, p.ny, p.nz, p.storage));
-        if (it != g_tuned.end()) return it->second;
-    }
+static Tiling choose_tiling(const mcb_params& p) {
     Tiling t = p.nx >= 64 ? Tiling{64, 8, 16} : (p.nx >= 32 ? Tiling{32, 8, 16} : Tiling{16, 16, 16});
     // 16-bit forms: half the bytes per cell, so longer z runs pay off
     // (measured at 256^3: 64x8x32 fastest, 64x4x32 4% and 32x8x32 17%
@@ -225,15 +233,18 @@ Tiling batch_tiling(const mcb_params& p) {
         t.zc = std::min(t.zc, p.nz);
         return t;
     }
-    return choose_tiling(p);
+    // Stored 16-bit g: the sums of phi follow these tiles (build_own_table), and
+    // so do a run's bits; they don't depend on what was tuned before.
+    Tiling t;
+    return p.tau_g == 1.0f && tuned(p, false, &t) ? t : choose_tiling(p);
 }
 
 Tiling choose_tiling_single(const mcb_params& p) {
-    {
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        auto it = g_tuned.find(std::make_tuple(p.nx, p.ny, p.nz, p.storage));
-        if (it != g_tuned.end()) return it->second;
-    }
+    Tiling t;
+    return p.f_form == MCB_F_POPULATIONS && tuned(p, true, &t) ? t : rule_tiling_single(p);
+}
+
+Tiling rule_tiling_single(const mcb_params& p) {
     Tiling t = choose_tiling(p);
     const bool fp32 = p.storage == MCB_STORE_FP32;
     // A lattice alone on the device (us per step, this rule against 64x8x16,
@@ -1166,59 +1177,20 @@ mcb_status Batch::synchronize() {
 
 // --------------------------------------------------------------- autotune
 
-mcb_status autotune(const mcb_params& p0, int device, Tiling* best, double* ms_per_step) {
-    mcb_params p = p0;
-    p.bc_mode = MCB_BC_PERIODIC;
-    if (hipSetDevice(device) != hipSuccess) return MCB_ERR_NO_DEVICE;
-    hipStream_t s = nullptr;
-    if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return MCB_ERR_HIP;
-    mcb_status result = MCB_OK;
-    double best_ms = 1e30;
-    Tiling best_t = choose_tiling(p);
-    {
-        Batch b(device, s);
-        // A centred bubble of radius nx/4 as the scratch state.
-        mcb_bubble bub{p.nx * 0.5f, p.ny * 0.5f, p.nz * 0.5f, p.nx * 0.25f};
-        int id = 0;
-        mcb_status st = b.add_bubbles(p, &bub, 1, 3.0f, &id);
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (st == MCB_OK && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)) st = MCB_ERR_HIP;
-        const long long cells = (long long)p.nx * p.ny * p.nz;
-        const int steps = (int)std::max<long long>(4, std::min<long long>(40, 400000000LL / std::max<long long>(cells, 1)));
-        for (int i = 0; st == MCB_OK && i < tiling_count(); ++i) {
-            for (int zc : {8, 16, 32}) {
-                Tiling t = tiling_at(i);
-                t.zc = std::min(zc, p.nz);
-                if (!supported_for(t, p.storage) || t.tx > 2 * p.nx || t.ty > 2 * p.ny) continue;
-                if ((st = b.set_tiling(id, t)) != MCB_OK) break;
-                if ((st = b.step(2)) != MCB_OK) break;
-                float ms = 0.0f;
-                if (hipEventRecord(e0, s) != hipSuccess) { st = MCB_ERR_HIP; break; }
-                if ((st = b.step(steps)) != MCB_OK) break;
-                if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                    hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                    st = MCB_ERR_HIP;
-                    break;
-                }
-                if (ms / steps < best_ms) {
-                    best_ms = ms / steps;
-                    best_t = t;
-                }
-            }
+void remember_tiling(const mcb_params& p, bool alone, const Tiling& t) {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    g_tuned[tune_key(p, alone)] = t;
+}
+
+std::vector<Tiling> tune_candidates(const mcb_params& p, bool alone) {
+    std::vector<Tiling> v{alone ? rule_tiling_single(p) : choose_tiling(p)};
+    for (int i = 0; i < tiling_count(); ++i)
+        for (int zc : {1, 2, 4, 8, 16, 32}) {
+            const Tiling t{tiling_at(i).tx, tiling_at(i).ty, zc};
+            if (zc <= p.nz && supported_for(t, p.storage) && t.tx <= 2 * p.nx && t.ty <= 2 * p.ny && !same_tiling(t, v[0]))
+                v.push_back(t);
         }
-        if (e0) (void)hipEventDestroy(e0);
-        if (e1) (void)hipEventDestroy(e1);
-        result = st;
-    }
-    (void)hipStreamDestroy(s);
-    if (result != MCB_OK) return result;
-    {
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_tuned[std::make_tuple(p0.nx, p0.ny, p0.nz, p0.storage)] = best_t;
-    }
-    if (best) *best = best_t;
-    if (ms_per_step) *ms_per_step = best_ms;
-    return MCB_OK;
+    return v;
 }
 
 }  // namespace mcb

@@ -200,17 +200,17 @@ private:
     size_t pool_limit_ = 0;
 };
 
-// Tile shape for a lattice: the autotuned choice for (nx, ny, nz, storage)
-// when one exists, else a size rule.
-Tiling choose_tiling(const mcb_params& p);
 // The tiling of a single-case context: the autotuned choice, else a rule for a
-// lattice that has the device to itself.
+// lattice that has the device to itself (rule_tiling_single).
 Tiling choose_tiling_single(const mcb_params& p);
+Tiling rule_tiling_single(const mcb_params& p);
 // The tiling of a batch case, where the batch fills the device: by row length
-// in FP32, the 16-bit rule of choose_tiling otherwise.
+// in FP32, else the autotuned choice (tau_g = 1) or a rule.
 Tiling batch_tiling(const mcb_params& p);
-// Measure every supported tile shape and z-chunk on a scratch case and
-// remember the fastest for (nx, ny, nz, storage).
-mcb_status autotune(const mcb_params& p, int device, Tiling* best, double* ms_per_step);
+// Autotuning: the tiles to measure for a context (alone) or a batch case, the
+// rule's own first, and the choice for later ones of these sides, storage and
+// form of g.
+std::vector<Tiling> tune_candidates(const mcb_params& p, bool alone);
+void remember_tiling(const mcb_params& p, bool alone, const Tiling& t);
 
 }  // namespace mcb

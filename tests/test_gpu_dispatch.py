@@ -319,3 +319,32 @@ def test_batch_steps_inside_a_caller_graph(gpu_lib, storage, sides):
         hip.hipGraphExecDestroy(exe)
         hip.hipGraphDestroy(graph)
     hip.hipStreamDestroy(stream)
+
+
+@pytest.mark.parametrize("storage,tau_g,nx,ny,nz", [(0, 1.0, 40, 36, 44), (0, 0.8, 40, 36, 44), (1, 1.0, 66, 20, 50), (1, 0.8, 48, 30, 20)])
+def test_autotuned_context(gpu_lib, storage, tau_g, nx, ny, nz):
+    """The tuner measures what a context runs, the rule's tile among the rest: contexts of the same form of g take its
+    choice, others keep the rule's, and no choice changes a result."""
+    mcb = gpu_lib
+    p = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.6, tau_g=tau_g)
+    q = mcb.make_params(nx, ny, nz, storage=storage, tau_f=0.6, tau_g=1.8 - tau_g)
+    bub = (0.4 * nx, 0.5 * ny, 0.5 * nz, 0.3 * min(nx, ny, nz))
+
+    def tiling(params):
+        with mcb.Lattice(params) as lat:
+            return lat.tiling()
+
+    rule, other = tiling(p), tiling(q)
+    want = alone(mcb, p, bub, 6)
+    tx, ty, zc, ms = mcb.autotune(p)
+    assert ms > 0 and tiling(p) == (tx, ty, zc) and tiling(q) == other
+    assert np.array_equal(alone(mcb, p, bub, 6), want)
+    with mcb.Lattice(p) as lat, mcb.Batch(storage) as b:
+        lat.init_bubbles([bub], 3.0)
+        lat.step(3)
+        cid = b.add_state(lat.save_state())
+        lat.step(3)
+        b.step(3)
+        assert np.array_equal(lat.read("phi"), b.read(cid, "phi"))
+    # From the tuned state the rule's tile is still a candidate.
+    assert mcb.autotune(p)[:2] in mcb.tilings() and rule[:2] in mcb.tilings()
