@@ -109,10 +109,11 @@ Geo fused_geo(const mcb_params& p, bool pad_rows) {
 // each of theirs, 8 rows 1.29 (256^3 FP16: 117 against 103 VALU and 37 against 34
 // LDS instructions a cell, 92 us a pass against 85),
 // while the collide pass wants the many small workgroups. Where 8 rows and
-// longer chunks leave three workgroups a CU: 100 steps and a read of 256^3 FP16
-// 41.1 ms against 42.2, 192^3 BF16 18.7 against 18.6; below that 4 rows keep more
-// of the device busy (117x90x133 57 us per step against 59). The fixed-point
-// sums of phi do not depend on the tiles.
+// longer chunks leave three workgroups a CU (us per step, 8 rows against 4, FP16
+// and BF16 alike): 256^3 380 against 390, 256x256x128 197 against 203, 250^3 414
+// against 429; 192^3, 224^3 and 256x200x130 the same. Below that 4 rows keep more
+// of the device busy (117x90x133 57 against 59). The fixed-point sums of phi do
+// not depend on the tiles.
 static Tiling phase_tiling16(const mcb_params& p, const Tiling& t) {
     if (t.tx != 64 || t.ty != 4) return t;
     auto groups = [&](int zc) { return (long long)((p.nx + 63) / 64) * ((p.ny + 7) / 8) * ((p.nz + zc - 1) / zc); };

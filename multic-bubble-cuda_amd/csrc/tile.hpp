@@ -1805,9 +1805,17 @@ __device__ __forceinline__ void mass_partial(const CaseView& c, const WorkItem& 
     if (threadIdx.y == 0 && threadIdx.x == 0) c.partial[tile] = s;
 }
 
+// The BF16 phase pass on 64x8 tiles is held to 64 VGPRs, so that 8 waves share a
+// SIMD as in FP16 (60): by itself it took 67 (its stored-g path decodes with
+// more), a workgroup per CU less (256^3 398 us per step, held 381, FP16 380).
+template <int TX, int TY, class S> constexpr int phase_waves_per_eu() {
+    return std::is_same_v<S, StoreBF16> && TX * TY == 512 ? 8 : 1;
+}
+
 template <int TX, int TY, class S>
-__global__ __launch_bounds__(TX * TY) void k_phase_batch(const CaseView* __restrict__ cases,
-                                                         const WorkItem* __restrict__ work) {
+__global__ __launch_bounds__(TX * TY)
+__attribute__((amdgpu_waves_per_eu(phase_waves_per_eu<TX, TY, S>())))
+void k_phase_batch(const CaseView* __restrict__ cases, const WorkItem* __restrict__ work) {
     const WorkItem w = work[blockIdx.x];
     const CaseView c = cases[w.c];
     const Geo& G = c.geo;
