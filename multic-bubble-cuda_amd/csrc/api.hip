@@ -836,9 +836,8 @@ mcb_status mcb_read_field(mcb_ctx* c, int field, float* host, size_t n) {
                                              0, c->geo, +1, c->stream));
             }
             const float* tmp = field == MCB_FIELD_F || c->gm != GM_POPULATIONS ? idle_f : c->g[c->cur ^ 1];
-            for (int l = 0; l < 19; ++l)
-                MCB_HIP(c, Readback::copy(c->readback.get(), host + l * cells, tmp + (size_t)l * c->geo.plane, cells * sizeof(float),
-                                             c->stream));
+            MCB_HIP(c, Readback::copy_rows(c->readback.get(), host, tmp, cells * sizeof(float),
+                                           (size_t)c->geo.plane * sizeof(float), 19, c->stream));
             if (c->p.bc_mode == MCB_BC_REFERENCE)   // restore the idle buffer's face populations (w_l)
                 MCB_HIP(c, launch_init_pull(c->phi, c->f[c->cur ^ 1], nullptr, c->geo, c->phys, c->stream));
         }

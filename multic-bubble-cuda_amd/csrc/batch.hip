@@ -880,8 +880,8 @@ mcb_status Batch::read(int id, int field, float* host, size_t n) {
         else
             e = launch_decode16(isf ? c->f[c->cur] : c->g[c->cur], isf ? nullptr : c->phi[c->cur ^ 1], tmp, c->geo,
                                 c->phys, c->storage, stream_);
-        for (int l = 0; l < 19 && e == hipSuccess; ++l)
-            e = Readback::copy(readback_.get(), host + l * cells, tmp + l * P, cells * sizeof(float), stream_);
+        if (e == hipSuccess)
+            e = Readback::copy_rows(readback_.get(), host, tmp, cells * sizeof(float), P * sizeof(float), 19, stream_);
         (void)hipFree(tmp);
         B_HIP(e);
         return MCB_OK;

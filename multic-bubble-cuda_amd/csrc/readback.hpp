@@ -21,6 +21,10 @@ public:
     // host[0, bytes) = dev[0, bytes) behind the work queued on `stream` (of
     // the current device); returns when the copy is complete. r may be null.
     static hipError_t copy(Readback* r, void* host, const void* dev, size_t bytes, hipStream_t stream);
+    // The same for `rows` rows of `bytes`, `pitch` bytes apart on the device and
+    // dense on the host; small rows share one wait.
+    static hipError_t copy_rows(Readback* r, void* host, const void* dev, size_t bytes, size_t pitch, int rows,
+                                hipStream_t stream);
 
 private:
     bool ready(size_t bytes);
