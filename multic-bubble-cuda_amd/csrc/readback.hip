@@ -33,6 +33,15 @@ constexpr size_t kOneWait = 32u << 10;
 
 struct Events {
     hipEvent_t e[kSlots] = {};
+    bool create() {
+        for (auto& x : e)
+            if (hipEventCreateWithFlags(&x, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                x = nullptr;
+                return false;
+            }
+        return true;
+    }
     ~Events() {
         for (auto x : e)
             if (x) (void)hipEventDestroy(x);
@@ -87,8 +96,10 @@ hipError_t Readback::copy(Readback* r, void* host, const void* dev, size_t bytes
     if (r && bytes >= kMinBytes && pageable(host) && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
         cs == hipStreamCaptureStatusNone) {
         std::unique_lock<std::mutex> lk(r->mu_, std::try_to_lock);
-        if (lk.owns_lock() && r->ready(bytes))
-            return r->staged(static_cast<char*>(host), static_cast<const char*>(dev), bytes, stream);
+        Events ev;
+        int device = 0;
+        if (lk.owns_lock() && r->ready(bytes) && hipGetDevice(&device) == hipSuccess && ev.create())
+            return r->staged(static_cast<char*>(host), static_cast<const char*>(dev), bytes, stream, device, ev.e);
     }
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream);
     return e != hipSuccess ? e : hipStreamSynchronize(stream);
@@ -106,14 +117,8 @@ hipError_t Readback::copy_rows(Readback* r, void* host, const void* dev, size_t 
     return hipStreamSynchronize(stream);
 }
 
-hipError_t Readback::staged(char* host, const char* dev, size_t bytes, hipStream_t stream) {
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    if (e != hipSuccess) return e;
-    Events ev;
-    for (auto& x : ev.e)
-        if ((e = hipEventCreateWithFlags(&x, hipEventDisableTiming)) != hipSuccess) return e;
-
+hipError_t Readback::staged(char* host, const char* dev, size_t bytes, hipStream_t stream, int device,
+                            const hipEvent_t* ev) {
     const size_t chunk = chunk_of(bytes), per = chunk / kSlice;
     const size_t chunks = (bytes + chunk - 1) / chunk, slices = (bytes + kSlice - 1) / kSlice;
     // Slices are claimed in order. Chunk i may enter its slot when the slices
@@ -127,7 +132,7 @@ hipError_t Readback::staged(char* host, const char* dev, size_t bytes, hipStream
     auto send = [&](size_t i) {
         const size_t s = i % kSlots, at = i * chunk;
         hipError_t r = hipMemcpyAsync(ring_ + s * chunk, dev + at, std::min(chunk, bytes - at), hipMemcpyDeviceToHost, stream);
-        if (r == hipSuccess) r = hipEventRecord(ev.e[s], stream);
+        if (r == hipSuccess) r = hipEventRecord(ev[s], stream);
         if (r != hipSuccess) error = r;
         sent[s].store(i / kSlots + 1, std::memory_order_release);
     };
@@ -139,7 +144,7 @@ hipError_t Readback::staged(char* host, const char* dev, size_t bytes, hipStream
                 std::this_thread::yield();
             if (error.load() != hipSuccess) return;
             if (i != here) {
-                const hipError_t r = hipEventSynchronize(ev.e[s]);
+                const hipError_t r = hipEventSynchronize(ev[s]);
                 if (r != hipSuccess) {
                     error = r;
                     return;

@@ -28,7 +28,8 @@ public:
 
 private:
     bool ready(size_t bytes);
-    hipError_t staged(char* host, const char* dev, size_t bytes, hipStream_t stream);
+    // ev: an event per slot, of the current device.
+    hipError_t staged(char* host, const char* dev, size_t bytes, hipStream_t stream, int device, const hipEvent_t* ev);
 
     std::mutex mu_;
     char* ring_ = nullptr;
