@@ -106,9 +106,8 @@ template <int L> MCB_HD float cdot(float vx, float vy, float vz) {
 // The compiler's IEEE division and square root scale their operands, refine
 // and fix up for the whole float range: 11 instructions for a reciprocal, 28
 // for 1 / sqrtf. The step's arguments need less: 4 and 10. Each form below
-// gives the bits of the expression it stands for on the range it states (every
-// float of it compared on the device); div_fixup supplies zeros, infinities
-// and NaN. Outside that range, where a subnormal or a value beyond 2^126 is
+// gives the bits of the expression it stands for on the range it states; div_fixup
+// supplies zeros, infinities and NaN. Outside that range, where a subnormal or a value beyond 2^126 is
 // involved, the last bit may differ. Host code divides. With the products
 // of gradCalc formed once per staged cell and the halves of HeF once per cell,
 // an FP32 collide lane issues 657 + 61 per normal VALU instructions per plane
@@ -196,32 +195,39 @@ struct Moments {
     float pxx, pyy, pzz, pxy, pxz, pyz;
 };
 
+// Any: the same bits for every float, for the populations and densities of a
+// caller (operators). Otherwise (the step) the reciprocals take the short forms
+// above, and the factor 0.5 of HeF is taken into 1 / (rho cs^2) once per cell:
+// scaling by a power of two commutes with rounding, and where a product with a
+// small force is subnormal, HeF is lost next to feq. Both hold while rho lies
+// between 2^-50 and 2^100; beyond, the last bits may differ.
+template <bool Any> MCB_HD float recip(float x) { return Any ? 1.0f / x : recip_rn(x); }
+
 // lbm.cu:161-224. fv[l] are the 19 pre-collision populations of the cell.
-// The factor 0.5 of HeF is taken into invRhoCssq once per cell: scaling by a
-// power of two commutes with rounding, and where a subnormal breaks that,
-// HeF is far below the last bit of the value that it is added to.
+template <bool Any = false>
 MCB_HD Moments moments(const float (&fv)[Q], const Phys& p, float fx, float fy, float fz) {
     Moments m;
     float rho = 0.0f;
     for_links([&](auto lc) { rho += fv[decltype(lc)::value]; });
-    const float invRho = recip_rn(rho);
+    const float invRho = recip<Any>(rho);
     const float sumUx = invRho * (fv[1] - fv[2] + fv[7] - fv[8] + fv[9] - fv[10] + fv[13] - fv[14] + fv[15] - fv[16]);
     const float sumUy = invRho * (fv[3] - fv[4] + fv[7] - fv[8] + fv[11] - fv[12] + fv[14] - fv[13] + fv[17] - fv[18]);
     const float sumUz = invRho * (fv[5] - fv[6] + fv[9] - fv[10] + fv[11] - fv[12] + fv[16] - fv[15] + fv[18] - fv[17]);
     const float ux = sumUx + fx * 0.5f * invRho;
     const float uy = sumUy + fy * 0.5f * invRho;
     const float uz = sumUz + fz * 0.5f * invRho;
-    const float uu = (0.5f * INV_CSSQ) * (ux * ux + uy * uy + uz * uz);
-    const float halfInvRhoCssq = 0.5f * recip_rn(rho * CSSQ);
+    const float u2 = ux * ux + uy * uy + uz * uz;
+    const float uu = Any ? 0.5f * u2 * INV_CSSQ : (0.5f * INV_CSSQ) * u2;
+    const float invRhoCssq = (Any ? 1.0f : 0.5f) * recip<Any>(rho * CSSQ);
     float fneq[Q];
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
         const float udotc = cdot<l>(ux, uy, uz) * INV_CSSQ;
         const float eqBase = rho * (udotc + 0.5f * udotc * udotc - uu);
         const float common = p.w[WC[l]] * (rho + eqBase);
-        const float HeF = common *
+        const float HeF = (Any ? 0.5f * common : common) *
                           (((float)CX[l] - ux) * fx + ((float)CY[l] - uy) * fy + ((float)CZ[l] - uz) * fz) *
-                          halfInvRhoCssq;
+                          invRhoCssq;
         const float feq = common - HeF;
         fneq[l] = fv[l] - feq;
     });
@@ -243,31 +249,32 @@ MCB_HD Moments moments(const float (&fv)[Q], const Phys& p, float fx, float fy, 
 struct FluidCell {
     float rho, ux, uy, uz, fx, fy, fz;
     float pxx, pyy, pzz, pxy, pxz, pyz;
-    float uu, halfInvRhoCssq;
+    float uu, invRhoCssq;   // half of 1 / (rho cs^2) unless Any
 };
 
-MCB_HD FluidCell fluid_cell(const Moments& m, float fx, float fy, float fz) {
+template <bool Any = false> MCB_HD FluidCell fluid_cell(const Moments& m, float fx, float fy, float fz) {
     FluidCell c;
     c.rho = m.rho; c.ux = m.ux; c.uy = m.uy; c.uz = m.uz;
     c.fx = fx; c.fy = fy; c.fz = fz;
     c.pxx = m.pxx; c.pyy = m.pyy; c.pzz = m.pzz;
     c.pxy = m.pxy; c.pxz = m.pxz; c.pyz = m.pyz;
     // Division, as lbm.cu:263 (a uu below 2^-104 is lost next to rho).
-    c.uu = div_cssq(0.5f * (m.ux * m.ux + m.uy * m.uy + m.uz * m.uz));
-    c.halfInvRhoCssq = 0.5f * recip_rn(m.rho * CSSQ);
+    const float half_u2 = 0.5f * (m.ux * m.ux + m.uy * m.uy + m.uz * m.uz);
+    c.uu = Any ? half_u2 / CSSQ : div_cssq(half_u2);
+    c.invRhoCssq = (Any ? 1.0f : 0.5f) * recip<Any>(m.rho * CSSQ);
     return c;
 }
 
 // Post-collision population of link L (lbm.cu:273-286).
-template <int L>
+template <int L, bool Any = false>
 MCB_HD float fluid_post(const FluidCell& c, const Phys& p, const Derived& d) {
     constexpr int cx = CX[L], cy = CY[L], cz = CZ[L];
     const float w = p.w[WC[L]];
     const float udotc = cdot<L>(c.ux, c.uy, c.uz) * INV_CSSQ;
     const float feq = w * (c.rho + c.rho * (udotc + 0.5f * udotc * udotc - c.uu));
-    const float HeF = feq *
+    const float HeF = (Any ? 0.5f * feq : feq) *
                       (((float)cx - c.ux) * c.fx + ((float)cy - c.uy) * c.fy + ((float)cz - c.uz) * c.fz) *
-                      c.halfInvRhoCssq;
+                      c.invRhoCssq;
     constexpr float kx = cx != 0 ? DIAG1 : DIAG0;
     constexpr float ky = cy != 0 ? DIAG1 : DIAG0;
     constexpr float kz = cz != 0 ? DIAG1 : DIAG0;

@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void k_momentiCalc(float* ux, float* uy, float
         constexpr int l = decltype(lc)::value;
         fv[l] = get(f + l * a.geo.plane, x);
     });
-    const Moments m = moments(fv, a.phys, get(ffx, x), get(ffy, x), get(ffz, x));
+    const Moments m = moments<true>(fv, a.phys, get(ffx, x), get(ffy, x), get(ffz, x));
     put(pxx, x, m.pxx);
     put(pyy, x, m.pyy);
     put(pzz, x, m.pzz);
@@ -208,10 +208,10 @@ __global__ __launch_bounds__(256) void k_collisionFluid(float* f, const float* u
     m.pxy = get(pxy, x);
     m.pxz = get(pxz, x);
     m.pyz = get(pyz, x);
-    const FluidCell c = fluid_cell(m, get(ffx, x), get(ffy, x), get(ffz, x));
+    const FluidCell c = fluid_cell<true>(m, get(ffx, x), get(ffy, x), get(ffz, x));
     for_links([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        put(f + l * a.geo.plane, h.template nb<l>(), fluid_post<l>(c, a.phys, d));
+        put(f + l * a.geo.plane, h.template nb<l>(), fluid_post<l, true>(c, a.phys, d));
     });
 }
 
