@@ -291,7 +291,8 @@ Tiling rule_tiling_single(const mcb_params& p) {
     // planes, 12.2 waves, 54.8, 4 planes 56.1) and before single planes
     // (40x100x60 64x4x2, 11.7 waves, 25.9, 1 plane 31); 7 with whole rows, whose
     // halo is small (112^3 8 planes 58.9, 4 planes 60.8). One plane is the
-    // least, 2 in 16 bits.
+    // least, 2 in 16 bits but where 3 planes are halved (lattices of 3, 6 and 7:
+    // 64x64x6 14.1 with 1, 17.7 with 2).
     auto want = [&] { return (row ? 7 : (fp32 && t.zc > 2 ? 13 : 11)) * wave_per_cu; };
     while (t.zc > (fp32 ? 1 : 2) && lanes(t) < want()) t.zc /= 2;
     // Single planes restage their own halo: 8 rows where they pad no more

@@ -477,6 +477,13 @@ Tiling phase_tiling(const Geo& geo, const Tiling& t, bool rn) {
 // 77.2 + 20.6).
 bool phase_recomputes_n(const Geo& geo, const Tiling& t) { return phase_tiling(geo, t, true).zc >= 16; }
 
+template <int TX, int TY> static hipError_t launch_phase_gm_t(const CaseView& c, unsigned tiles, bool rn, hipStream_t s) {
+    if (rn) hipLaunchKernelGGL((k_phase_gm<TX, TY, true>), dim3(tiles), dim3(TX, TY, 1), 0, s, c);
+    else if constexpr (TX == 64 && TY == 4) return hipErrorInvalidValue;   // phase_tiling takes 8 rows
+    else hipLaunchKernelGGL((k_phase_gm<TX, TY, false>), dim3(tiles), dim3(TX, TY, 1), 0, s, c);
+    return hipGetLastError();
+}
+
 hipError_t launch_phase(const CaseView& c0, const Tiling& t, hipStream_t s) {
     if (c0.gm == GM_MOMENTS) {
         CaseView c = c0;
@@ -490,12 +497,8 @@ hipError_t launch_phase(const CaseView& c0, const Tiling& t, hipStream_t s) {
                                dim3(MCB_PHASE_RN_TX, MCB_PHASE_RN_TY, 1), 0, s, c);
             return hipGetLastError();
         }
-#define MCB_PHASE_GM(TX, TY)                                                                                     \
-    if (p.tx == TX && p.ty == TY) {                                                                              \
-        if (rn) hipLaunchKernelGGL((k_phase_gm<TX, TY, true>), dim3(tiles), dim3(TX, TY, 1), 0, s, c);          \
-        else hipLaunchKernelGGL((k_phase_gm<TX, TY, false>), dim3(tiles), dim3(TX, TY, 1), 0, s, c);            \
-        return hipGetLastError();                                                                                \
-    }
+#define MCB_PHASE_GM(TX, TY) \
+    if (p.tx == TX && p.ty == TY) return launch_phase_gm_t<TX, TY>(c, tiles, rn, s);
         MCB_TILES_FP32(MCB_PHASE_GM)
 #undef MCB_PHASE_GM
         return hipErrorInvalidValue;
