@@ -29,6 +29,16 @@ constexpr int kMacroFields = 10;
 // other groups the halves of the largest one hold up the rest (16 FP16 cubes of
 // 48 to 128: 467 against 433).
 constexpr long long kSplitCells = 8LL << 20, kSplitCellsFp32 = 24LL << 20, kSplitCellsFp32Bgk = 16LL << 20;
+// FP32 cases of different shapes step shape by shape, side by side, in calls of
+// two steps or more, where a shape has kShapeCases cases on average; otherwise,
+// and in calls of one step, all on 64x8 tiles in one group (us per step, by shape
+// against one group, 20 steps a call: 16 cubes of 32 to 64 cells 87 against 108,
+// 32 of 32 to 128 825 and with stored g 1396 against 843 and 1435, 30 of 48 to 112
+// 1065 against 1143; but 6 cubes of 5 shapes 168 against 160, 8 of 48 to 192 with
+// stored g 2540 against 2510, 12 of 24 and 33, 0.3M cells, 55 against 49; one step
+// a call 16 of 32 to 64 122 against 108).
+constexpr size_t kShapeCases = 5;
+constexpr long long kShapeCells = 1LL << 20;
 // What a group's launches of a step cost on their lane beside its cells, in
 // cells (about 25 us).
 constexpr long long kGroupCells = 1LL << 20;
@@ -317,8 +327,7 @@ Batch::~Batch() {
     if (fork_) (void)hipEventDestroy(fork_);
     for (auto& e : join_)
         if (e) (void)hipEventDestroy(e);
-    for (auto& g : groups_)
-        if (g.d_work) (void)hipFree(g.d_work);
+    if (d_work_) (void)hipFree(d_work_);
     for (auto& v : d_views_)
         if (v) (void)hipFree(v);
     if (d_partial_) (void)hipFree(d_partial_);
@@ -621,32 +630,36 @@ mcb_status Batch::rebuild() {
     B_HIP(hipStreamSynchronize(stream_));
     mcb_status st = ensure_macro_scratch();
     if (st != MCB_OK) return st;
-    // FP32 cases whose rules name different shapes all step on 64x8 tiles: one
-    // launch per pass for a mode. Groups of their own, side by side, gained 8% at
-    // best (16 cubes of 32 to 64 cells, 100 steps a call: 120 against 111 us; 32
-    // of 32 to 128: 897 against 905) and cost a call of one step the events that
-    // join them (16, 32, 48 and 64: 50 against 84 us).
-    // (All the rules' chunks are 8 planes, so the views serve either shape.)
+    // FP32 cases whose rules name different shapes can step on 64x8 tiles all
+    // together, one launch per pass for a mode (kShapeCases). All the rules'
+    // chunks are 8 planes, so the views serve either shape.
     auto ruled = [&](const CaseState* c) { return storage_ == MCB_STORE_FP32 && !c->own_tiling; };
     bool mixed = false;
-    const CaseState* first = nullptr;
+    const CaseState* some = nullptr;
+    long long total = 0;
     for (auto& kv : cases_) {
         const CaseState* c = kv.second.get();
+        total += c->geo.n;
         if (!ruled(c)) continue;
-        if (!first) first = c;
-        mixed |= c->tiling.tx != first->tiling.tx || c->tiling.ty != first->tiling.ty;
+        if (!some) some = c;
+        mixed |= c->tiling.tx != some->tiling.tx || c->tiling.ty != some->tiling.ty;
     }
-    auto shape = [&](const CaseState* c) { return mixed && ruled(c) ? Tiling{64, 8, c->tiling.zc} : c->tiling; };
-    auto phase_shape = [&](const CaseState* c) { return mixed && ruled(c) ? shape(c) : c->phase; };
-    // Cases in the order of their groups (tile shapes and collide mode).
+    auto merged = [&](const CaseState* c) { return mixed && ruled(c) ? Tiling{64, 8, c->tiling.zc} : c->tiling; };
+    // Cases in the order of their groups: collide mode, then tile shapes, merged
+    // ones together.
     auto key = [&](int id) {
         const CaseState* c = cases_[id].get();
-        const Tiling t = shape(c), pt = phase_shape(c);
-        return std::make_tuple(t.tx, t.ty, c->mode, pt.tx, pt.ty);
+        const Tiling m = merged(c);
+        return std::make_tuple(c->mode, m.tx, m.ty, c->phase.tx * (mixed && ruled(c) ? 0 : 1),
+                               c->phase.ty * (mixed && ruled(c) ? 0 : 1));
+    };
+    auto shape_key = [&](int id) {
+        const CaseState* c = cases_[id].get();
+        return std::tuple_cat(key(id), std::make_tuple(c->tiling.tx, c->tiling.ty));
     };
     order_.clear();
     for (auto& kv : cases_) order_.push_back(kv.first);
-    std::stable_sort(order_.begin(), order_.end(), [&](int a, int b) { return key(a) < key(b); });
+    std::stable_sort(order_.begin(), order_.end(), [&](int a, int b) { return shape_key(a) < shape_key(b); });
     const size_t n = order_.size();
     if (n > views_cap_) {
         for (auto& v : d_views_) {
@@ -673,36 +686,61 @@ mcb_status Batch::rebuild() {
     }
     for (int q = 0; q < 2; ++q)
         if (n) B_HIP(hipMemcpyAsync(d_views_[q], hv_[q].data(), n * sizeof(CaseView), hipMemcpyHostToDevice, stream_));
-    // Groups: [start[k], start[k + 1]) are the cases of group k. Behind them the
-    // halves of a single large one.
+    // The groups of short calls, then those of longer ones where they differ: by
+    // shape, or the halves of a large one.
     std::vector<std::pair<size_t, size_t>> range;
-    for (size_t i = 0; i < n; ++i) {
-        if (i == 0 || key(order_[i]) != key(order_[i - 1])) range.emplace_back(i, i);
-        range.back().second = i + 1;
-    }
+    auto ranges_by = [&](auto&& of) {
+        for (size_t i = 0; i < n; ++i) {
+            if (i == 0 || of(order_[i]) != of(order_[i - 1])) range.emplace_back(i, i);
+            range.back().second = i + 1;
+        }
+    };
+    auto cells = [&](size_t i) { return cases_[order_[i]]->geo.n; };
+    ranges_by(key);
     n_groups_ = range.size();
-    n_halves_ = 0;
-    if (n_groups_ == 1 && n > 1) {
-        auto cells = [&](size_t i) { return cases_[order_[i]]->geo.n; };
-        long long work = 0, half = 0;
-        for (size_t i = 0; i < n; ++i) work += cells(i);
+    bool by_shape = false;
+    if (mixed && total >= kShapeCells) {
+        ranges_by(shape_key);
+        by_shape = n >= kShapeCases * (range.size() - n_groups_);
+        if (!by_shape) range.resize(n_groups_);
+    }
+    const bool one = n_groups_ == 1 && !by_shape;
+    if (one || by_shape) {
+        // The largest group in two, if it holds most of the work.
+        size_t at = 0;
+        long long work = 0;
+        for (size_t k = one ? 0 : n_groups_; k < range.size(); ++k) {
+            long long w = 0;
+            for (size_t i = range[k].first; i < range[k].second; ++i) w += cells(i);
+            if (w > work) {
+                work = w;
+                at = k;
+            }
+        }
+        const size_t begin = range[at].first, end = range[at].second;
         const long long most = cases_[order_[0]]->mode == COLLIDE_STEP ? kSplitCellsFp32 : kSplitCellsFp32Bgk;
-        if (work >= kSplitCells && (storage_ != MCB_STORE_FP32 || work < most)) {
-            size_t cut = 0;
-            while (cut < n - 1 && 2 * half < work) half += cells(cut++);
-            range.emplace_back(0, cut);
-            range.emplace_back(cut, n);
-            n_halves_ = 2;
+        if (end - begin > 1 && work >= kSplitCells && (one ? (storage_ != MCB_STORE_FP32 || work < most) : 2 * work > total)) {
+            long long half = 0;
+            size_t cut = begin;
+            while (cut < end - 1 && 2 * half < work) half += cells(cut++);
+            if (one) range.emplace_back(begin, cut);
+            else range[at].second = cut;
+            range.emplace_back(cut, end);
         }
     }
+    n_long_ = range.size() - n_groups_;
     if (groups_.size() < range.size()) groups_.resize(range.size());
-    std::vector<std::pair<long long, size_t>> load;   // cost and index of a group
+    std::vector<WorkItem> tables;
+    std::vector<std::pair<long long, size_t>> load[2];   // cost and index of a group, of either list
     for (size_t k = 0; k < range.size(); ++k) {
         Group& gr = groups_[k];
         const size_t begin = range[k].first, end = range[k].second;
         gr.first = (unsigned)begin;
         gr.cases = (unsigned)(end - begin);
         const CaseState* c0 = cases_[order_[begin]].get();
+        const bool own = by_shape && k >= n_groups_;   // each case's own shape
+        auto shape = [&](const CaseState* c) { return own ? c->tiling : merged(c); };
+        auto phase_shape = [&](const CaseState* c) { return own || !(mixed && ruled(c)) ? c->phase : merged(c); };
         gr.t = shape(c0);
         gr.pt = phase_shape(c0);
         gr.mode = c0->mode;
@@ -715,45 +753,50 @@ mcb_status Batch::rebuild() {
         long long work = 0;
         for (size_t i = begin; i < end; ++i) {
             const CaseState* c = cases_[order_[i]].get();
-            if (c->massq || c->mass) gr.mass = true;
-            const auto tl = tiles_of(*c, (int)i, shape(c)), pl = tiles_of(*c, (int)i, phase_shape(c));
-            items.insert(items.end(), tl.begin(), tl.end());
-            phase.insert(phase.end(), pl.begin(), pl.end());
+            gr.mass |= c->massq || c->mass;
             differ |= !same_tiling(phase_shape(c), shape(c));
             work += c->geo.n;
         }
+        for (size_t i = begin; i < end; ++i) {
+            const CaseState* c = cases_[order_[i]].get();
+            const auto tl = tiles_of(*c, (int)i, shape(c));
+            items.insert(items.end(), tl.begin(), tl.end());
+            if (!differ) continue;
+            const auto pl = tiles_of(*c, (int)i, phase_shape(c));
+            phase.insert(phase.end(), pl.begin(), pl.end());
+        }
         items = xcd_permute(items);
+        phase = xcd_permute(phase);
         gr.n = (unsigned)items.size();
-        gr.n_phase = 0;
-        if (differ) {
-            phase = xcd_permute(phase);
-            gr.n_phase = (unsigned)phase.size();
-            items.insert(items.end(), phase.begin(), phase.end());
-        }
-        if (items.size() > gr.cap) {
-            if (gr.d_work) B_HIP(hipFree(gr.d_work));
-            gr.d_work = nullptr;
-            gr.cap = 0;
-            const size_t cap = 2 * items.size();
-            B_HIP(hipMalloc(reinterpret_cast<void**>(&gr.d_work), cap * sizeof(WorkItem)));
-            gr.cap = cap;
-        }
-        B_HIP(hipMemcpyAsync(gr.d_work, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, stream_));
-        B_HIP(hipStreamSynchronize(stream_));   // items is a host temporary
-        if (k < n_groups_) load.emplace_back(work + kGroupCells, k);
-        else gr.lane = (int)(k - n_groups_);
+        gr.n_phase = (unsigned)phase.size();
+        gr.at = tables.size();
+        tables.insert(tables.end(), items.begin(), items.end());
+        tables.insert(tables.end(), phase.begin(), phase.end());
+        load[k >= n_groups_].emplace_back(work + kGroupCells, k);
     }
-    B_HIP(hipStreamSynchronize(stream_));   // the copies of hv_
+    if (tables.size() > work_cap_) {
+        if (d_work_) B_HIP(hipFree(d_work_));
+        d_work_ = nullptr;
+        work_cap_ = 0;
+        const size_t cap = 2 * tables.size();
+        B_HIP(hipMalloc(reinterpret_cast<void**>(&d_work_), cap * sizeof(WorkItem)));
+        work_cap_ = cap;
+    }
+    if (!tables.empty())
+        B_HIP(hipMemcpyAsync(d_work_, tables.data(), tables.size() * sizeof(WorkItem), hipMemcpyHostToDevice, stream_));
+    B_HIP(hipStreamSynchronize(stream_));   // the copies of hv_ and tables
     // Lanes: each group to the least loaded one, largest first.
-    std::sort(load.rbegin(), load.rend());
-    lanes_ = (int)std::max<size_t>(1, std::min<size_t>(kLanes, n_groups_));
-    long long lane_load[kLanes] = {};
-    for (const auto& l : load) {
-        const int at = (int)(std::min_element(lane_load, lane_load + lanes_) - lane_load);
-        groups_[l.second].lane = at;
-        lane_load[at] += l.first;
+    for (int j = 0; j < 2; ++j) {
+        std::sort(load[j].rbegin(), load[j].rend());
+        lanes_[j] = (int)std::max<size_t>(1, std::min<size_t>(kLanes, load[j].size()));
+        long long lane_load[kLanes] = {};
+        for (const auto& l : load[j]) {
+            const int at = (int)(std::min_element(lane_load, lane_load + lanes_[j]) - lane_load);
+            groups_[l.second].lane = at;
+            lane_load[at] += l.first;
+        }
     }
-    const int lanes = std::max(lanes_, n_halves_);
+    const int lanes = std::max(lanes_[0], lanes_[1]);
     if (lanes > 1 && !fork_) B_HIP(hipEventCreateWithFlags(&fork_, hipEventDisableTiming));
     for (int i = 0; i + 1 < lanes; ++i) {
         if (!lane_[i]) B_HIP(hipStreamCreateWithFlags(&lane_[i], hipStreamNonBlocking));
@@ -765,12 +808,12 @@ mcb_status Batch::rebuild() {
 
 mcb_status Batch::launch_steps(int q, int n) {
     // A caller capturing stream_ gets everything recorded there.
-    int lanes = n > 1 ? std::max(lanes_, n_halves_) : lanes_;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (lanes > 1) B_HIP(hipStreamIsCapturing(stream_, &cap));
-    if (cap != hipStreamCaptureStatusNone) lanes = 1;
-    const bool fork = lanes > 1, halves = fork && n_halves_ > 0;
-    const size_t first = halves ? n_groups_ : 0, last = halves ? n_groups_ + (size_t)n_halves_ : n_groups_;
+    if (std::max(lanes_[0], lanes_[1]) > 1) B_HIP(hipStreamIsCapturing(stream_, &cap));
+    const bool captured = cap != hipStreamCaptureStatusNone, longer = n_long_ > 0 && n > 1 && !captured;
+    const int lanes = captured ? 1 : lanes_[longer];
+    const bool fork = lanes > 1;
+    const size_t first = longer ? n_groups_ : 0, last = longer ? n_groups_ + n_long_ : n_groups_;
     if (fork) {
         B_HIP(hipEventRecord(fork_, stream_));
         for (int i = 0; i + 1 < lanes; ++i) B_HIP(hipStreamWaitEvent(lane_[i], fork_, 0));
@@ -780,11 +823,12 @@ mcb_status Batch::launch_steps(int q, int n) {
         for (size_t i = first; i < last && e == hipSuccess; ++i) {
             const Group& gr = groups_[i];
             const hipStream_t s = fork && gr.lane ? lane_[gr.lane - 1] : stream_;
-            e = gr.n_phase ? launch_phase_batch(d_views_[q], gr.d_work + gr.n, gr.n_phase, gr.pt, storage_, s)
-                           : launch_phase_batch(d_views_[q], gr.d_work, gr.n, gr.t, storage_, s);
+            const WorkItem* const work = d_work_ + gr.at;
+            e = gr.n_phase ? launch_phase_batch(d_views_[q], work + gr.n, gr.n_phase, gr.pt, storage_, s)
+                           : launch_phase_batch(d_views_[q], work, gr.n, gr.t, storage_, s);
             if (e == hipSuccess && gr.sum.zc) e = launch_mass_sum(d_views_[q] + gr.first, gr.geo, gr.sum, s);
             if (e == hipSuccess && gr.mass) e = launch_mass_finish(d_views_[q] + gr.first, gr.cases, s);
-            if (e == hipSuccess) e = launch_collide_batch(d_views_[q], gr.d_work, gr.n, gr.t, gr.mode, storage_, s);
+            if (e == hipSuccess) e = launch_collide_batch(d_views_[q], work, gr.n, gr.t, gr.mode, storage_, s);
         }
     // Also after an error: whatever was launched is ordered before stream_'s next work.
     for (int i = 0; fork && i + 1 < lanes; ++i) {

@@ -167,27 +167,29 @@ private:
     // device arrays
     CaseView* d_views_[2] = {nullptr, nullptr};
     size_t views_cap_ = 0;
-    // Cases of one tile shape and collide mode: views [first, first + cases) of
-    // the arrays, one work table, one lane.
+    // Cases that step on one tile shape in one collide mode: views
+    // [first, first + cases) of the arrays, one work table, one lane.
     struct Group {
         Tiling t{}, pt{};                // tiles of the collide and phase passes
         int mode = COLLIDE_STEP;
-        WorkItem* d_work = nullptr;      // [0, n) collide, [n, n + n_phase) phase where its tiles differ
-        size_t cap = 0;
-        unsigned n = 0, n_phase = 0;
+        size_t at = 0;                   // its items in d_work_: [at, at + n) collide, then n_phase of the phase
+        unsigned n = 0, n_phase = 0;     // pass where its tiles differ
         unsigned first = 0, cases = 0;
         Tiling sum{};                    // zc > 0: its only case sums phi on tiles of its own (launch_mass_sum)
         Geo geo{};                       // of that case
         bool mass = false;               // a case keeps a mass-drift correction (MassCell or MassQ)
         int lane = 0;                    // 0: stream_, i: lane_[i - 1]
     };
-    std::vector<Group> groups_;          // the first n_groups_ + n_halves_ are in use (tables are kept for reuse)
-    size_t n_groups_ = 0;
-    int n_halves_ = 0;                   // 2: behind a single group stand its halves (kSplitCells)
+    // The first n_groups_ serve calls of one step, the n_long_ behind them (if any)
+    // longer ones.
+    std::vector<Group> groups_;
+    size_t n_groups_ = 0, n_long_ = 0;
+    WorkItem* d_work_ = nullptr;         // the groups' work tables
+    size_t work_cap_ = 0;
     static constexpr int kLanes = 4;     // hardware queues of a process
     hipStream_t lane_[kLanes - 1] = {};  // created when a batch first needs them
     hipEvent_t fork_ = nullptr, join_[kLanes - 1] = {};
-    int lanes_ = 1;                      // lanes in use
+    int lanes_[2] = {1, 1};              // lanes that either list uses
     std::vector<CaseView> hv_[2];     // host copies of the view arrays
     bool any_initial_ = false;        // a moment-form case has not stepped yet
     double* d_partial_ = nullptr;     // reduction scratch (2 * kReduceBlocks + 2 doubles)

@@ -348,3 +348,24 @@ def test_autotuned_context(gpu_lib, storage, tau_g, nx, ny, nz):
         assert np.array_equal(lat.read("phi"), b.read(cid, "phi"))
     # From the tuned state the rule's tile is still a candidate.
     assert mcb.autotune(p)[:2] in mcb.tilings() and rule[:2] in mcb.tilings()
+
+
+@pytest.mark.parametrize("tau_gs", [(1.0,), (0.8, 1.0)])
+@pytest.mark.parametrize("sides", [[(48, 40, 40), (64, 40, 40), (32, 40, 50)] * 6, [(192, 160, 80), (32, 40, 40)] * 5])
+def test_fp32_batch_shape_by_shape(gpu_lib, sides, tau_gs):
+    """Enough cases of each shape: longer calls step shape by shape (the second batch with its largest one in two), calls
+    of one step all together; with a case that leaves, which changes the order."""
+    mcb = gpu_lib
+    with mcb.Batch(0) as b:
+        cases = []
+        for i, (nx, ny, nz) in enumerate(sides):
+            p = mcb.make_params(nx, ny, nz, tau_f=0.55 + 0.01 * i, tau_g=tau_gs[i % len(tau_gs)])
+            bub = ((0.3 + 0.02 * i) * nx, 0.5 * ny, 0.6 * nz, 0.28 * min(nx, ny, nz))
+            cases.append((b.add(p, [bub], 3.0), p, bub))
+        for steps in (3, 1, 2):
+            b.step(steps)
+        b.remove(cases.pop(1)[0])
+        for steps in (1, 4):
+            b.step(steps)
+        for cid, p, bub in cases:
+            assert np.array_equal(b.read(cid, "phi"), alone(mcb, p, bub, 11)), cid
