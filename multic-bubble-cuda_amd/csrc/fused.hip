@@ -287,7 +287,8 @@ __global__ __launch_bounds__(RB) void k_reduce_partial(const float* __restrict__
 // The partials' sums, one workgroup: thread t adds partials t, t + RB, ... in
 // order, then the butterfly of k_reduce_partial. Bound by latency: one thread
 // adding the 1024 pairs in turn waited for each load and add and took 84 us
-// (64^3, against 5 us for k_reduce_partial); this form takes 2.5 us (the whole call 87 -> 9.6 us).
+// (64^3, against 3.7 us for k_reduce_partial); this form takes 2.5 us in a row
+// of calls, 4.1 by itself (the whole call 87 -> 11 us).
 __global__ __launch_bounds__(RB) void k_reduce_final(const double* __restrict__ partial, int nb,
                                                      double* __restrict__ out) {
     double a = 0.0, b = 0.0;
